@@ -139,7 +139,7 @@ struct HostTables {
     // (P threads per line, Q rows each; rows past M are padding), so a wave's loads of one
     // row index are contiguous
     std::vector<double> am_x, bm_x, cm_x, r2inv_x;
-    std::vector<double> ytwc_re, ytwc_im, ytwr_re, ytwr_im;
+    std::vector<double> ytwc_re, ytwc_im, ytwr_re, ytwr_im, ydm;
     std::vector<double> ztwc_re, ztwc_im, ztwr_re, ztwr_im, zdct_re, zdct_im;
 };
 
@@ -152,7 +152,7 @@ static int upload_tables(DevTables<T>& dt, const HostTables& h) {
         (rc = upload(dt, h.wsum, &t.wsum)) || (rc = upload(dt, h.qf, &t.qf)) || (rc = upload(dt, h.qiT, &t.qiT)) ||
         (rc = upload(dt, h.ytwc_re, &t.ytwc_re)) || (rc = upload(dt, h.ytwc_im, &t.ytwc_im)) ||
         (rc = upload(dt, h.ytwr_re, &t.ytwr_re)) || (rc = upload(dt, h.ytwr_im, &t.ytwr_im)) ||
-        (rc = upload(dt, h.ztwc_re, &t.ztwc_re)) || (rc = upload(dt, h.ztwc_im, &t.ztwc_im)) ||
+        (rc = upload(dt, h.ydm, &t.ydm)) || (rc = upload(dt, h.ztwc_re, &t.ztwc_re)) || (rc = upload(dt, h.ztwc_im, &t.ztwc_im)) ||
         (rc = upload(dt, h.ztwr_re, &t.ztwr_re)) || (rc = upload(dt, h.ztwr_im, &t.ztwr_im)) ||
         (rc = upload(dt, h.zdct_re, &t.zdct_re)) || (rc = upload(dt, h.zdct_im, &t.zdct_im)))
         return rc;
@@ -169,6 +169,23 @@ static void twiddles(int n, int count, std::vector<double>& re, std::vector<doub
         re[t] = std::cos(a);
         im[t] = -std::sin(a);
     }
+}
+
+// cos and sin(2 pi r c / L) for r, c <= L/2 in the operand order of the dense y DFT: entry
+// ((rb * steps + ks) * 2 + {0 cos, 1 sin}) * 64 + lane holds row r = 16 rb + lane % 16, column
+// c = 4 ks + lane / 16; rows and columns past L/2, and the sines that vanish, are 0.
+static void ydft_tab(int L, std::vector<double>& tab) {
+    const int nk = dft_steps(L), nrb = dft_blocks(L), h = L / 2;
+    std::vector<double> re, im;
+    twiddles(L, L, re, im);
+    tab.assign((size_t)nrb * nk * 128, 0.0);
+    for (int r = 0; r <= h; ++r)
+        for (int c = 0; c <= h; ++c) {
+            const int t = (int)((long)r * c % L);
+            double* e = &tab[((size_t)(r / 16) * nk + c / 4) * 128 + (c % 4) * 16 + r % 16];
+            e[0] = re[t];
+            e[64] = (2 * t) % L == 0 ? 0.0 : -im[t];
+        }
 }
 
 static void free_plan(eddy_plan_s* P) {
@@ -699,14 +716,15 @@ static int create_plan(eddy_plan_s** out, int nx, int ny, int nz, double delysq,
     if (ydense) P->fpy = FftPlan{0, 0, {}};
     {
         auto ylds = [&](int ti) {
-            return ydense ? ((size_t)ti * fft_ld(L) + 2 * (size_t)L) * sizeof(double)
+            return ydense ? (size_t)ti * dft_pitch(L) * sizeof(double)
                           : (2 * (size_t)ti * fft_ld(L / 2) + 4 * (size_t)fft_ld(L / 2)) * sizeof(double);
         };
         auto yok = [&](int ti) {
             return ylds(ti) <= lds_cap && (ydense || (long)ti * (L / 2) <= (long)min_radix(P->fpy) * kFftThreads);
         };
         while (P->tune.yfft_pencils > 1 && !yok(P->tune.yfft_pencils)) P->tune.yfft_pencils /= 2;
-        if (!yok(P->tune.yfft_pencils)) {
+        // (the dense DFT's matrices grow with L^2: lengths above 6500 or so stay refused)
+        if (!yok(P->tune.yfft_pencils) || (ydense && (fft_ld(L) + 2 * (size_t)L) * sizeof(double) > lds_cap)) {
             set_error("periodic length too large for the in-place FFT");
             return EDDY_ERR_UNSUPPORTED;
         }
@@ -928,9 +946,9 @@ static int create_plan(eddy_plan_s** out, int nx, int ny, int nz, double delysq,
             }
         P->fpz = FftPlan{1, 0, {}};
     }
-    // y real FFT tables (L = 2H; radix plan made above); the dense DFT reads all L roots
+    // y real FFT tables (L = 2H; radix plan made above), or the dense DFT's matrices
     if (ydense) {
-        twiddles(L, L, h.ytwr_re, h.ytwr_im);
+        ydft_tab(L, h.ydm);
     } else {
         twiddles(L / 2, L / 2, h.ytwc_re, h.ytwc_im);
         twiddles(L, L / 2 + 1, h.ytwr_re, h.ytwr_im);

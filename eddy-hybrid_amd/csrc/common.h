@@ -41,7 +41,18 @@ struct Tables {
     // y real DFT as dense matrices for the matrix-core variant (FP32 tables only, else null):
     // ydft_f[j*L + p] = F(p, j) forward, ydft_b[p*L + j] = G(j, p) inverse with 1/L
     const T* ydft_f; const T* ydft_b;
+    // y real DFT of the lengths the radix FFT does not take (ydft_tab in yfft.hip), else null
+    const T* ydm;
 };
+
+// Half-length DFT matrices of a length-L real transform: wavenumbers and folded samples 0..L/2,
+// the samples padded to whole 4-deep matrix-core steps, the outputs to whole 16-row blocks.
+__host__ __device__ inline int dft_steps(int L) { return (L / 2) / 4 + 1; }
+__host__ __device__ inline int dft_blocks(int L) { return (L / 2) / 16 + 1; }
+// LDS row of one pencil: the two folded halves of 4 * dft_steps values; the pitch is 2 mod 4, so
+// that the 16 rows and the two sample indices of a half-wave's operand read fall in distinct
+// banks (FP64)
+__host__ __device__ inline int dft_pitch(int L) { return 8 * dft_steps(L) + 2; }
 
 struct Dims {
     int nx, ny, nz;   // DP(NX,NY,NZ)

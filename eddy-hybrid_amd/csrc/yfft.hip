@@ -5,9 +5,8 @@
 // fftpack (fftpack.f:140-240): [Re X0, Re X1, Im X1, ..., Re X_{L/2}] (L even).
 //
 // Periodic lengths the radix FFT cannot take (L odd, or L/2 with a prime factor >= 7) go through
-// the same tiles with the transform done as a dense real DFT (the DENSE kernels): the tile holds
-// TI real rows of length L in LDS and every output is its O(L) sum against the table
-// exp(-2 pi i t/L), t < L, the packing and scaling as above.
+// the same tiles with the transform done as a dense real DFT on the matrix cores (the DENSE
+// kernels, dft_fwd_tile / dft_inv_tile), the packing and scaling as above.
 //
 // A workgroup owns TI (a power of two) consecutive x1 pencils at one x2 index k. The pencils
 // are read row by row (TI contiguous doubles per y index: coalesced), with several loads in
@@ -22,6 +21,7 @@
 #include "batch_device.h"
 #include "fft_device.h"
 #include "kernels.h"
+#include "mma_device.h"
 #include "reduce_device.h"
 #include "stencil_device.h"
 
@@ -193,6 +193,66 @@ __device__ __forceinline__ void residual_rows(const Dims& d, const Op64& op, con
     }
 }
 
+// The dense real DFT of a tile, on the matrix cores. Folding the samples halves its products:
+// with P_j = x_j + x_{L-j} (P_0 = x_0, P_{L/2} = x_{L/2}) and Q_j = x_j - x_{L-j} (Q_0 = 0),
+//   Re X_q = sum_{j <= L/2} P_j cos(2 pi q j/L),   Im X_q = -sum_{j <= L/2} Q_j sin(2 pi q j/L),
+// and the inverse takes the same two symmetric matrices over q to x_j and x_{L-j}. The plan lays
+// them out in operand order (ydft_tab: block rb of 16 outputs, step ks of 4 samples, cosine then
+// sine, lane), so an operand load is one contiguous 512-byte (FP32 256-byte) read served by L2.
+// A wave owns 16 outputs of 16 pencils: per step two LDS reads feed one cosine and one sine
+// product, 64 matrix-core cycles each in FP64, which hide both the reads and the additions of
+// the fold. L multiply-adds per value: at 160 x 96 x 112 the forward transform takes 0.029 ms and
+// the inverse 0.022 ms, where a sum per output on the vector ALUs (L multiply-adds with two LDS
+// reads and an index step each) took 0.716 and 0.708 ms.
+constexpr int kDftAhead = 4;  // steps whose matrix operands are loaded ahead of their products
+
+template <typename T>
+struct DftAcc {
+    typename Mma<T>::v4 c, s;
+};
+
+// sum over the samples of `row` (this lane's pencil) for output block rb; FOLD: the row holds x_j
+// and x_{L-j} (forward), else the two operands as they are (inverse).
+template <typename T, bool FOLD>
+__device__ __forceinline__ DftAcc<T> dft_block(const T* __restrict__ ydm, const T* row, int nk, int rb, int lane) {
+    DftAcc<T> acc;
+    acc.c = typename Mma<T>::v4{T(0), T(0), T(0), T(0)};
+    acc.s = acc.c;
+    const T* m = ydm + (size_t)rb * nk * 128 + lane;
+    const T* a = row + (lane >> 4);
+    const T* b = a + 4 * nk;
+    for (int k0 = 0; k0 < nk; k0 += kDftAhead) {
+        T mc[kDftAhead], ms[kDftAhead];
+#pragma unroll
+        for (int u = 0; u < kDftAhead; ++u) {
+            const int k = min(k0 + u, nk - 1);  // past the end: the last step's operands, unused
+            mc[u] = m[k * 128];
+            ms[u] = m[k * 128 + 64];
+        }
+#pragma unroll
+        for (int u = 0; u < kDftAhead; ++u) {
+            if (k0 + u < nk) {
+                const T x = a[4 * (k0 + u)], y = b[4 * (k0 + u)];
+                acc.c = Mma<T>::run(mc[u], FOLD ? x + y : x, acc.c);
+                acc.s = Mma<T>::run(ms[u], FOLD ? x - y : y, acc.s);
+            }
+        }
+    }
+    return acc;
+}
+
+// Zero the slots of a tile's rows that no sample fills: 0 and the padding of both halves (and the
+// second half's L/2 of an even L, its own partner).
+template <typename T>
+__device__ __forceinline__ void dft_zero_pads(T* rows, int pitch, int L, int TI, int tid, int nthr) {
+    const int half = 4 * dft_steps(L), h = L / 2, h1 = (L - 1) / 2;
+    const int na = half - 1 - h, npad = na + 1 + (half - 1 - h1);
+    for (int e = tid; e < TI * npad; e += nthr) {
+        const int ii = e / npad, t = e - ii * npad;
+        rows[ii * pitch + (t < na ? h + 1 + t : (t == na ? half : half + h1 + t - na))] = T(0);
+    }
+}
+
 // One tile (TI pencils at one x2 index) of the forward transform; `tile` is the logical tile,
 // ntx the tiles per x2 row, `slot`/`nslots` the reduction partial index and count.
 template <typename T, int MODE, bool DENSE = false>
@@ -202,22 +262,19 @@ __device__ __forceinline__ void yfft_fwd_tile(const YArgs<T>& a, int tile, int n
     const Dims d = a.d;
     const int TI = a.TI, lti = a.lti, ld = a.ld, H = d.L / 2, L = d.L;
     // FFT: TI complex rows (split re/im) transformed in place, then the two twiddle tables;
-    // DENSE: TI real rows, then the table exp(-2 pi i t/L), t < L
+    // DENSE: TI real rows, x_j (j <= L/2) at j and x_{L-j} at 4 dft_steps(L) + j
     T* Ar = smem;
     T* Ai = Ar + TI * ld;
     T* twc_r = Ai + TI * ld;  // exp(-2 pi i t/H), t < H
     T* twc_i = twc_r + H;
-    T* twr_r = DENSE ? Ar + TI * ld : twc_i + H;  // exp(-2 pi i k/L), k <= H (DENSE: k < L)
-    T* twr_i = twr_r + (DENSE ? L : H + 1);
+    T* twr_r = twc_i + H;  // exp(-2 pi i k/L), k <= H
+    T* twr_i = twr_r + H + 1;
     const int i0 = (tile % ntx) * TI;
     const int k = tile / ntx;
     const int tid = threadIdx.x, nthr = blockDim.x;
     const int total = TI * L;
     if (DENSE) {
-        for (int t = tid; t < L; t += nthr) {
-            twr_r[t] = a.tb.ytwr_re[t];
-            twr_i[t] = a.tb.ytwr_im[t];
-        }
+        dft_zero_pads<T>(Ar, ld, L, TI, tid, nthr);
     } else {
         for (int t = tid; t <= H; t += nthr) {
             if (t < H) {
@@ -241,7 +298,7 @@ __device__ __forceinline__ void yfft_fwd_tile(const YArgs<T>& a, int tile, int n
     const int jstep = nthr >> lti;
     auto put = [&](double x, int j) {  // row j of pencil ii into the packed complex buffer
         if (j < L) {
-            if (DENSE) Ar[ii * ld + pidx(j)] = T(x);
+            if (DENSE) Ar[ii * ld + (j <= H ? j : 4 * dft_steps(L) + L - j)] = T(x);
             else if (j & 1) Ai[ii * ld + pidx((j >> 1))] = T(x);
             else Ar[ii * ld + pidx((j >> 1))] = T(x);
         }
@@ -311,24 +368,21 @@ __device__ __forceinline__ void yfft_fwd_tile(const YArgs<T>& a, int tile, int n
     const size_t js = (size_t)d.M * (size_t)d.N;
     T* outK = a.S + (size_t)d.M * (size_t)k;
     if (DENSE) {
-        // packed slot s of pencil ii: sum_j x_j W^{q j}, q = (s+1)/2, its real part for s = 0
-        // and odd s (the Nyquist slot L-1 of an even L included), its imaginary part for even s
-        for (int e = tid; e < total; e += nthr) {
-            const int ii = e & (TI - 1);
-            const int sl = e >> lti;
-            const int gi = i0 + ii;
-            if (gi >= d.M) continue;
-            const int q = (sl + 1) >> 1;
-            const T* w = (sl == 0 || (sl & 1)) ? twr_r : twr_i;
-            const T* row = Ar + ii * ld;
-            T acc = T(0);
-            int t = 0;
-            for (int j = 0; j < L; ++j) {
-                acc += row[pidx(j)] * w[t];
-                t += q;
-                if (t >= L) t -= L;
+        // item: 16 wavenumbers of 16 pencils to a wave (fewer pencils in the tile: the lanes past
+        // TI repeat a row and store nothing); packed slots 2q-1 (Re) and 2q (Im), slot 0 Re X_0
+        const int nk = dft_steps(L), nrb = dft_blocks(L), ncb = (TI + 15) >> 4;
+        const int lane = tid & 63;
+        for (int it = __builtin_amdgcn_readfirstlane(tid >> 6); it < nrb * ncb; it += nthr >> 6) {
+            const int rb = it / ncb, p = 16 * (it - rb * ncb) + (lane & 15);
+            const DftAcc<T> r = dft_block<T, true>(a.tb.ydm, Ar + (p & (TI - 1)) * ld, nk, rb, lane);
+            const int gi = i0 + p;
+            if (p >= TI || gi >= d.M) continue;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int q = 16 * rb + Mma<T>::row(lane >> 4, v);
+                if (q <= H) outK[js * (size_t)(q ? 2 * q - 1 : 0) + gi] = r.c[v];
+                if (q > 0 && 2 * q < L) outK[js * (size_t)(2 * q) + gi] = -r.s[v];
             }
-            outK[js * (size_t)sl + gi] = acc;
         }
         return;
     }
@@ -392,20 +446,17 @@ __device__ __forceinline__ void yfft_inv_tile(const YArgs<T>& a, int tile, int n
     T* smem = reinterpret_cast<T*>(smem_raw);
     const Dims d = a.d;
     const int TI = a.TI, lti = a.lti, ld = a.ld, H = d.L / 2, L = d.L;
-    T* Ar = smem;  // FFT: TI complex rows, transformed in place; DENSE: TI real rows
+    T* Ar = smem;  // FFT: TI complex rows, transformed in place; DENSE: TI rows of coefficients
     T* Ai = Ar + TI * ld;
     T* twc_r = Ai + TI * ld;
     T* twc_i = twc_r + H;
-    T* twr_r = DENSE ? Ar + TI * ld : twc_i + H;
-    T* twr_i = twr_r + (DENSE ? L : H + 1);
+    T* twr_r = twc_i + H;
+    T* twr_i = twr_r + H + 1;
     const int i0 = (tile % ntx) * TI;
     const int k = tile / ntx;
     const int tid = threadIdx.x, nthr = blockDim.x;
     if (DENSE) {
-        for (int t = tid; t < L; t += nthr) {
-            twr_r[t] = a.tb.ytwr_re[t];
-            twr_i[t] = a.tb.ytwr_im[t];
-        }
+        dft_zero_pads<T>(Ar, ld, L, TI, tid, nthr);
     } else {
         for (int t = tid; t <= H; t += nthr) {
             if (t < H) {
@@ -420,10 +471,11 @@ __device__ __forceinline__ void yfft_inv_tile(const YArgs<T>& a, int tile, int n
     const T* inK = a.Sin + (size_t)d.M * (size_t)k;
     __syncthreads();  // the twiddle tables are read below by other threads than wrote them
     if (DENSE) {
-        // the packed coefficients of the tile's pencils into LDS rows, scaled by 1/L (rows
-        // of contiguous x1 values: coalesced); pencils past M read a clamped in-range row
-        const T invL = T(1) / T(L);
-        const int ii = tid & (TI - 1);
+        // the packed coefficients of the tile's pencils into LDS rows (rows of contiguous x1
+        // values: coalesced): w_q Re X_q / L at q and -2 Im X_q / L at 4 dft_steps(L) + q, with
+        // w = 1 for q = 0 and L/2 (their own partners), else 2; pencils past M read a clamped row
+        const T invL = T(1) / T(L), inv2 = T(2) * invL;
+        const int ii = tid & (TI - 1), half = 4 * dft_steps(L);
         const bool iok = i0 + ii < d.M;
         const T* col = inK + (iok ? i0 + ii : d.M - 1);
         const int sstep = nthr >> lti;
@@ -432,8 +484,12 @@ __device__ __forceinline__ void yfft_inv_tile(const YArgs<T>& a, int tile, int n
 #pragma unroll
             for (int u = 0; u < kLoadBatch; ++u) x[u] = col[js * (size_t)min(s0 + u * sstep, L - 1)];
 #pragma unroll
-            for (int u = 0; u < kLoadBatch; ++u)
-                if (s0 + u * sstep < L) Ar[ii * ld + pidx(s0 + u * sstep)] = iok ? x[u] * invL : T(0);
+            for (int u = 0; u < kLoadBatch; ++u) {
+                const int s = s0 + u * sstep, q = (s + 1) >> 1;
+                const bool re = s == 0 || (s & 1);
+                const T w = !iok ? T(0) : (!re ? -inv2 : ((q == 0 || 2 * q == L) ? invL : inv2));
+                if (s < L) Ar[ii * ld + (re ? q : half + q)] = iok ? x[u] * w : T(0);
+            }
         }
         __syncthreads();
     }
@@ -519,30 +575,9 @@ __device__ __forceinline__ void yfft_inv_tile(const YArgs<T>& a, int tile, int n
     const int total = TI * L;
     // DP addresses as 32-bit byte offsets from the field base (DP < 4 GiB)
     const unsigned nx8 = 8u * (unsigned)d.nx, pl8K = nx8 * (unsigned)d.ny * (unsigned)K;
-    for (int e = tid; e < total; e += nthr) {
-        const int ii = e & (TI - 1);
-        const int j = e >> lti;
-        const int gi = i0 + ii;
-        if (gi >= d.M) continue;
+    // the value v of cell (gi, j) of the plane, as MODE stores it
+    auto emit = [&](int gi, int j, double v) {
         const unsigned oj = pl8K + nx8 * (unsigned)(j + 1) + 8u * (unsigned)(gi + 1);
-        double v;
-        if (DENSE) {
-            // x_j = X_0 + 2 sum_q (Re X_q cos(2 pi q j/L) - Im X_q sin(2 pi q j/L)) + X_{L/2} (-1)^j,
-            // the coefficients already scaled by 1/L (fftpack's RFFTB after direct.f:1036)
-            const T* row = Ar + ii * ld;
-            T acc = T(0);
-            int t = j;
-            for (int q = 1; 2 * q < L; ++q) {
-                acc += row[pidx(2 * q - 1)] * twr_r[t] + row[pidx(2 * q)] * twr_i[t];
-                t += j;
-                if (t >= L) t -= L;
-            }
-            T x = row[pidx(0)] + T(2) * acc;
-            if ((L & 1) == 0) x += (j & 1) ? -row[pidx(L - 1)] : row[pidx(L - 1)];
-            v = (double)x;
-        } else {
-            v = (double)((j & 1) ? Zi[ii * ld + pidx((j >> 1))] : Zr[ii * ld + pidx((j >> 1))]);
-        }
         const int I = gi + 1, J = j + 1;
         if (MODE == YI_UPDATE_FINAL) v = ld_off(a.dp, oj) + v - mean;
         if (MODE == YI_DIRECT || MODE == YI_UPDATE_FINAL) {
@@ -568,6 +603,31 @@ __device__ __forceinline__ void yfft_inv_tile(const YArgs<T>& a, int tile, int n
             const double nv = ld_off(a.dp, oj) + v;
             st_off(a.dp, oj, nv);
             psum += nv;
+        }
+    };
+    if (DENSE) {
+        // x_j = E_j + O_j and x_{L-j} = E_j - O_j, E and O the cosine and sine sums (fftpack's
+        // RFFTB after direct.f:1036)
+        const int nk = dft_steps(L), nrb = dft_blocks(L), ncb = (TI + 15) >> 4;
+        const int lane = tid & 63;
+        for (int it = __builtin_amdgcn_readfirstlane(tid >> 6); it < nrb * ncb; it += nthr >> 6) {
+            const int rb = it / ncb, p = 16 * (it - rb * ncb) + (lane & 15);
+            const DftAcc<T> r = dft_block<T, false>(a.tb.ydm, Ar + (p & (TI - 1)) * ld, nk, rb, lane);
+            const int gi = i0 + p;
+            if (p >= TI || gi >= d.M) continue;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int j = 16 * rb + Mma<T>::row(lane >> 4, v);
+                if (j <= H) emit(gi, j, (double)(r.c[v] + r.s[v]));
+                if (j > 0 && 2 * j < L) emit(gi, L - j, (double)(r.c[v] - r.s[v]));
+            }
+        }
+    } else {
+        for (int e = tid; e < total; e += nthr) {
+            const int ii = e & (TI - 1);
+            const int j = e >> lti;
+            if (i0 + ii >= d.M) continue;
+            emit(i0 + ii, j, (double)((j & 1) ? Zi[ii * ld + pidx((j >> 1))] : Zr[ii * ld + pidx((j >> 1))]));
         }
     }
     if (MODE == YI_DIRECT || MODE == YI_UPDATE_FINAL) {
@@ -599,8 +659,8 @@ __global__ void __launch_bounds__(kFftThreads) __attribute__((amdgpu_waves_per_e
 
 // TI complex rows (transformed in place) + the two twiddle tables
 static inline size_t ylds_bytes(int TI, int ld, size_t tsz) { return (2 * (size_t)TI * ld + 4 * (size_t)ld) * tsz; }
-// the dense DFT: TI real rows + the table of L complex roots
-static inline size_t ylds_dense_bytes(int TI, int L, size_t tsz) { return ((size_t)TI * fft_ld(L) + 2 * (size_t)L) * tsz; }
+// the dense DFT: TI real rows
+static inline size_t ylds_dense_bytes(int TI, int L, size_t tsz) { return (size_t)TI * dft_pitch(L) * tsz; }
 
 static inline int ilog2(int v) {
     int l = 0;
@@ -636,7 +696,7 @@ void launch_yfft_fwd(hipStream_t st, const Dims& d, const FftPlan& fp, const Tab
     a.lti = ilog2(TI);
     a.iblk = iblk;
     const bool dense = fp.n == 0;  // the plan's dense-DFT marker (no radix plan for L)
-    a.ld = dense ? fft_ld(d.L) : fft_ld(d.L / 2);
+    a.ld = dense ? dft_pitch(d.L) : fft_ld(d.L / 2);
     a.shift = shift;
     dim3 grid(ceil_div(d.M, TI), d.N);
     size_t sh = dense ? ylds_dense_bytes(TI, d.L, sizeof(T)) : ylds_bytes(TI, a.ld, sizeof(T));
@@ -691,7 +751,7 @@ void launch_yfft_inv(hipStream_t st, const Dims& d, const FftPlan& fp, const Tab
     a.TI = TI;
     a.lti = ilog2(TI);
     const bool dense = fp.n == 0;
-    a.ld = dense ? fft_ld(d.L) : fft_ld(d.L / 2);
+    a.ld = dense ? dft_pitch(d.L) : fft_ld(d.L / 2);
     dim3 grid(ceil_div(d.M, TI), d.N);
     size_t sh = dense ? ylds_dense_bytes(TI, d.L, sizeof(T)) : ylds_bytes(TI, a.ld, sizeof(T));
     auto go = [&](auto fn) {
