@@ -621,7 +621,7 @@ static int build_x1_basis(eddy_plan_s* P, int M, int L, int N, const double* ap,
     const size_t n = (size_t)zp * zq;
     z.am_x.assign(n, 0.0);
     z.cm_x.assign(n, 0.0);
-    z.bm_x.assign(n, 1.0);
+    z.bm_x.assign(n, -1.0);  // padding rows, as for the x1 lines
     z.r2inv_x.assign(n, 0.0);
     for (int pp = 0; pp < zp; ++pp)
         for (int r = 0; r < zq; ++r) {
@@ -772,7 +772,7 @@ static int create_plan(eddy_plan_s** out, int nx, int ny, int nz, double delysq,
         const size_t n = (size_t)xp * xq;
         h.am_x.assign(n, 0.0);
         h.cm_x.assign(n, 0.0);
-        h.bm_x.assign(n, 1.0);
+        h.bm_x.assign(n, -1.0);  // padding rows: -1 + lam is never 0 (lam <= 0)
         h.r2inv_x.assign(n, 0.0);
         for (int pp = 0; pp < xp; ++pp)
             for (int r = 0; r < xq; ++r) {

@@ -12,10 +12,18 @@
 // own chunk with a modified Thomas sweep that expresses each row through the chunk's first
 // and last unknowns; the 2P chunk-end unknowns form a tridiagonal system solved by parallel
 // cyclic reduction across the P lanes of the line (wave shuffles); each thread then
-// back-substitutes its chunk. The line block is staged through LDS so global reads/writes
-// are contiguous (lines are x1-contiguous in S).
+// back-substitutes its chunk. A wave stages the elements of its 64/P lines, which are contiguous
+// in S, through LDS of its own, so that global reads and writes are contiguous and no workgroup
+// barrier is needed.
+//
+// What bounds it: FP64 instruction issue beside HBM (16 B per cell). A wave's 64/P lines are 64 Q
+// elements, so lane and element index differ by multiples of 64: the staging addresses are one
+// base plus constants, where indexing a padded 2-D tile took a quotient per element each way.
+// 512 x 256 x 256 FP64 (P = 64, Q = 8): 0.153 -> 0.127 ms, 4.2 TB/s; the production grid's 1024-row
+// x2 lines (P = 64, Q = 16): 0.231 -> 0.169 ms.
 #include <algorithm>
 #include <numeric>
+#include <type_traits>
 
 #include "batch_device.h"
 #include "kernels.h"
@@ -55,107 +63,78 @@ struct XArgs {
     T* linesum;
     Dims d;
     Tables<T> tb;
-    int P, Q, ldw;
+    int P, Q;
     long lbeg, lend;  // line range (j-major lines j*N + m) of this launch
     // periodic lines (the CYC kernels): row 0 couples to x(M-1) through beta (AM(1)) and row
     // M-1 to x(0) through alpha (CM(M)); the tables hold 0 in those two slots
     T alpha, beta;
 };
 
-// One block of 256/P lines (logical line block `lb`). CYC: periodic lines, solved as the
-// tridiagonal part T' plus a rank-one correction (Sherman-Morrison, the method of the
-// reference's CYCLIC, numrec.f:754-781): T = T' + u v^T with u = (g, 0, ..., 0, alpha),
-// v = (1, 0, ..., 0, beta/g), g = -b(0); the elimination carries the second right-hand side
-// u beside d, and x = y - z (y_0 + beta y_{M-1}/g) / (1 + z_0 + beta z_{M-1}/g). The singular
-// line is pinned at x(0) = 0 and solved without the correction (its corner couplings act on
-// x(0) = 0).
-template <typename T, int QMAX, bool CYC = false>
-__device__ __forceinline__ void xsolve_tile(const XArgs<T>& a, int lb) {
-    extern __shared__ unsigned char smem_raw[];
-    const Dims d = a.d;
-    const int P = a.P, Q = a.Q, M = d.M, N = d.N;
-    const int LPW = blockDim.x / P;
-    const int ldw = a.ldw;  // P*(Q+1): padded line stride in LDS
-    T* tile = reinterpret_cast<T*>(smem_raw);
-    const int tid = threadIdx.x, nthr = blockDim.x;
-    const int lw = tid / P, p = tid - (tid / P) * P;
-    // line numbers and element offsets in 32 bits: S holds fewer than 2^29 elements (the plan
-    // rejects fields of 4 GiB and more)
-    const int nlines = (int)a.lend;
-    const int line0 = (int)a.lbeg + lb * LPW;
+// LDS elements of a wave's 64 Q staged values (index e at e + e/8: a lane's Q consecutive values
+// and the staging's 64 consecutive ones both spread over the banks)
+__host__ __device__ inline int xlds_wave(int Q) { return 72 * Q + 2; }
 
-    // stage the block's lines (contiguous in S) into LDS, several loads in flight per thread;
-    // small-integer quotients through a float reciprocal (exact: the dividends stay below 2^14)
-    // and 24-bit products; global addresses as 32-bit byte offsets from the block's first line.
-    // Elements past the last line read a clamped in-range element and are zeroed afterwards.
-    T* const blk = a.S + (size_t)line0 * (size_t)M;
-    const int nel = LPW * M;
-    const int nvalid = min(nel, (nlines - line0) * M);
-    const float rM = 1.0f / (float)M, rQ = 1.0f / (float)Q;
-    constexpr int U = 8;
-    for (int e0 = tid; e0 < nel; e0 += nthr * U) {
-        T v[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-            v[u] = ld_off(blk, (unsigned)sizeof(T) * (unsigned)min(e0 + u * nthr, nvalid - 1));
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int e = e0 + u * nthr;
-            if (e >= nel) continue;
-            const int l2 = (int)(((float)e + 0.5f) * rM);
-            const int i = e - (int)__umul24(l2, M);
-            const int c = (int)(((float)i + 0.5f) * rQ);
-            tile[__umul24(l2, ldw) + i + c] = (e < nvalid) ? v[u] : T(0);  // row c*(Q+1) + (i - c*Q)
-        }
-    }
-    __syncthreads();
+// A coupling to a chunk end this small no longer reaches a result (2^-80 of its neighbour): the
+// even unknowns are decoupled and the remaining reduction steps would return them unchanged.
+// Each step squares the couplings, so on most lines (those of all but the lowest wavenumbers)
+// two or three of the log2 P steps are left over.
+constexpr double kDecoupled = 0x1p-80;
 
-    const int l = line0 + lw;
-    const bool valid = l < nlines;
-    const int j = valid ? l / N : 0;
-    const int m = valid ? l - j * N : 0;
-    const T akj = a.tb.akj[j];
-    const T lam = a.tb.lamj ? a.tb.lamj[valid ? l : 0] : a.tb.lam[m];
-    const bool pin = valid && j == 0 && m == d.null_m;
-    const T* row = tile + lw * ldw + p * (Q + 1);
+// Solve the wave's 64/P lines, P lanes and Q rows per lane (FIXED: Q = QMAX and M = P*Q, no row
+// checks). get(r) is the right-hand side of this lane's row r, put(r, x) takes its solution.
+// Returns the sum of the lane's solution rows. CYC: periodic lines, solved as the tridiagonal
+// part T' plus a rank-one correction (Sherman-Morrison, the method of the reference's CYCLIC,
+// numrec.f:754-781): T = T' + u v^T with u = (g, 0, ..., 0, alpha), v = (1, 0, ..., 0, beta/g),
+// g = -b(0); the elimination carries the second right-hand side u beside d, and
+// x = y - z (y_0 + beta y_{M-1}/g) / (1 + z_0 + beta z_{M-1}/g). The singular line is pinned at
+// x(0) = 0 and solved without the correction (its corner couplings act on x(0) = 0).
+template <typename T, int QMAX, bool FIXED, bool CYC, typename Get, typename Put>
+__device__ __forceinline__ T xsolve_lines(const XArgs<T>& a, int p, int lane, T akj, T lam, bool pin, Get get,
+                                          Put put) {
+    const int P = a.P, Q = FIXED ? QMAX : a.Q, M = a.d.M;
     // periodic line: the corrected diagonals of rows 0 and M-1 and the second right-hand side
-    const bool cyc = CYC && valid && !pin;
+    const bool cyc = CYC && !pin;
     const T g = CYC ? -(a.tb.bm[0] - akj * a.tb.r2inv[0] + lam) : T(0);
 
     T aa[QMAX], cc[QMAX], dd[QMAX];
     T ee[CYC ? QMAX : 1];
     const int ib = p * Q;
+    // rows in batches of 4 whose coefficients (tables in thread order: row p*Q + r at r*P + p) are
+    // loaded together; rows past M are identity rows of the tables with a zero right-hand side
+    constexpr int B = QMAX < 4 ? QMAX : 4;
 #pragma unroll
-    for (int r = 0; r < QMAX; ++r) {
-        if (r < Q) {
-            const int i = ib + r;
-            T av = T(0), cv = T(0), bv = T(1), dv = T(0);  // rows past M pad the line: x = 0
-            if (i < M) {
-                const int ti = r * P + p;  // tables in thread order (row p*Q + r)
-                av = a.tb.am[ti];
-                cv = a.tb.cm[ti];
-                bv = a.tb.bm[ti] - akj * a.tb.r2inv[ti] + lam;
-                dv = row[r];
-            }
-            if (!valid) {
-                av = T(0);
-                cv = T(0);
-                bv = T(1);
-                dv = T(0);
-            }
-            if (pin && i == 0) {
-                av = T(0);
-                bv = T(1);
-                cv = T(0);
-                dv = T(0);
+    for (int r0 = 0; r0 < QMAX; r0 += B) {
+        T ta[B], tc[B], tb[B], tr[B], td[B];
+#pragma unroll
+        for (int u = 0; u < B && r0 + u < QMAX; ++u) {
+            const int r = FIXED ? r0 + u : min(r0 + u, Q - 1);
+            const unsigned o = (unsigned)sizeof(T) * (unsigned)(r * P + p);
+            ta[u] = ld_off(a.tb.am, o);
+            tc[u] = ld_off(a.tb.cm, o);
+            tb[u] = ld_off(a.tb.bm, o);
+            tr[u] = ld_off(a.tb.r2inv, o);
+            td[u] = get(r);
+        }
+#pragma unroll
+        for (int u = 0; u < B && r0 + u < QMAX; ++u) {
+            const int r = r0 + u;
+            if (!FIXED && r >= Q) continue;
+            T av = ta[u], cv = tc[u], bv = tb[u] - akj * tr[u] + lam;
+            T dv = (FIXED || ib + r < M) ? td[u] : T(0);
+            if (r == 0) {  // the singular line: x(0) = 0
+                const bool z = pin && p == 0;
+                av = z ? T(0) : av;
+                bv = z ? T(1) : bv;
+                cv = z ? T(0) : cv;
+                dv = z ? T(0) : dv;
             }
             T ev = T(0);
             if (CYC && cyc) {
-                if (i == 0) {
+                if (ib + r == 0) {
                     bv = bv - g;
                     ev = g;
                 }
-                if (i == M - 1) {
+                if (ib + r == M - 1) {
                     bv = bv - a.alpha * a.beta / g;
                     ev = a.alpha;
                 }
@@ -212,7 +191,6 @@ __device__ __forceinline__ void xsolve_tile(const XArgs<T>& a, int lb) {
     // multiplied by 0.
     T a0 = aa[0], c0 = cc[0], d0 = dd[0], e0 = CYC ? ee[0] : T(0);
     const T a1 = lastA, c1 = lastC, d1 = lastD, e1 = lastE;
-    const int lane = tid & 63;
     {  // even row 2p minus a0 * row 2p-1 (lane p-1's odd row) minus c0 * row 2p+1 (own odd row)
         const int up = ((lane - 1) & 63) << 2;
         const T ua = lane_get(a1, up), uc = lane_get(c1, up), ud = lane_get(d1, up);
@@ -224,6 +202,7 @@ __device__ __forceinline__ void xsolve_tile(const XArgs<T>& a, int lb) {
         d0 = nd0;
     }
     for (int dl = 1; dl < P; dl <<= 1) {  // even rows at distance dl lanes
+        if (!__any(fabs(a0) > T(kDecoupled) || fabs(c0) > T(kDecoupled))) break;
         const int up = ((lane - dl) & 63) << 2, dn = ((lane + dl) & 63) << 2;
         const T ua = lane_get(a0, up), uc = lane_get(c0, up), ud = lane_get(d0, up);
         const T va = lane_get(a0, dn), vc = lane_get(c0, dn), vd = lane_get(d0, dn);
@@ -256,12 +235,11 @@ __device__ __forceinline__ void xsolve_tile(const XArgs<T>& a, int lb) {
         zM = lane_get(zM, (first + pl1) << 2);
         if (cyc) fact = (y0l + a.beta * yM / g) / (T(1) + z0l + a.beta * zM / g);
     }
-    // back-substitute into LDS (own rows only), accumulate the line sum
-    T* wrow = tile + lw * ldw + p * (Q + 1);
+    // back-substitute (own rows only), accumulate the line sum
     T part = T(0);
 #pragma unroll
     for (int r = 0; r < QMAX; ++r) {
-        if (r < Q) {
+        if (FIXED || r < Q) {
             T x;
             if (r == 0) x = x0;
             else if (r == Q - 1) x = xl;
@@ -273,27 +251,103 @@ __device__ __forceinline__ void xsolve_tile(const XArgs<T>& a, int lb) {
                 else z = ee[r] - aa[r] * z0 - cc[r] * zl;
                 x -= fact * z;
             }
-            wrow[r] = x;
+            put(r, x);
             part += x;
         }
     }
+    return part;
+}
+
+// One block of 256/P lines (logical line block `lb`), 64/P lines per wave.
+template <typename T, int QMAX, bool FIXED, bool CYC = false>
+__device__ __forceinline__ void xsolve_tile(const XArgs<T>& a, int lb) {
+    extern __shared__ unsigned char smem_raw[];
+    const Dims d = a.d;
+    const int P = a.P, Q = FIXED ? QMAX : a.Q, M = d.M, N = d.N;
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int LW = 64 / P;  // lines per wave
+    T* const tile = reinterpret_cast<T*>(smem_raw) + w * xlds_wave(Q);
+    // line numbers and element offsets in 32 bits: S holds fewer than 2^29 elements (the plan
+    // rejects fields of 4 GiB and more)
+    const int line0 = (int)a.lbeg + (lb * 4 + w) * LW;
+    const int nl = min(LW, (int)a.lend - line0);  // the wave's lines
+    if (nl <= 0) return;
+
+    // The wave's lines, contiguous in S, into its LDS: element lane + 64 u, every load in flight
+    // together; elements past the last line read the last one (finite values for lanes whose
+    // results are not stored)
+    T* const blk = a.S + (size_t)line0 * (size_t)M;
+    const int nel = nl * M;
+    const int wi = lane + (lane >> 3);
+    {
+        T v[QMAX];
+        if (nel == 64 * QMAX) {  // wave-uniform
+#pragma unroll
+            for (int u = 0; u < QMAX; ++u) v[u] = blk[lane + 64 * u];
+        } else {
+#pragma unroll
+            for (int u = 0; u < QMAX; ++u)
+                v[u] = ld_off(blk, (unsigned)sizeof(T) * (unsigned)min(lane + 64 * u, nel - 1));
+        }
+#pragma unroll
+        for (int u = 0; u < QMAX; ++u)
+            if (FIXED || u < Q) tile[wi + 72 * u] = v[u];
+    }
+    // the wave's LDS operations complete in order; this only keeps the compiler from moving them
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+
+    const int lw = lane / P, p = lane - lw * P;
+    const int l = line0 + min(lw, nl - 1);
+    int j, m;
+    if (LW <= N) {  // one quotient for the wave
+        const int j0 = line0 / N;
+        m = line0 - j0 * N + (l - line0);
+        j = j0;
+        if (m >= N) {
+            m -= N;
+            ++j;
+        }
+    } else {
+        j = l / N;
+        m = l - j * N;
+    }
+    const T akj = a.tb.akj[j];
+    const T lam = a.tb.lamj ? a.tb.lamj[l] : a.tb.lam[m];
+    const bool pin = j == 0 && m == d.null_m;
+    // the lane's rows: elements e0 + r of the wave's region
+    const int e0 = FIXED ? lane * QMAX : lw * M + p * Q;
+    auto at = [&](int r) { return e0 + r + ((e0 + r) >> 3); };
+    T part = xsolve_lines<T, QMAX, FIXED, CYC>(
+        a, p, lane, akj, lam, pin,
+        [&](int r) { return tile[FIXED ? at(r) : min(at(r), xlds_wave(Q) - 1)]; },
+        [&](int r, T x) {
+            if (FIXED || p * Q + r < M) tile[at(r)] = x;
+        });
     if (j == 0) {
         // reduce over the P lanes of this line (consecutive lanes of one wave, P <= 64)
         for (int off = P >> 1; off > 0; off >>= 1) part += __shfl_xor(part, off, 64);
-        if (valid && p == 0) a.linesum[m] = part;
+        if (lw < nl && p == 0) a.linesum[m] = part;
     }
-    __syncthreads();
-    for (int e = tid; e < nvalid; e += nthr) {
-        const int l2 = (int)(((float)e + 0.5f) * rM);
-        const int i = e - (int)__umul24(l2, M);
-        const int c = (int)(((float)i + 0.5f) * rQ);
-        st_off(blk, (unsigned)sizeof(T) * (unsigned)e, tile[__umul24(l2, ldw) + i + c]);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    if (nel == 64 * QMAX) {
+#pragma unroll
+        for (int u = 0; u < QMAX; ++u) blk[lane + 64 * u] = tile[wi + 72 * u];
+    } else {
+#pragma unroll
+        for (int u = 0; u < QMAX; ++u)
+            if (lane + 64 * u < nel) st_off(blk, (unsigned)sizeof(T) * (unsigned)(lane + 64 * u), tile[wi + 72 * u]);
     }
 }
 
-template <typename T, int QMAX, bool CYC>
-__global__ void __launch_bounds__(256) k_xsolve(XArgs<T> a) {
-    xsolve_tile<T, QMAX, CYC>(a, xcd_tile(blockIdx.x, gridDim.x));
+template <typename T, int QMAX, bool FIXED, bool CYC>
+__global__ void __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 && FIXED ? (QMAX <= 8 ? 6 : 4) : 1)))
+k_xsolve(XArgs<T> a) {
+    xsolve_tile<T, QMAX, FIXED, CYC>(a, xcd_tile(blockIdx.x, gridDim.x));
 }
 
 // Pick P (threads per line, a power of two <= 64) and Q (rows per thread, 3 <= Q <= qmax):
@@ -321,16 +375,29 @@ static bool pick_pq_any(int M, int chunk, int& P, int& Q) {
 
 bool xsolve_partition(int M, int chunk, int& P, int& Q) { return pick_pq_any(M, chunk, P, Q); }
 
-template <typename T, bool CYC>
-static void launch_xsolve_q(hipStream_t st, dim3 grid, size_t sh, const XArgs<T>& a) {
-    auto go = [&](auto fn) {
-        (void)hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sh);
-        hipLaunchKernelGGL(fn, grid, dim3(256), sh, st, a);
-    };
-    if (a.Q <= 4) go(k_xsolve<T, 4, CYC>);
-    else if (a.Q <= 8) go(k_xsolve<T, 8, CYC>);
-    else if (a.Q <= 16) go(k_xsolve<T, 16, CYC>);
-    else go(k_xsolve<T, 32, CYC>);
+// Kernel template of a line length: the exact splits M = P*Q with Q of the usual grids have their
+// own (kFixed + Q: no row checks, constant LDS offsets), every other split runs the smallest
+// template of at least Q rows.
+constexpr int kFixed = 64;
+static int xsolve_class(int M, int P, int Q, bool cyc) {
+    if (!cyc && P * Q == M && (Q == 6 || Q == 8 || Q == 10 || Q == 12 || Q == 16)) return kFixed + Q;
+    return Q <= 4 ? 4 : (Q <= 8 ? 8 : (Q <= 16 ? 16 : 32));
+}
+
+// go(integral QMAX, FIXED) of a class
+template <typename Go>
+static void xsolve_dispatch(int cls, Go go) {
+    switch (cls) {
+        case kFixed + 6: go(std::integral_constant<int, 6>{}, std::true_type{}); break;
+        case kFixed + 8: go(std::integral_constant<int, 8>{}, std::true_type{}); break;
+        case kFixed + 10: go(std::integral_constant<int, 10>{}, std::true_type{}); break;
+        case kFixed + 12: go(std::integral_constant<int, 12>{}, std::true_type{}); break;
+        case kFixed + 16: go(std::integral_constant<int, 16>{}, std::true_type{}); break;
+        case 4: go(std::integral_constant<int, 4>{}, std::false_type{}); break;
+        case 8: go(std::integral_constant<int, 8>{}, std::false_type{}); break;
+        case 16: go(std::integral_constant<int, 16>{}, std::false_type{}); break;
+        default: go(std::integral_constant<int, 32>{}, std::false_type{}); break;
+    }
 }
 
 template <typename T>
@@ -347,31 +414,35 @@ int launch_xsolve(hipStream_t st, const Dims& d, const Tables<T>& tb, T* S, T* l
     if (!pick_pq_any(d.M, chunk, P, Q)) return -1;
     a.P = P;
     a.Q = Q;
-    a.ldw = P * (a.Q + 1);
     const int LPW = 256 / P;
     a.lbeg = (long)j0 * d.N;
     a.lend = (long)(j0 + nj) * d.N;
     const long nlines = a.lend - a.lbeg;
     dim3 grid((unsigned)((nlines + LPW - 1) / LPW));
-    size_t sh = (size_t)LPW * a.ldw * sizeof(T);
-    if (cyc) launch_xsolve_q<T, true>(st, grid, sh, a);
-    else launch_xsolve_q<T, false>(st, grid, sh, a);
+    const size_t sh = 4 * (size_t)xlds_wave(Q) * sizeof(T);
+    xsolve_dispatch(xsolve_class(d.M, P, Q, cyc != 0), [&](auto qmax, auto fixed) {
+        auto go = [&](auto fn) {
+            (void)hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sh);
+            hipLaunchKernelGGL(fn, grid, dim3(256), sh, st, a);
+        };
+        if constexpr (decltype(fixed)::value) go(k_xsolve<T, decltype(qmax)::value, true, false>);
+        else if (cyc) go(k_xsolve<T, decltype(qmax)::value, false, true>);
+        else go(k_xsolve<T, decltype(qmax)::value, false, false>);
+    });
     return 0;
 }
 
 // ------------------------------------------------------------------ batched (one item per workgroup)
 // One kernel per rows-per-thread template: a kernel holding every template would take the
 // registers of the largest (QMAX = 32) for all problems.
-template <typename T, int QMAX>
-// the 16-row class at no more than 128 VGPRs in FP64 (4 workgroups per CU; 130 unbounded) and
-// 80 in FP32 (6 workgroups per CU; 83 unbounded)
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(QMAX == 16 ? (sizeof(T) == 4 ? 6 : 4) : 1)))
+// Bounds where the unbounded kernel sits just above an occupancy step (8 rows: 86 VGPRs, 6 waves
+// per SIMD at 80; 16 rows: 148, 4 waves at 128).
+template <typename T, int QMAX, bool FIXED>
+__global__ void __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 && FIXED ? (QMAX <= 8 ? 6 : 4) : 1)))
 k_batch_xsolve(const Job<XArgs<T>>* jobs, int njobs, int total) {
-    run_item(jobs, njobs, total, [](const Job<XArgs<T>>& J, int t) { xsolve_tile<T, QMAX>(J.a, t); });
+    run_item(jobs, njobs, total, [](const Job<XArgs<T>>& J, int t) { xsolve_tile<T, QMAX, FIXED>(J.a, t); });
 }
-
-
-static int qmax_class(int Q) { return Q <= 4 ? 4 : (Q <= 8 ? 8 : (Q <= 16 ? 16 : 32)); }
 
 template <typename T>
 int prepare_xsolve(const std::vector<BatchProblem<T>>& pr, StageLaunch& out, std::vector<void*>& owned) {
@@ -382,12 +453,13 @@ int prepare_xsolve(const std::vector<BatchProblem<T>>& pr, StageLaunch& out, std
     for (int idx = 0; idx < (int)pr.size(); ++idx) {
         int P = 0, Q = 0;
         if (!pick_pq_any(pr[idx].d.M, pr[idx].chunk, P, Q)) return -2;
-        items.push_back({idx, P, Q, qmax_class(Q)});
+        items.push_back({idx, P, Q, xsolve_class(pr[idx].d.M, P, Q, false)});
     }
-    auto lds_of = [&](const Item& it) { return (size_t)(256 / it.P) * it.P * (it.Q + 1) * sizeof(T); };
-    // grouped by template class (largest first); the tiles of most LDS first, then the
+    auto lds_of = [&](const Item& it) { return 4 * (size_t)xlds_wave(it.Q) * sizeof(T); };
+    // grouped by template class (most rows first); the tiles of most LDS first, then the
     // longest x1 lines
     std::stable_sort(items.begin(), items.end(), [&](const Item& x, const Item& y) {
+        if (x.cls % kFixed != y.cls % kFixed) return x.cls % kFixed > y.cls % kFixed;
         if (x.cls != y.cls) return x.cls > y.cls;
         const int ox = lds_occupancy(lds_of(x)), oy = lds_occupancy(lds_of(y));
         return ox != oy ? ox < oy : pr[x.idx].d.M > pr[y.idx].d.M;
@@ -404,7 +476,6 @@ int prepare_xsolve(const std::vector<BatchProblem<T>>& pr, StageLaunch& out, std
         a.tb = p.tb;
         a.P = it.P;
         a.Q = it.Q;
-        a.ldw = it.P * (a.Q + 1);
         a.lbeg = 0;
         a.lend = (long)p.d.L * p.d.N;
         const int LPW = 256 / it.P;
@@ -416,25 +487,18 @@ int prepare_xsolve(const std::vector<BatchProblem<T>>& pr, StageLaunch& out, std
     return upload_jobs(jobs, out, owned);
 }
 
-template <typename T, int QMAX>
-static void batch_xsolve_class(hipStream_t st, const StageLaunch& sl, int c) {
-    auto fn = k_batch_xsolve<T, QMAX>;
-    const size_t lds = sl.cls_lds[c];
-    (void)hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    const int total = sl.cls_total[c];
-    const Job<XArgs<T>>* jobs = (const Job<XArgs<T>>*)sl.jobs + sl.cls_job[c];
-    hipLaunchKernelGGL(fn, dim3(std::max(total, 1)), dim3(256), lds, st, jobs, sl.cls_job[c + 1] - sl.cls_job[c], total);
-}
-
 template <typename T>
 void batch_xsolve(hipStream_t st, const StageLaunch& sl) {
     for (int c = 0; c < sl.ncls; ++c) {
-        switch (sl.cls_q[c]) {
-            case 4: batch_xsolve_class<T, 4>(st, sl, c); break;
-            case 8: batch_xsolve_class<T, 8>(st, sl, c); break;
-            case 16: batch_xsolve_class<T, 16>(st, sl, c); break;
-            default: batch_xsolve_class<T, 32>(st, sl, c); break;
-        }
+        xsolve_dispatch(sl.cls_q[c], [&](auto qmax, auto fixed) {
+            auto fn = k_batch_xsolve<T, decltype(qmax)::value, decltype(fixed)::value>;
+            const size_t lds = sl.cls_lds[c];
+            (void)hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+            const int total = sl.cls_total[c];
+            const Job<XArgs<T>>* jobs = (const Job<XArgs<T>>*)sl.jobs + sl.cls_job[c];
+            hipLaunchKernelGGL(fn, dim3(std::max(total, 1)), dim3(256), lds, st, jobs, sl.cls_job[c + 1] - sl.cls_job[c],
+                               total);
+        });
     }
 }
 
