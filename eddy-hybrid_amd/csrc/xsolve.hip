@@ -343,11 +343,15 @@ __device__ __forceinline__ void xsolve_tile(const XArgs<T>& a, int lb) {
     }
 }
 
+// The lines are walked from the last to the first, against the order of the x2 transforms on both
+// sides: each then starts on what the pass before it left in the 256 MiB memory-side cache. At
+// 768 x 384 x 256 (a spectrum of 604 MB) this solve takes 0.284 ms instead of 0.310 and the inverse
+// x2 transform 0.369 instead of 0.387; nothing changes at 512 x 256 x 256 (268 MB) and below.
 template <typename T, int QMAX, bool FIXED, bool CYC>
 __global__ void __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 && FIXED ? (QMAX <= 8 ? 6 : 4) : 1)))
 k_xsolve(XArgs<T> a) {
-    xsolve_tile<T, QMAX, FIXED, CYC>(a, xcd_tile(blockIdx.x, gridDim.x));
+    xsolve_tile<T, QMAX, FIXED, CYC>(a, xcd_tile(gridDim.x - 1 - blockIdx.x, gridDim.x));
 }
 
 // Pick P (threads per line, a power of two <= 64) and Q (rows per thread, 3 <= Q <= qmax):
