@@ -22,25 +22,14 @@ struct Job {
     int aux;     // stage-specific: x2 transform kind, x1-solve rows-per-thread class, y blocks per plane
 };
 
-// Item of workgroup b when runs of C consecutive items share an XCD. Workgroups are dealt
-// to the 8 XCDs in turn (XCD b % 8), so workgroup b takes item ((s / C) * 8 + b % 8) * C + s % C
-// with s = b / 8: a tile's x1 and x2 neighbours (the items next to it) are read through the
-// same L2. Bijective on the first total - total % (8 C) items; the rest keep item b.
-__device__ __forceinline__ int xcd_run(int b, int total, int C) {
-    const int full = total - total % (8 * C);
-    if (b >= full) return b;
-    const int s = b >> 3;
-    return ((s / C) * 8 + (b & 7)) * C + s % C;
-}
-
 constexpr int kXcdRun = 64;
 
 // The item of this workgroup (launches have exactly `total` workgroups).
-template <typename Args, typename Body>
+template <int RUN = kXcdRun, typename Args, typename Body>
 __device__ __forceinline__ void run_item(const Job<Args>* __restrict__ jobs, int njobs, int total, Body body) {
     const int b = __builtin_amdgcn_readfirstlane((int)blockIdx.x);
     if (b >= total) return;
-    const int it = xcd_run(b, total, kXcdRun);
+    const int it = xcd_run(b, total, RUN);
     int lo = 0, hi = njobs - 1;
     while (lo < hi) {
         const int mid = (lo + hi + 1) >> 1;

@@ -93,6 +93,18 @@ __device__ __forceinline__ int xcd_tile(int b, int n) {
     return x * q + (x < r ? x : r) + (b >> 3);
 }
 
+// Item of workgroup b when runs of C consecutive items share an XCD. Workgroups are dealt
+// to the 8 XCDs in turn (XCD b % 8), so workgroup b takes item ((s / C) * 8 + b % 8) * C + s % C
+// with s = b / 8: an item's neighbours are read through the same L2, and the eight XCDs stay
+// within 8 C items of each other. Bijective on the first total - total % (8 C) items; the rest
+// keep item b.
+__device__ __forceinline__ int xcd_run(int b, int total, int C) {
+    const int full = total - total % (8 * C);
+    if (b >= full) return b;
+    const int s = b >> 3;
+    return ((s / C) * 8 + (b & 7)) * C + s % C;
+}
+
 // Tiles (ix, k) of an ntx x nk grid taken in blocks of W consecutive ix: ix fastest within a
 // block, then k, then the block (the last block may be narrower). Consecutive logical tiles
 // then walk down x2 over a narrow x1 range, so a tile's x2 neighbour planes were touched a few

@@ -171,8 +171,9 @@ struct StageLaunch {
     int cls_total[kMaxClasses] = {};
     size_t cls_lds[kMaxClasses] = {};
     // the forward y transform with the divergence: 1 every problem Cartesian, 2 every one
-    // cylindrical (a kernel with only that metric's registers), 0 mixed
+    // cylindrical (a kernel with only that metric's registers), 0 mixed; CORRECT: 1 the span kernel
     int kind = 0;
+    const double* alf = nullptr;  // CORRECT: device {ALFXDT, 1/ALFXDT}
 };
 
 // Workgroups of 256 threads that one CU holds at once when each takes `lds` bytes of its

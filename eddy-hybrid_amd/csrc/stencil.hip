@@ -88,7 +88,8 @@ __global__ void __launch_bounds__(256) k_div_minmax(Dims d, Metrics mt, const do
     block_partial<RED_OP_MAX>(mx, part + nb, linear_bid());
 }
 
-// Rows of CORRECT per thread: rows j0, j0 + 4, ... of a block of 64 x1 cells by 4 * kCorrectRows
+// CORRECT of fields that are not all 16-byte aligned (k_correct_span takes the others).
+// Rows per thread: rows j0, j0 + 4, ... of a block of 64 x1 cells by 4 * kCorrectRows
 // y rows; every load of a thread is issued before its first store (rows past L load a clamped
 // in-range row and store nothing). Addresses are 32-bit byte offsets (fields below 4 GiB).
 constexpr int kCorrectRows = 2;
@@ -159,6 +160,158 @@ __global__ void __launch_bounds__(256) k_correct(Dims d, Metrics mt, const doubl
             if (ghost) st_off(wo, o[q] + (unsigned)gofs, wn);
         }
     }
+}
+
+// CORRECT along memory instead of along rows: the interior rows J = 1..L of a plane are one span
+// of L*nx consecutive elements, cut into blocks of 512 * kSpanParts elements that start on a
+// 128-byte line (when the bases do), two neighbouring elements per lane and part. Every access of
+// the six velocity fields and of dp is then a whole aligned 1 KiB per wave, where a 64-cell block of
+// a row (nx = M + 2 elements, starting one past a ghost) straddles five lines with partial lines at
+// both ends, read and written by two blocks. The ghosts inside the span (4 of nx) are loaded and
+// not stored. Needs 16-byte aligned fields (the row kernel above takes the others). HBM bound;
+// with the streamed velocities and the block order below 0.398 -> 0.343 ms at 512 x 256 x 256,
+// 0.493 -> 0.407 ms at 302 x 130 x 1026, 0.058 -> 0.044 ms at 300 x 128 x 128.
+constexpr int kSpanParts = 2;
+constexpr int kSpan = 512 * kSpanParts;  // elements per block
+
+typedef double d2 __attribute__((ext_vector_type(2)));
+typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));  // rows of odd nx
+
+struct CorrArgs {
+    Dims d;
+    Metrics mt;
+    const double *us, *vs, *ws;
+    double *uo, *vo, *wo;
+    const double* dp;
+    unsigned rnx;  // ceil(2^32 / nx)
+};
+
+// Blocks of a plane's span (its start rounded down to 16 elements).
+__host__ __device__ inline int span_blocks(const Dims& d) { return ceil_div(d.L * d.nx + 15, kSpan); }
+
+// The velocities are streamed (read once, written once): non-temporal, so that they do not push
+// dp's planes out of L2 nor the solve's arrays out of the memory-side cache.
+template <typename V>
+__device__ __forceinline__ V ld_stream(const double* b, unsigned off) {
+    return __builtin_nontemporal_load(reinterpret_cast<const V*>(reinterpret_cast<const char*>(b) + off));
+}
+template <typename V>
+__device__ __forceinline__ void st_stream(double* b, unsigned off, V v) {
+    __builtin_nontemporal_store(v, reinterpret_cast<V*>(reinterpret_cast<char*>(b) + off));
+}
+
+// Block `b` of plane k's span (k 0-based interior).
+__device__ __forceinline__ void correct_span(const CorrArgs& c, double alfxdt, int refresh, int k, int b, int tid) {
+    const Dims& d = c.d;
+    const unsigned nx = (unsigned)d.nx, pl = nx * (unsigned)d.ny;
+    const unsigned plane = pl * (unsigned)(k + 1);
+    const unsigned e0 = ((plane + nx) & ~15u) + (unsigned)b * kSpan + 2u * (unsigned)tid;
+    const double cwK = c.mt.cw[k + 1];
+    const bool wface = k + 1 <= d.nz - 3 + d.cyc_z;
+    const int ulast = d.nx - 3 + d.cyc_x, vlast = d.ny - 2 - d.ycopy;
+    unsigned o[kSpanParts];
+    int I[kSpanParts], J[kSpanParts];
+    bool on[kSpanParts];
+    d2 p0[kSpanParts], u[kSpanParts], v[kSpanParts], w[kSpanParts];
+    d2u pn[kSpanParts], pt[kSpanParts];
+    double pe[kSpanParts];
+#pragma unroll
+    for (int q = 0; q < kSpanParts; ++q) {
+        const unsigned r = e0 + 512u * q - plane;  // element of the plane (>= nx - 15)
+        int j = (int)__umulhi(r, c.rnx);           // exact or one too large
+        int i = (int)(r - (unsigned)j * nx);
+        if (i < 0) {
+            --j;
+            i += d.nx;
+        }
+        // pairs that hold an interior cell: elements (i, j), (i + 1, j), or (0, j + 1) past a row's end
+        on[q] = j >= 1 && j <= d.L && i <= d.M;
+        I[q] = i;
+        J[q] = j;
+        o[q] = 8u * (e0 + 512u * q);
+        if (!on[q]) o[q] = 8u * (plane + nx);
+        p0[q] = ld_off(reinterpret_cast<const d2*>(c.dp), o[q] & ~15u);
+        pe[q] = ld_off(c.dp, (o[q] & ~15u) + 16u);
+        pn[q] = ld_off(reinterpret_cast<const d2u*>(c.dp), (o[q] & ~15u) + 8u * nx);
+        pt[q] = ld_off(reinterpret_cast<const d2u*>(c.dp), (o[q] & ~15u) + 8u * pl);
+        u[q] = ld_stream<d2>(c.us, o[q] & ~15u);
+        v[q] = ld_stream<d2>(c.vs, o[q] & ~15u);
+        w[q] = ld_stream<d2>(c.ws, o[q] & ~15u);
+    }
+#pragma unroll
+    for (int q = 0; q < kSpanParts; ++q) {
+        if (!on[q]) continue;
+        const int i = I[q], j = J[q];
+        const int i1 = min(i + 1, d.nx - 1);
+        const double bvJ = c.mt.bv[j];
+        d2 un, vn, wn;
+        un.x = u[q].x - c.mt.au[i] * (p0[q].y - p0[q].x) * alfxdt;
+        un.y = u[q].y - c.mt.au[i1] * (pe[q] - p0[q].y) * alfxdt;
+        const double gx = bvJ * (pn[q].x - p0[q].x) * alfxdt, gy = bvJ * (pn[q].y - p0[q].y) * alfxdt;
+        vn.x = v[q].x - (c.mt.cart ? gx : gx / c.mt.rp[i]);
+        vn.y = v[q].y - (c.mt.cart ? gy : gy / c.mt.rp[i1]);
+        wn.x = w[q].x - cwK * (pt[q].x - p0[q].x) * alfxdt;
+        wn.y = w[q].y - cwK * (pt[q].y - p0[q].y) * alfxdt;
+        const bool a0 = i >= 1, a1 = i + 1 <= d.M;  // the pair's interior cells
+        const bool u0 = a0 && i <= ulast, u1 = a1 && i + 1 <= ulast;
+        const bool vf = j <= vlast;
+        auto put = [&](double* f, unsigned at, d2 x, bool s0, bool s1) {
+            if (s0 && s1) st_stream<d2u>(f, at, x);
+            else if (s0) st_off(f, at, x.x);
+            else if (s1) st_off(f, at + 8u, x.y);
+        };
+        if (a0 && a1 && u0 && u1) {
+            st_stream<d2>(c.uo, o[q], un);
+            if (vf) st_stream<d2>(c.vo, o[q], vn);
+            if (wface) st_stream<d2>(c.wo, o[q], wn);
+        } else {
+            put(c.uo, o[q], un, u0, u1);
+            if (vf) put(c.vo, o[q], vn, a0, a1);
+            if (wface) put(c.wo, o[q], wn, a0, a1);
+        }
+        // periodic y ghost rows of the corrected faces (the velocity BC step after CORRECT,
+        // Eddy6.f:2746-2761): row J=1 mirrors J=NY-1, row J=NY mirrors J=2
+        if (refresh && !d.ycopy && (j == 1 || j == d.L)) {
+            const unsigned g = o[q] + (j == d.L ? 0u - 8u * nx * (unsigned)(d.ny - 2) : 8u * nx * (unsigned)(d.ny - 2));
+            put(c.uo, g, un, u0, u1);
+            if (vf) put(c.vo, g, vn, a0, a1);
+            if (wface) put(c.wo, g, wn, a0, a1);
+        }
+    }
+}
+
+// Item t of a problem's nb x N blocks, the planes in pairs (dp's plane k + 1, read with plane k, is
+// then read again by the block after it).
+__device__ __forceinline__ void correct_item(const CorrArgs& c, double alfxdt, int refresh, int t, int nb) {
+    const int c0 = t / (2 * nb), r = t - c0 * 2 * nb, kc = min(2, c.d.N - 2 * c0);
+    const int b = r / kc;
+    correct_span(c, alfxdt, refresh, 2 * c0 + r - b * kc, b, (int)threadIdx.x);
+}
+
+// The XCDs share the field in runs of kCorrectRun blocks, so that the eight of them work within a
+// window of it, once the fields exceed the 256 MiB memory-side cache: 0.392 -> 0.343 ms at
+// 512 x 256 x 256 (5.5 TB/s of 56 B/cell; runs of 2 to 64 within 2 %) and 0.457 -> 0.415 ms at
+// 302 x 130 x 1026 over one contiguous eighth per XCD, which ties up 56 far-apart streams. Smaller
+// fields come out of the cache and take the eighths (256 x 128 x 128: 0.0385 against 0.0397 ms).
+constexpr int kCorrectRun = 16;
+
+__global__ void __launch_bounds__(256) k_correct_span(CorrArgs c, double alfxdt, int refresh, int runs,
+                                                      const double* __restrict__ dscale) {
+    const int b = blockIdx.x, n = gridDim.x;
+    if (dscale) alfxdt = dscale[0];
+    correct_item(c, alfxdt, refresh, runs ? xcd_run(b, n, kCorrectRun) : xcd_tile(b, n), n / c.d.N);
+}
+
+// The bases of every field at 16 bytes, as correct_span's pairs need them.
+static bool pairs_aligned(const double* us, const double* vs, const double* ws, const double* uo, const double* vo,
+                          const double* wo, const double* dp) {
+    return (((uintptr_t)us | (uintptr_t)vs | (uintptr_t)ws | (uintptr_t)uo | (uintptr_t)vo | (uintptr_t)wo |
+             (uintptr_t)dp) & 15) == 0;
+}
+
+static CorrArgs corr_args(const Dims& d, const Metrics& mt, const double* us, const double* vs, const double* ws,
+                          double* uo, double* vo, double* wo, const double* dp) {
+    return CorrArgs{d, mt, us, vs, ws, uo, vo, wo, dp, (unsigned)(((1ull << 32) + d.nx - 1) / d.nx)};
 }
 
 __global__ void __launch_bounds__(256) k_laplacian(Dims d, Op64 op, const double* __restrict__ phi,
@@ -416,6 +569,14 @@ __global__ void __launch_bounds__(256) k_batch_cells(const Job<CellArgs>* jobs, 
     run_item(jobs, njobs, total, [](const Job<CellArgs>& J, int t) { cell_tile<OP>(J.a, t, J.ntx, J.aux); });
 }
 
+// CORRECT of a batch whose fields are all 16-byte aligned; alf = {ALFXDT, 1/ALFXDT} on the device.
+__global__ void __launch_bounds__(256) k_batch_correct(const Job<CorrArgs>* jobs, int njobs, int total,
+                                                       const double* __restrict__ alf) {
+    const double alfxdt = alf[0];
+    run_item<kCorrectRun>(jobs, njobs, total,
+                          [=](const Job<CorrArgs>& J, int t) { correct_item(J.a, alfxdt, 1, t, J.ntx); });
+}
+
 template <typename T>
 static int prepare_cells_t(const std::vector<BatchProblem<T>>& pr, int op, StageLaunch& out,
                            std::vector<void*>& owned) {
@@ -459,7 +620,21 @@ static int prepare_cells_t(const std::vector<BatchProblem<T>>& pr, int op, Stage
 }
 
 int prepare_cells(const std::vector<BatchProblem<double>>& pr, int op, StageLaunch& out, std::vector<void*>& owned) {
-    return prepare_cells_t(pr, op, out, owned);
+    bool pairs = op == BC_CORRECT;
+    for (const auto& p : pr) pairs = pairs && pairs_aligned(p.us, p.vs, p.ws, p.uo, p.vo, p.wo, p.dp);
+    if (!pairs) return prepare_cells_t(pr, op, out, owned);
+    std::vector<Job<CorrArgs>> jobs;
+    out = StageLaunch{};
+    for (const auto& p : pr) {
+        Job<CorrArgs> j{};
+        j.a = corr_args(p.d, p.mt, p.us, p.vs, p.ws, p.uo, p.vo, p.wo, p.dp);
+        j.ntx = span_blocks(p.d);
+        j.ntiles = j.ntx * p.d.N;
+        if (!add_class_job(out, jobs, j, 0, 0)) return -1;
+    }
+    out.kind = 1;
+    out.alf = pr.empty() ? nullptr : pr[0].dscale;
+    return upload_jobs(jobs, out, owned);
 }
 int prepare_cells_f(const std::vector<BatchProblem<float>>& pr, int op, StageLaunch& out,
                     std::vector<void*>& owned) {
@@ -467,6 +642,11 @@ int prepare_cells_f(const std::vector<BatchProblem<float>>& pr, int op, StageLau
 }
 
 void batch_cells(hipStream_t st, const StageLaunch& sl, int op) {
+    if (op == BC_CORRECT && sl.kind == 1) {
+        hipLaunchKernelGGL(k_batch_correct, dim3(std::max(sl.total, 1)), dim3(256), 0, st,
+                           (const Job<CorrArgs>*)sl.jobs, sl.njobs, sl.total, sl.alf);
+        return;
+    }
     auto go = [&](auto fn) {
         hipLaunchKernelGGL(fn, dim3(std::max(sl.total, 1)), dim3(256), 0, st, (const Job<CellArgs>*)sl.jobs, sl.njobs,
                            sl.total);
@@ -532,6 +712,12 @@ void launch_div_minmax(hipStream_t st, const Dims& d, const Metrics& mt, const d
 void launch_correct(hipStream_t st, const Dims& d, const Metrics& mt, const double* us, const double* vs,
                     const double* ws, double* uo, double* vo, double* wo, const double* dp, double alfxdt,
                     int refresh_periodic, const double* dscale) {
+    if (pairs_aligned(us, vs, ws, uo, vo, wo, dp)) {
+        const int runs = 7 * sizeof(double) * (size_t)d.nx * d.ny * d.nz > ((size_t)256 << 20);
+        hipLaunchKernelGGL(k_correct_span, dim3(span_blocks(d) * d.N), dim3(256), 0, st,
+                           corr_args(d, mt, us, vs, ws, uo, vo, wo, dp), alfxdt, refresh_periodic, runs, dscale);
+        return;
+    }
     const dim3 grid(ceil_div(d.M, 64), ceil_div(d.L, 4 * kCorrectRows), d.N);
     hipLaunchKernelGGL(k_correct<kCorrectRows>, grid, kCellBlock, 0, st, d, mt, us, vs, ws, uo, vo, wo, dp, alfxdt,
                        refresh_periodic, dscale);
