@@ -284,8 +284,9 @@ static FwdInput direct_input(const double* src, int shift) {
     return in;
 }
 
-// forward y-FFT of the input `in` into S, x2 transform (zero y-mode shifted by
-// L*red[VOLB]/red[VOL] when zshift != 0), x1 solve, inverse x2 transform.
+// forward y-FFT of the input `in` into S, x2 transform (zero y-mode less L times the mean of the
+// RHS when zshift != 0: from the forward transform's partials, or folded into red if the input
+// asks for that), x1 solve, inverse x2 transform.
 template <typename T>
 static int solve_core(eddy_plan_s* P, const FwdInput& in, int zshift) {
     const Tables<T>& tb = tables<T>(P);
@@ -296,6 +297,11 @@ static int solve_core(eddy_plan_s* P, const FwdInput& in, int zshift) {
         KTimer kt(P, EDDY_K_YFFT_FWD);
         launch_yfft_fwd<T>(P->stream, P->d, P->fpy, tb, in, P->op, rd(P), S, P->tune.yfft_pencils,
                            P->tune.yfft_iblock);
+    }
+    MeanShift shift{};
+    if (zshift) {
+        if (in.fold) shift.red = P->red;
+        else shift = MeanShift{nullptr, P->part, ceil_div(P->d.M, P->tune.yfft_pencils) * P->d.N, P->mt.vol_total};
     }
     // The x2 transform, x1 solve and inverse x2 transform of a y-mode touch only that mode's
     // slab of S; running the three over one chunk of modes at a time keeps the chunk's slabs
@@ -310,7 +316,7 @@ static int solve_core(eddy_plan_s* P, const FwdInput& in, int zshift) {
             const Tables<T>& tz = xtables<T>(P);
             {
                 KTimer kt(P, EDDY_K_ZTRANS_FWD);
-                if (launch_xgemm_fwd<T>(P->stream, P->blas, P->d, tz, S, S2, zshift ? P->red : nullptr, j0,
+                if (launch_xgemm_fwd<T>(P->stream, P->blas, P->d, tz, S, S2, shift, j0,
                                         j1 - j0)) {
                     set_error("the forward x1 transform products failed to launch");
                     return EDDY_ERR_DEVICE;
@@ -338,13 +344,13 @@ static int solve_core(eddy_plan_s* P, const FwdInput& in, int zshift) {
         {
             KTimer kt(P, EDDY_K_ZTRANS_FWD);
             if (P->zgemm) {
-                if (launch_zgemm_fwd<T>(P->stream, P->blas, P->d, tb, S, S2, zshift ? P->red : nullptr, j0, j1 - j0)) {
+                if (launch_zgemm_fwd<T>(P->stream, P->blas, P->d, tb, S, S2, shift, j0, j1 - j0)) {
                     set_error("the forward x2 transform products failed to launch");
                     return EDDY_ERR_DEVICE;
                 }
             } else {
                 launch_ztrans_fwd<T>(P->stream, P->d, P->fpz, tb, S, P->tune.ztrans_pencils, P->dense,
-                                     zshift ? P->red : nullptr, j0, j1 - j0);
+                                     shift, j0, j1 - j0);
             }
         }
         {
@@ -463,6 +469,7 @@ static int run_refined(eddy_plan_s* P, double* dp, int sweeps, int want_resid, i
         }
         FwdInput in = *div_in;
         in.rhs_out = P->rhs;
+        in.fold = shift;  // the residuals read it too
         rc = solve_core<float>(P, in, shift);
         res_shift = shift;
     } else {
@@ -1022,10 +1029,6 @@ static int create_plan(eddy_plan_s** out, int nx, int ny, int nz, double delysq,
     if ((rc = upload64(P.get(), hvx, &P->mt.volx)) || (rc = upload64(P.get(), hvy, &P->mt.voly)) ||
         (rc = upload64(P.get(), hvz, &P->mt.volz)))
         return rc;
-    {
-        std::vector<double> vt(1, P->mt.vol_total);
-        if ((rc = upload64(P.get(), vt, &P->vol_total_dev))) return rc;
-    }
 
     // work buffers
     const size_t cells = (size_t)M * L * N;
@@ -1067,10 +1070,10 @@ static int create_plan(eddy_plan_s** out, int nx, int ny, int nz, double delysq,
         float* S32 = reinterpret_cast<float*>(P->S);
         float* S232 = reinterpret_cast<float*>(P->S2);
         const bool fail =
-            P->zgemm ? (launch_zgemm_fwd<double>(P->stream, P->blas, P->d, P->t64.t, P->S, P->S2, nullptr, 0, L) ||
-                        launch_zgemm_fwd<float>(P->stream, P->blas, P->d, P->t32.t, S32, S232, nullptr, 0, L))
-                     : (launch_xgemm_fwd<double>(P->stream, P->blas, P->d, P->tz64.t, P->S, P->S2, nullptr, 0, L) ||
-                        launch_xgemm_fwd<float>(P->stream, P->blas, P->d, P->tz32.t, S32, S232, nullptr, 0, L) ||
+            P->zgemm ? (launch_zgemm_fwd<double>(P->stream, P->blas, P->d, P->t64.t, P->S, P->S2, MeanShift{}, 0, L) ||
+                        launch_zgemm_fwd<float>(P->stream, P->blas, P->d, P->t32.t, S32, S232, MeanShift{}, 0, L))
+                     : (launch_xgemm_fwd<double>(P->stream, P->blas, P->d, P->tz64.t, P->S, P->S2, MeanShift{}, 0, L) ||
+                        launch_xgemm_fwd<float>(P->stream, P->blas, P->d, P->tz32.t, S32, S232, MeanShift{}, 0, L) ||
                         launch_xgemm_inv<double>(P->stream, P->blas, P->d, P->tz64.t, P->S2, P->S,
                                                  reinterpret_cast<double*>(P->linesum), P->dz.null_m, 0, L) ||
                         launch_xgemm_inv<float>(P->stream, P->blas, P->d, P->tz32.t, S232, S32,
@@ -1256,10 +1259,6 @@ namespace eddy {
 static int project_core(eddy_plan_s* plan, const double* us, const double* vs, const double* ws, double* uo,
                         double* vo, double* wo, double* dp, double alfxdt, const double* dscale, int remove_mean,
                         int precision, int sweeps) {
-    {
-        KTimer kt(plan, EDDY_K_OTHER);
-        launch_fill(plan->stream, plan->red, RED_COUNT, 0.0);
-    }
     int rc = 0;
     if (precision == EDDY_FP64) {
         // divergence fused into the forward y-FFT: the RHS is never written to DP, and its
@@ -1272,6 +1271,7 @@ static int project_core(eddy_plan_s* plan, const double* us, const double* vs, c
         in.mt = plan->mt;
         in.scale = 1.0 / alfxdt;
         in.dscale = dscale;
+        in.fold = remove_mean && plan->blas;  // rocBLAS products take the shift from a kernel of its own
         rc = solve_core<double>(plan, in, remove_mean);
         if (!rc) rc = finish_direct64(plan, dp);
     } else {
@@ -1558,7 +1558,6 @@ struct eddy_batch_s {
     StageLaunch d_yf, d_zf, d_xs, d_zi, d_yi;              // FP64 DIRECT
     StageLaunch d_yf_div, d_zf_shift, d_cells_corr;        // FP64 projection
     StageLaunch f_copy, f_yf, f_zf, f_xs, f_zi, f_yi_store, f_yf_res, f_yi_upd, f_shift;  // FP32 + refine
-    FoldJob* fold_div = nullptr;   // per problem: VOLB, VOL
     FoldJob* fold_phi = nullptr;   // per problem: PHISUM
     // {ALFXDT, 1/ALFXDT} of the projection, written by a fill kernel before each launch and
     // read by the kernels: one captured graph (branches) or one set of job arrays (one launch per stage)
@@ -1799,20 +1798,16 @@ int eddy_batch_bind(eddy_batch_t B, double* const* dp, const double* const* us, 
         (rc = prepare_cells_f(B->p32, BC_SHIFT_GHOSTS, B->f_shift, own)))
         return (set_error("batch preparation failed"), EDDY_ERR_DEVICE);
     // fold jobs: the y-stage partials of each problem (one slot per y tile)
-    std::vector<FoldJob> fd, fp;
+    std::vector<FoldJob> fp;
     for (int p = 0; p < n; ++p) {
         eddy_plan_s* P = B->plans[p];
         const int ntiles = ceil_div(P->d.M, P->tune.yfft_pencils) * P->d.N;
-        fd.push_back(FoldJob{P->part, ntiles, RED_OP_SUM, P->red + RED_VOLB});
-        fd.push_back(FoldJob{P->vol_total_dev, 1, RED_OP_SUM, P->red + RED_VOL});
         fp.push_back(FoldJob{P->part, ntiles, RED_OP_SUM, P->red + RED_PHISUM});
     }
     void* q = nullptr;
-    HIP_TRY(hipMalloc(&q, (fd.size() + fp.size()) * sizeof(FoldJob)));
+    HIP_TRY(hipMalloc(&q, fp.size() * sizeof(FoldJob)));
     own.push_back(q);
-    B->fold_div = static_cast<FoldJob*>(q);
-    B->fold_phi = B->fold_div + fd.size();
-    HIP_TRY(hipMemcpy(B->fold_div, fd.data(), fd.size() * sizeof(FoldJob), hipMemcpyHostToDevice));
+    B->fold_phi = static_cast<FoldJob*>(q);
     HIP_TRY(hipMemcpy(B->fold_phi, fp.data(), fp.size() * sizeof(FoldJob), hipMemcpyHostToDevice));
     B->items = std::max({(long)B->d_yf.total, (long)B->d_zf.total, (long)B->d_xs.total});
     B->bound = true;
@@ -1878,7 +1873,6 @@ int eddy_batch_project_dev(eddy_batch_t B, double alfxdt, int remove_mean) {
     }
     hipStream_t st = B->stream;
     batch_yfft<double>(st, B->d_yf_div, 1, YF_DIVERGENCE);
-    batch_fold(st, B->fold_div, 2 * (int)B->plans.size());
     batch_ztrans<double>(st, remove_mean ? B->d_zf_shift : B->d_zf, 0);
     batch_xsolve<double>(st, B->d_xs);
     batch_ztrans<double>(st, B->d_zi, 1);

@@ -81,6 +81,19 @@ enum RedSlot {
     RED_COUNT = 11
 };
 
+// Where the volume-weighted mean sum vol*b / sum vol of an RHS is read from: its two sums at
+// red[RED_VOLB] and red[RED_VOL], or the n per-workgroup partials of the first and the constant
+// second (the reader folds them itself: at 64 x 64 x 32 a projection of 9 launches takes 0.0424 ms,
+// of 6 0.0379, at 512 x 256 x 256 1.088 and 1.080; the 8192 partials of the latter cost the 32 zero-mode
+// workgroups a few us beside the others); no
+// shift when both are null.
+struct MeanShift {
+    const double* red;
+    const double* part;
+    int n;
+    double vol;
+};
+
 __host__ __device__ inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
 
 // Workgroups are dispatched round-robin over the 8 XCDs (workgroup b runs on XCD b % 8) and

@@ -59,6 +59,7 @@ struct FwdInput {
     // captured graph then serves every time step)
     const double* dscale;
     int shift;
+    int fold;         // YF_DIVERGENCE: sum vol*b and sum vol into red[RED_VOLB], red[RED_VOL]
     double* rhs_out;  // YF_DIVERGENCE of the FP32 transform: the FP64 RHS, DP layout (interior)
 };
 // YI_UPDATE_FINAL: the last update of the defect correction with its closing pass fused in:
@@ -90,11 +91,11 @@ void launch_ygemm_inv(hipStream_t st, const Dims& d, const float* GT, const floa
                       int mode);
 
 // Forward x2 transform (DCT-II when uniform, dense eigenvectors otherwise), in place on S.
-// When shift_red != null, the zero y-mode first loses L * red[RED_VOLB]/red[RED_VOL] (the
-// volume-weighted solvability shift of an RHS whose y-FFT was taken before its mean was known).
+// The zero y-mode first loses L times the mean `shift` (the volume-weighted solvability shift of
+// an RHS whose y-FFT was taken before its mean was known).
 template <typename T>
 void launch_ztrans_fwd(hipStream_t st, const Dims& d, const FftPlan& fpz, const Tables<T>& tb, T* S,
-                       int TI, int dense, const double* shift_red, int j0, int nj);
+                       int TI, int dense, const MeanShift& shift, int j0, int nj);
 // Inverse x2 transform; for the y-mode j=0 it first applies the plain-mean correction from
 // the line sums (direct.f:894-898).
 template <typename T>
@@ -105,13 +106,13 @@ void launch_ztrans_inv(hipStream_t st, const Dims& d, const FftPlan& fpz, const 
 // the plain-mean correction). Return 0, or -1 if rocBLAS refused the call.
 template <typename T>
 int launch_zgemm_fwd(hipStream_t st, void* blas, const Dims& d, const Tables<T>& tb, T* S, T* S2,
-                     const double* shift_red, int j0, int nj);
+                     const MeanShift& shift, int j0, int nj);
 template <typename T>
 int launch_zgemm_inv(hipStream_t st, void* blas, const Dims& d, const Tables<T>& tb, T* S2, T* S, const T* linesum,
                      int j0, int nj);
 template <typename T>
 int launch_xgemm_fwd(hipStream_t st, void* blas, const Dims& d, const Tables<T>& tz, T* S, T* S2,
-                     const double* shift_red, int j0, int nj);
+                     const MeanShift& shift, int j0, int nj);
 template <typename T>
 int launch_xgemm_inv(hipStream_t st, void* blas, const Dims& d, const Tables<T>& tz, T* S2, T* S, const T* linesum,
                      int null_x, int j0, int nj);

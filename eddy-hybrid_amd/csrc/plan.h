@@ -66,7 +66,6 @@ struct eddy_plan_s {
     double* part = nullptr;     // per-workgroup reduction partials
     double* rhs = nullptr;      // RHS copy for the defect correction (NX*NY*NZ), lazily allocated
     double* dp_dev = nullptr;   // device DP for the host-pointer entry point, lazily allocated
-    const double* vol_total_dev = nullptr;  // mt.vol_total on the device (batched folds read it)
     // pressure update (eddy_plan_set_pressure_bc): implicit masks (device, NX) and BC types
     const double* rvimplx = nullptr;
     const double* rvimply = nullptr;

@@ -66,4 +66,21 @@ __device__ __forceinline__ void block_partial(double v, double* part, int slot) 
     }
 }
 
+// The mean of `s` for every thread of a 1-D workgroup (of at most 16 waves, `scratch` 16 doubles of
+// LDS); every thread calls it.
+__device__ __forceinline__ double mean_shift(const MeanShift& s, double* scratch) {
+    if (s.red) return s.red[RED_VOLB] / s.red[RED_VOL];
+    if (!s.part) return 0.0;
+    const int nthr = blockDim.x;
+    double v = 0.0;
+    for (int t = threadIdx.x; t < s.n; t += nthr) v += s.part[t];
+    v = wave_sum(v);
+    if ((threadIdx.x & 63) == 0) scratch[threadIdx.x >> 6] = v;
+    __syncthreads();
+    double tot = 0.0;
+    for (int w = 0; w < (nthr + 63) >> 6; ++w) tot += scratch[w];
+    __syncthreads();
+    return tot / s.vol;
+}
+
 }  // namespace eddy

@@ -721,9 +721,10 @@ void launch_yfft_fwd(hipStream_t st, const Dims& d, const FftPlan& fp, const Tab
             if (in.mt.cart) go(k_yfft_fwd<T, YF_DIV_CART, false>);
             else go(k_yfft_fwd<T, YF_DIV_CYL, false>);
         }
-        const int nb = (int)(grid.x * grid.y);
-        launch_fold(st, rd.part, nb, rd.red + RED_VOLB, RED_OP_SUM, 0);
-        launch_fill(st, rd.red + RED_VOL, 1, in.mt.vol_total);
+        if (in.fold) {
+            launch_fold(st, rd.part, (int)(grid.x * grid.y), rd.red + RED_VOLB, RED_OP_SUM, 0);
+            launch_fill(st, rd.red + RED_VOL, 1, in.mt.vol_total);
+        }
     } else {
         if (dense) go(k_yfft_fwd<T, YF_RESIDUAL, true>);
         else go(k_yfft_fwd<T, YF_RESIDUAL, false>);

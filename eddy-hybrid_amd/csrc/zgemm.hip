@@ -20,6 +20,7 @@
 
 #include "kernels.h"
 #include "mma_device.h"
+#include "reduce_device.h"
 
 namespace eddy {
 
@@ -71,8 +72,8 @@ struct MmArgs {
     int R, Cn, P, nb;
     int ntr, ntc;     // tiles along r and along c
     int zb;           // batch of the zero y-mode (-1: not in this launch)
-    // forward: operand A of the zero mode minus shiftL * red[RED_VOLB] / red[RED_VOL]
-    const double* shift_red;
+    // forward: operand A of the zero mode minus shiftL times this mean
+    MeanShift shift;
     double shiftL;
     // inverse: operand dop (0 A, 1 B) of the zero mode plus delta where p == dnull, delta =
     // -sum_{m < dn} wsum[m] linesum[m] / (wsum[dnull] * dnorm)
@@ -186,7 +187,7 @@ __global__ void __launch_bounds__(256) k_mma(MmArgs<T> a) {
     constexpr int NR = BR / 32, NC = BC / 32;  // 16 x 16 tiles per wave along r and c
     extern __shared__ __align__(16) unsigned char mm_lds[];
     T* lds = reinterpret_cast<T*>(mm_lds);  // 2 x (OA::ELEMS + OB::ELEMS)
-    __shared__ double red4[4];
+    __shared__ double red4[16];
 
     const int tid = threadIdx.x;
     const int tile = xcd_tile(blockIdx.x, gridDim.x);
@@ -203,7 +204,7 @@ __global__ void __launch_bounds__(256) k_mma(MmArgs<T> a) {
     const bool zm = (b == a.zb);
     T shift = T(0), delta = T(0);
     if (zm) {
-        if (a.shift_red) shift = T(a.shiftL * a.shift_red[RED_VOLB] / a.shift_red[RED_VOL]);
+        shift = T(a.shiftL * mean_shift(a.shift, red4));
         if (a.linesum) {
             double s = 0.0;
             for (int m = tid; m < a.dn; m += 256) s += (double)a.wsum[m] * (double)a.linesum[m];
@@ -407,7 +408,7 @@ __global__ void __launch_bounds__(256) k_mma_dma(MmArgs<double> a) {
     const bool zm = (b == a.zb);
     double shift = 0.0, delta = 0.0;
     if (zm) {
-        if (a.shift_red) shift = a.shiftL * a.shift_red[RED_VOLB] / a.shift_red[RED_VOL];
+        shift = a.shiftL * mean_shift(a.shift, red4);
         if (a.linesum) {
             double s = 0.0;
             for (int m = tid; m < a.dn; m += 256) s += a.wsum[m] * a.linesum[m];
@@ -607,19 +608,19 @@ static rocblas_status gemm(rocblas_handle h, int M, int N, const float* A, const
 // for the MFMA kernel.
 template <typename T>
 int launch_zgemm_fwd(hipStream_t st, void* blas, const Dims& d, const Tables<T>& tb, T* S, T* S2,
-                     const double* shift_red, int j0, int nj) {
+                     const MeanShift& shift, int j0, int nj) {
     const size_t slab = (size_t)d.M * d.N;
     if (!blas) {
         MmArgs<T> a = mm_args<T>(S + slab * j0, d.M, (long)slab, tb.qf, d.N, 0, S2 + slab * j0, d.M, (long)slab, d.M,
                                  d.N, d.N, nj, j0);
-        a.shift_red = shift_red;
+        a.shift = shift;
         a.shiftL = (double)d.L;
         launch_mma<T>(st, false, a);
         return 0;
     }
-    if (shift_red && j0 == 0)
+    if (shift.red && j0 == 0)
         hipLaunchKernelGGL(k_zgemm_shift<T>, dim3((unsigned)((slab + 255) / 256)), dim3(256), 0, st, S, (long)slab,
-                           shift_red, (double)d.L);
+                           shift.red, (double)d.L);
     const rocblas_status r = gemm((rocblas_handle)blas, d.M, d.N, S + slab * j0, tb.qf, S2 + slab * j0, nj);
     return r == rocblas_status_success ? 0 : -1;
 }
@@ -654,19 +655,19 @@ int launch_zgemm_inv(hipStream_t st, void* blas, const Dims& d, const Tables<T>&
 // the x2 lines of each x1 mode are contiguous for the line solve; inverse: S_j = QI_j S2_j^T.
 template <typename T>
 int launch_xgemm_fwd(hipStream_t st, void* blas, const Dims& d, const Tables<T>& tz, T* S, T* S2,
-                     const double* shift_red, int j0, int nj) {
+                     const MeanShift& shift, int j0, int nj) {
     const size_t slab = (size_t)d.M * d.N, mm = (size_t)d.M * d.M;
     if (!blas) {
         MmArgs<T> a = mm_args<T>(S + slab * j0, d.M, (long)slab, tz.qf + mm * j0, d.M, (long)mm, S2 + slab * j0, d.N,
                                  (long)slab, d.N, d.M, d.M, nj, j0);
-        a.shift_red = shift_red;
+        a.shift = shift;
         a.shiftL = (double)d.L;
         launch_mma<T>(st, true, a);
         return 0;
     }
-    if (shift_red && j0 == 0)
+    if (shift.red && j0 == 0)
         hipLaunchKernelGGL(k_zgemm_shift<T>, dim3((unsigned)((slab + 255) / 256)), dim3(256), 0, st, S, (long)slab,
-                           shift_red, (double)d.L);
+                           shift.red, (double)d.L);
     const rocblas_status r = gemm((rocblas_handle)blas, true, false, d.N, d.M, d.M, S + slab * j0, d.M, (long)slab,
                                   tz.qf + mm * j0, d.M, (long)mm, S2 + slab * j0, d.N, (long)slab, nj);
     return r == rocblas_status_success ? 0 : -1;
@@ -719,17 +720,17 @@ void zgemm_destroy(void* blas) {
 }
 
 template int launch_zgemm_fwd<double>(hipStream_t, void*, const Dims&, const Tables<double>&, double*, double*,
-                                      const double*, int, int);
+                                      const MeanShift&, int, int);
 template int launch_zgemm_fwd<float>(hipStream_t, void*, const Dims&, const Tables<float>&, float*, float*,
-                                     const double*, int, int);
+                                     const MeanShift&, int, int);
 template int launch_zgemm_inv<double>(hipStream_t, void*, const Dims&, const Tables<double>&, double*, double*,
                                       const double*, int, int);
 template int launch_zgemm_inv<float>(hipStream_t, void*, const Dims&, const Tables<float>&, float*, float*,
                                      const float*, int, int);
 template int launch_xgemm_fwd<double>(hipStream_t, void*, const Dims&, const Tables<double>&, double*, double*,
-                                      const double*, int, int);
+                                      const MeanShift&, int, int);
 template int launch_xgemm_fwd<float>(hipStream_t, void*, const Dims&, const Tables<float>&, float*, float*,
-                                     const double*, int, int);
+                                     const MeanShift&, int, int);
 template int launch_xgemm_inv<double>(hipStream_t, void*, const Dims&, const Tables<double>&, double*, double*,
                                       const double*, int, int, int);
 template int launch_xgemm_inv<float>(hipStream_t, void*, const Dims&, const Tables<float>&, float*, float*,

@@ -16,6 +16,7 @@
 #include "batch_device.h"
 #include "fft_device.h"
 #include "kernels.h"
+#include "reduce_device.h"
 #include "stencil_device.h"
 
 namespace eddy {
@@ -24,7 +25,7 @@ template <typename T>
 struct ZArgs {
     T* S;
     const T* linesum;
-    const double* shift_red;  // forward: zero y-mode shift (L * VOLB/VOL) when non-null
+    MeanShift shift;  // forward: the zero y-mode loses L times this mean
     Dims d;
     FftPlan fp;  // complex FFT of length N/2 (DCT mode)
     Tables<T> tb;
@@ -52,6 +53,12 @@ __device__ T mean_delta(const ZArgs<T>& a) {
     for (int w = 0; w < (int)(blockDim.x + 63) / 64; ++w) tot += part[w];
     __syncthreads();
     return T(-tot / ((double)a.tb.wsum[a.d.null_m] * (double)a.d.M));
+}
+
+// The solvability shift of the zero y-mode's workgroups.
+__device__ __forceinline__ double zmean(const MeanShift& s) {
+    __shared__ double scratch[16];
+    return mean_shift(s, scratch);
 }
 
 // Copy the DCT tables into LDS (layout: twc H, twr H+1, dct N complex values, split re/im).
@@ -101,8 +108,7 @@ __device__ __forceinline__ void zdct_fwd_tile(const ZArgs<T>& a, int tile, int n
     T* base = a.S + (size_t)d.M * (size_t)N * (size_t)j;
     // Makhoul order: v[k/2] = x[k] (k even), v[N-1-(k-1)/2] = x[k] (k odd); z[q] = v[2q] + i v[2q+1]
     const int lti = a.lti;
-    const T zshift = (j == 0 && a.shift_red)
-                         ? T((double)d.L * a.shift_red[RED_VOLB] / a.shift_red[RED_VOL]) : T(0);
+    const T zshift = j == 0 ? T((double)d.L * zmean(a.shift)) : T(0);
     // The thread's x1 offset is fixed (blockDim is a multiple of TI). Every load of a batch is
     // issued before any value is used (arithmetic inside a load's own guard makes the compiler
     // wait for it before the next load); rows past N and lines past M read a clamped
@@ -295,8 +301,7 @@ __device__ __forceinline__ void zdense_tile(const ZArgs<T>& a, int tl, int ntx) 
     const T* A = (DIR == 0) ? a.tb.qf : a.tb.qiT;
     T delta = T(0);
     if (DIR == 1 && j == 0) delta = mean_delta(a);
-    const T zshift = (DIR == 0 && j == 0 && a.shift_red)
-                         ? T((double)d.L * a.shift_red[RED_VOLB] / a.shift_red[RED_VOL]) : T(0);
+    const T zshift = (DIR == 0 && j == 0) ? T((double)d.L * zmean(a.shift)) : T(0);
     const int lti = a.lti;
     for (int e0 = tid; e0 < TI * N; e0 += nthr * kZBatch) {
         T vv[kZBatch];
@@ -368,10 +373,10 @@ static inline size_t zlds_bytes(int TI, int ld, int N, size_t tsz) {
 
 template <typename T>
 void launch_ztrans_fwd(hipStream_t st, const Dims& d, const FftPlan& fpz, const Tables<T>& tb, T* S, int TI,
-                       int dense, const double* shift_red, int j0, int nj) {
+                       int dense, const MeanShift& shift, int j0, int nj) {
     ZArgs<T> a{};
     a.S = S;
-    a.shift_red = shift_red;
+    a.shift = shift;
     a.d = d;
     a.fp = fpz;
     a.tb = tb;
@@ -456,7 +461,8 @@ int prepare_ztrans(const std::vector<BatchProblem<T>>& pr, int dir, int shift, S
         ZArgs<T>& a = j.a;
         a.S = p.S;
         a.linesum = p.linesum;
-        a.shift_red = (dir == 0 && shift) ? p.red : nullptr;
+        // the partials of the forward y transform's tiles
+        if (dir == 0 && shift) a.shift = MeanShift{nullptr, p.part, ceil_div(p.d.M, p.tiy) * p.d.N, p.mt.vol_total};
         a.d = p.d;
         a.fp = p.fpz;
         a.tb = p.tb;
@@ -498,9 +504,9 @@ template void batch_ztrans<double>(hipStream_t, const StageLaunch&, int);
 template void batch_ztrans<float>(hipStream_t, const StageLaunch&, int);
 
 template void launch_ztrans_fwd<double>(hipStream_t, const Dims&, const FftPlan&, const Tables<double>&, double*,
-                                        int, int, const double*, int, int);
+                                        int, int, const MeanShift&, int, int);
 template void launch_ztrans_fwd<float>(hipStream_t, const Dims&, const FftPlan&, const Tables<float>&, float*,
-                                       int, int, const double*, int, int);
+                                       int, int, const MeanShift&, int, int);
 template void launch_ztrans_inv<double>(hipStream_t, const Dims&, const FftPlan&, const Tables<double>&, double*,
                                         const double*, int, int, int, int);
 template void launch_ztrans_inv<float>(hipStream_t, const Dims&, const FftPlan&, const Tables<float>&, float*,
