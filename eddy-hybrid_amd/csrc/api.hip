@@ -306,6 +306,13 @@ static int solve_core(eddy_plan_s* P, const FwdInput& in, int zshift) {
     // The x2 transform, x1 solve and inverse x2 transform of a y-mode touch only that mode's
     // slab of S; running the three over one chunk of modes at a time keeps the chunk's slabs
     // in the memory-side cache between the sweeps (tuning slab_chunks).
+    // Planes that fit one workgroup's LDS take the three in one kernel (not while kernel timing is
+    // on: each stage then has a time of its own).
+    if (!P->zgemm && !P->xgemm && !P->timing &&
+        zplane_fits(P->d, P->fpz, P->dense, P->tune.xsolve_chunk)) {
+        launch_zplane<T>(P->stream, P->d, P->fpz, tb, S, P->dense, P->tune.xsolve_chunk, shift, 0, P->d.L);
+        return check_launch("solve kernels");
+    }
     const int L = P->d.L;
     const int nch = std::max(1, std::min(P->tune.slab_chunks, L));
     for (int c = 0; c < nch; ++c) {

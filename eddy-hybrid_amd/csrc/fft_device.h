@@ -126,13 +126,28 @@ __device__ __forceinline__ int udiv_small(int x, int d, float rd, int& rem) {
     return q;
 }
 
+// What separates the passes of an in-place FFT: the workgroup's barrier, or, when one wave owns
+// all its rows (WAVE), only an order for the compiler to keep (a wave's LDS operations complete in
+// order).
+template <bool WAVE>
+__device__ __forceinline__ void fft_sync() {
+    if constexpr (WAVE) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    } else {
+        __syncthreads();
+    }
+}
+
 // In-place complex FFT of P sequences of length fp.n held in ONE buffer (split re/im, row
 // stride ld). Each radix pass: every thread loads at most one butterfly (up to 8 points, the
 // radix chosen at run time with predicated loads/stores so that all radices share the same
 // registers), the workgroup synchronises, then every thread stores. Needs
 // P * n / (smallest radix of the plan) <= nthr. The caller synchronises before (data
-// ready); the result is visible on return.
-template <typename T>
+// ready); the result is visible on return. WAVE: tid is the lane of the one wave that owns the P
+// sequences, nthr = 64.
+template <typename T, bool WAVE = false>
 __device__ void cfft_lds_ip(T* __restrict__ xr, T* __restrict__ xi, int ld, int P, const FftPlan& fp,
                             const T* twr, const T* twi, T dir, int tid, int nthr) {
     const int n = fp.n;
@@ -174,7 +189,7 @@ __device__ void cfft_lds_ip(T* __restrict__ xr, T* __restrict__ xi, int ld, int 
             orow = pen;
             obase = blk * Ns * R + k;
         }
-        __syncthreads();
+        fft_sync<WAVE>();
         if (active) {
             T* qr = xr + orow * ld;
             T* qi = xi + orow * ld;
@@ -186,7 +201,7 @@ __device__ void cfft_lds_ip(T* __restrict__ xr, T* __restrict__ xi, int ld, int 
                 }
             }
         }
-        __syncthreads();
+        fft_sync<WAVE>();
         Ns *= R;
     }
 }
@@ -201,7 +216,7 @@ __device__ void cfft_lds_ip(T* __restrict__ xr, T* __restrict__ xi, int ld, int 
 // stores: base = blk*Ns*R + k with k < Ns), so the offsets fold into the LDS instructions.
 __device__ __forceinline__ constexpr int poff(int x) { return x + (x >> 3); }
 
-template <typename T, int n, int R, int Ns>
+template <typename T, bool WAVE, int n, int R, int Ns>
 __device__ __forceinline__ void cfft_pass_static(T* __restrict__ xr, T* __restrict__ xi, int ld, int P,
                                                  const T* twr, const T* twi, T dir, int tid) {
     constexpr int nb = n / R;
@@ -231,7 +246,7 @@ __device__ __forceinline__ void cfft_pass_static(T* __restrict__ xr, T* __restri
         else dft8(v, dir);
         oaddr = pen * ld + pidx(blk * Ns * R + k);
     }
-    __syncthreads();
+    fft_sync<WAVE>();
     if (active) {
 #pragma unroll
         for (int r = 0; r < R; ++r) {
@@ -239,14 +254,14 @@ __device__ __forceinline__ void cfft_pass_static(T* __restrict__ xr, T* __restri
             xi[oaddr + poff(r * Ns)] = v[r].im;
         }
     }
-    __syncthreads();
+    fft_sync<WAVE>();
 }
 
-template <typename T, int n, int Ns, int R, int... Rest>
+template <typename T, bool WAVE, int n, int Ns, int R, int... Rest>
 __device__ __forceinline__ void cfft_passes_static(T* xr, T* xi, int ld, int P, const T* twr, const T* twi, T dir,
                                                    int tid) {
-    cfft_pass_static<T, n, R, Ns>(xr, xi, ld, P, twr, twi, dir, tid);
-    if constexpr (sizeof...(Rest) > 0) cfft_passes_static<T, n, Ns * R, Rest...>(xr, xi, ld, P, twr, twi, dir, tid);
+    cfft_pass_static<T, WAVE, n, R, Ns>(xr, xi, ld, P, twr, twi, dir, tid);
+    if constexpr (sizeof...(Rest) > 0) cfft_passes_static<T, WAVE, n, Ns * R, Rest...>(xr, xi, ld, P, twr, twi, dir, tid);
 }
 
 template <int... Rs>
@@ -261,18 +276,18 @@ __device__ __forceinline__ bool plan_is(const FftPlan& fp) {
 
 // cfft_lds_ip with the power-of-two plans of radix_plan (largest radix 8) taken by the
 // compile-time passes; every other plan by the run-time passes. Same contract.
-template <typename T>
+template <typename T, bool WAVE = false>
 __device__ __forceinline__ void cfft_lds(T* __restrict__ xr, T* __restrict__ xi, int ld, int P, const FftPlan& fp,
                                          const T* twr, const T* twi, T dir, int tid, int nthr) {
-    if (fp.n == 128 && plan_is<8, 4, 4>(fp)) cfft_passes_static<T, 128, 1, 8, 4, 4>(xr, xi, ld, P, twr, twi, dir, tid);
-    else if (fp.n == 64 && plan_is<8, 8>(fp)) cfft_passes_static<T, 64, 1, 8, 8>(xr, xi, ld, P, twr, twi, dir, tid);
+    if (fp.n == 128 && plan_is<8, 4, 4>(fp)) cfft_passes_static<T, WAVE, 128, 1, 8, 4, 4>(xr, xi, ld, P, twr, twi, dir, tid);
+    else if (fp.n == 64 && plan_is<8, 8>(fp)) cfft_passes_static<T, WAVE, 64, 1, 8, 8>(xr, xi, ld, P, twr, twi, dir, tid);
     else if (fp.n == 256 && plan_is<8, 8, 4>(fp))
-        cfft_passes_static<T, 256, 1, 8, 8, 4>(xr, xi, ld, P, twr, twi, dir, tid);
+        cfft_passes_static<T, WAVE, 256, 1, 8, 8, 4>(xr, xi, ld, P, twr, twi, dir, tid);
     else if (fp.n == 512 && plan_is<8, 8, 8>(fp))
-        cfft_passes_static<T, 512, 1, 8, 8, 8>(xr, xi, ld, P, twr, twi, dir, tid);
-    else if (fp.n == 32 && plan_is<8, 4>(fp)) cfft_passes_static<T, 32, 1, 8, 4>(xr, xi, ld, P, twr, twi, dir, tid);
-    else if (fp.n == 16 && plan_is<4, 4>(fp)) cfft_passes_static<T, 16, 1, 4, 4>(xr, xi, ld, P, twr, twi, dir, tid);
-    else cfft_lds_ip<T>(xr, xi, ld, P, fp, twr, twi, dir, tid, nthr);
+        cfft_passes_static<T, WAVE, 512, 1, 8, 8, 8>(xr, xi, ld, P, twr, twi, dir, tid);
+    else if (fp.n == 32 && plan_is<8, 4>(fp)) cfft_passes_static<T, WAVE, 32, 1, 8, 4>(xr, xi, ld, P, twr, twi, dir, tid);
+    else if (fp.n == 16 && plan_is<4, 4>(fp)) cfft_passes_static<T, WAVE, 16, 1, 4, 4>(xr, xi, ld, P, twr, twi, dir, tid);
+    else cfft_lds_ip<T, WAVE>(xr, xi, ld, P, fp, twr, twi, dir, tid, nthr);
 }
 
 // Smallest radix of a plan (bounds the butterflies per pass of cfft_lds_ip).

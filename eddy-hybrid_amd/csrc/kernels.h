@@ -134,6 +134,13 @@ template <typename T>
 int launch_xsolve(hipStream_t st, const Dims& d, const Tables<T>& tb, T* S, T* linesum, int chunk, int j0, int nj,
                   int cyc = 0, double alpha = 0.0, double beta = 0.0);
 
+// The x2 transform, the line solves and the inverse x2 transform of modes [j0, j0 + nj) with each
+// plane in one workgroup's LDS (zplane.hip): whether a plan's planes take it, and the launch.
+bool zplane_fits(const Dims& d, const FftPlan& fpz, int dense, int chunk);
+template <typename T>
+void launch_zplane(hipStream_t st, const Dims& d, const FftPlan& fpz, const Tables<T>& tb, T* S, int dense, int chunk,
+                   const MeanShift& shift, int j0, int nj);
+
 // ------------------------------------------------------------------ batched launches
 // One problem of a batch, with everything its stages read and write (device pointers).
 template <typename T>
