@@ -1509,8 +1509,7 @@ int eddy_resident_create(eddy_resident_t* res, eddy_plan_t plan, double* u, doub
     launch_perturb(plan->stream, plan->d, u, v, w, us, vs, ws, sigma, (uint32_t)seed, R->step);
     rc = eddy_project_dev(plan, us, vs, ws, u, v, w, dp, alfxdt, 1, precision, sweeps);
     if (!rc) {
-        launch_div_minmax(plan->stream, plan->d, plan->mt, u, v, w, rd(plan));
-        launch_log_step(plan->stream, plan->red, R->log, R->step, R->cap);
+        launch_div_minmax(plan->stream, plan->d, plan->mt, u, v, w, rd(plan), R->log, R->step, R->cap);
     }
     hipGraph_t g = nullptr;
     hipError_t e = hipStreamEndCapture(plan->stream, &g);

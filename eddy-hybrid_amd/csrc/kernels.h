@@ -179,7 +179,7 @@ struct StageLaunch {
     int cls_total[kMaxClasses] = {};
     size_t cls_lds[kMaxClasses] = {};
     // the forward y transform with the divergence: 1 every problem Cartesian, 2 every one
-    // cylindrical (a kernel with only that metric's registers), 0 mixed; CORRECT: 1 the span kernel
+    // cylindrical (a kernel with only that metric's registers), 0 mixed
     int kind = 0;
     const double* alf = nullptr;  // CORRECT: device {ALFXDT, 1/ALFXDT}
 };
@@ -264,7 +264,7 @@ void batch_fold(hipStream_t st, const FoldJob* jobs, int njobs);
 
 // Stencils (FP64).
 int reduce_blocks(const Dims& d);
-void launch_fold(hipStream_t st, const double* part, int n, double* out, int op, int add);
+void launch_fold(hipStream_t st, const double* part, int n, double* out);
 // red[RED_CHK_VB] = sum vol*b, red[RED_CHK_VABS] = sum vol*|b| over the finite interior values
 // of b, red[RED_CHK_NF] = the count of non-finite ones.
 void launch_rhs_check(hipStream_t st, const Dims& d, const Metrics& mt, const double* b, const Reduce& rd);
@@ -287,8 +287,11 @@ void launch_fill(hipStream_t st, double* p, size_t n, double v);
 // ghost planes take the periodic images DP(:,:,1) = DP(:,:,NZ-1), DP(:,:,NZ) = DP(:,:,2).
 void launch_refresh_z(hipStream_t st, const Dims& d, double* dp);
 void launch_copy_shift(hipStream_t st, const Dims& d, const double* src, double* dst, const double* red);
+// SCRINFO's divergence range into red[RED_DMIN], red[RED_DMAX]; with a log the resident step's
+// epilogue too (the pair at log[2 s] for s = *step < cap, *step + 1).
 void launch_div_minmax(hipStream_t st, const Dims& d, const Metrics& mt, const double* us,
-                       const double* vs, const double* ws, const Reduce& rd);
+                       const double* vs, const double* ws, const Reduce& rd, double* log = nullptr,
+                       int* step = nullptr, int cap = 0);
 
 // Pressure update after CORRECT (Eddy6.f:2772-2846): P += DP minus the implicit corrections,
 // PREF subtracted (red[RED_PREF]), ghost values from the boundary copies.
@@ -306,10 +309,8 @@ struct PressArgs {
 void launch_pressure_update(hipStream_t st, const PressArgs& a);
 
 // Resident time loop: us = u + sigma * N(0,1) on the faces CORRECT updates (Philox4x32-10,
-// counter {cell, step}, key {seed, 0}; step read from device memory); the log epilogue
-// stores red[RED_DMIN], red[RED_DMAX] at log[2 step] and increments *step.
+// counter {cell, step}, key {seed, 0}; step read from device memory).
 void launch_perturb(hipStream_t st, const Dims& d, const double* u, const double* v, const double* w, double* us,
                     double* vs, double* ws, double sigma, uint32_t seed, const int* step);
-void launch_log_step(hipStream_t st, const double* red, double* log, int* step, int cap);
 
 }  // namespace eddy

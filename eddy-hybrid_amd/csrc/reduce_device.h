@@ -73,6 +73,7 @@ __device__ __forceinline__ double mean_shift(const MeanShift& s, double* scratch
     if (!s.part) return 0.0;
     const int nthr = blockDim.x;
     double v = 0.0;
+#pragma unroll 8
     for (int t = threadIdx.x; t < s.n; t += nthr) v += s.part[t];
     v = wave_sum(v);
     if ((threadIdx.x & 63) == 0) scratch[threadIdx.x >> 6] = v;

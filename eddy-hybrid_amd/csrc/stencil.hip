@@ -33,22 +33,6 @@ __device__ __forceinline__ Blk xcd_block() {
     return Blk{t % gx, (t / gx) % gy, t / (gx * gy)};
 }
 
-// The same blocks with the x2 planes taken in chunks of KC: x fastest, then the plane within
-// the chunk, then y, then the chunk. A block's x2 neighbour plane is then read by a block
-// dispatched gx blocks later on the same XCD, while it is still in that XCD's L2.
-template <int KC>
-__device__ __forceinline__ Blk xcd_block_kc() {
-    const int gx = gridDim.x, gy = gridDim.y, gz = gridDim.z;
-    const int t = xcd_tile(blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z), gx * gy * gz);
-    const int cb = gx * gy * KC;
-    const int c = t / cb;
-    int r = t - c * cb;
-    const int kc = min(KC, gz - c * KC);  // the last chunk may hold fewer planes
-    const int x = r % gx;
-    r /= gx;
-    return Blk{x, r / kc, c * KC + r % kc};
-}
-
 __global__ void __launch_bounds__(256) k_divergence(Dims d, Metrics mt, const double* __restrict__ us,
                                                     const double* __restrict__ vs, const double* __restrict__ ws,
                                                     double* __restrict__ div, double scale, double* part,
@@ -69,113 +53,22 @@ __global__ void __launch_bounds__(256) k_divergence(Dims d, Metrics mt, const do
     if (accumulate) block_partial<RED_OP_SUM>(vb, part, linear_bid());
 }
 
-__global__ void __launch_bounds__(256) k_div_minmax(Dims d, Metrics mt, const double* __restrict__ us,
-                                                    const double* __restrict__ vs, const double* __restrict__ ws,
-                                                    double* part) {
-    const Blk bk = xcd_block();
-    const int i = bk.x * 64 + threadIdx.x;
-    const int k = bk.z;
-    double mn = 1e300, mx = -1e300;
-    if (i < d.M) {
-        for (int j = threadIdx.y; j < d.L; j += 4) {
-            const double v = div_at(d, mt, us, vs, ws, i, j, k);
-            mn = fmin(mn, v);
-            mx = fmax(mx, v);
-        }
-    }
-    const int nb = gridDim.x * gridDim.y * gridDim.z;
-    block_partial<RED_OP_MIN>(mn, part, linear_bid());
-    block_partial<RED_OP_MAX>(mx, part + nb, linear_bid());
-}
-
-// CORRECT of fields that are not all 16-byte aligned (k_correct_span takes the others).
-// Rows per thread: rows j0, j0 + 4, ... of a block of 64 x1 cells by 4 * kCorrectRows
-// y rows; every load of a thread is issued before its first store (rows past L load a clamped
-// in-range row and store nothing). Addresses are 32-bit byte offsets (fields below 4 GiB).
-constexpr int kCorrectRows = 2;
-
-template <int R>
-__global__ void __launch_bounds__(256) k_correct(Dims d, Metrics mt, const double* __restrict__ us,
-                                                 const double* __restrict__ vs, const double* __restrict__ ws,
-                                                 double* __restrict__ uo, double* __restrict__ vo,
-                                                 double* __restrict__ wo, const double* __restrict__ dp,
-                                                 double alfxdt, int refresh, const double* __restrict__ dscale) {
-    // dp(k+1) is this block's neighbour plane; plane chunks of 2 (chunks of 1, 4 and 8 measured
-    // 2.6 %, 0.8 % and 1.4 % slower with two rows per thread)
-    const Blk bk = xcd_block_kc<2>();
-    if (dscale) alfxdt = dscale[0];
-    const int i = bk.x * 64 + threadIdx.x;
-    const int j0 = bk.y * (4 * R) + threadIdx.y;
-    const int k = bk.z;
-    if (i >= d.M || j0 >= d.L) return;
-    const int I = i + 1, K = k + 1;
-    const unsigned nx8 = 8u * (unsigned)d.nx, pl8 = nx8 * (unsigned)d.ny;
-    const unsigned oik = 8u * (unsigned)I + pl8 * (unsigned)K;
-    // U faces I = IBU..IEU: 2..NX-2 with x1 walls (MP=1), 2..NX-1 when x1 is periodic
-    // (ITYPE(2)=500, setup.f:34-35; DP(NX) is then DIRECT's periodic ghost); W faces K =
-    // KBW..KEW: 2..NZ-2 with x2 walls (NP=1), 2..NZ-1 when x2 is periodic (ITYPE(6)=500,
-    // setup.f:70; DP(NZ) then holds REFRESHBC's periodic image)
-    const bool uface = I <= d.nx - 3 + d.cyc_x, wface = K <= d.nz - 3 + d.cyc_z;
-    const double auI = mt.au[I], cwK = mt.cw[K], rpI = mt.cart ? 1.0 : mt.rp[I];
-    unsigned o[R];
-    double p0[R], pe[R], pn[R], pt[R], u[R], v[R], w[R], bvJ[R];
-#pragma unroll
-    for (int q = 0; q < R; ++q) {
-        const int J = min(j0 + 4 * q, d.L - 1) + 1;
-        o[q] = oik + nx8 * (unsigned)J;
-        p0[q] = ld_off(dp, o[q]);
-        pe[q] = ld_off(dp, o[q] + 8u);
-        pn[q] = ld_off(dp, o[q] + nx8);
-        pt[q] = ld_off(dp, o[q] + pl8);
-        u[q] = ld_off(us, o[q]);
-        v[q] = ld_off(vs, o[q]);
-        w[q] = ld_off(ws, o[q]);
-        bvJ[q] = mt.bv[J];
-    }
-#pragma unroll
-    for (int q = 0; q < R; ++q) {
-        const int j = j0 + 4 * q;
-        if (j >= d.L) continue;
-        const int J = j + 1;
-        // periodic y ghost rows of the corrected faces (the velocity BC step after CORRECT,
-        // Eddy6.f:2746-2761): row J=1 mirrors J=NY-1, row J=NY mirrors J=2
-        const int gofs = (j == d.L - 1) ? -(int)(nx8 * (unsigned)(d.ny - 2))
-                                        : ((j == 0) ? (int)(nx8 * (unsigned)(d.ny - 2)) : 0);
-        const bool ghost = refresh && gofs != 0 && !d.ycopy;
-        if (uface) {
-            const double un = u[q] - auI * (pe[q] - p0[q]) * alfxdt;
-            st_off(uo, o[q], un);
-            if (ghost) st_off(uo, o[q] + (unsigned)gofs, un);
-        }
-        // V faces J = JBV..JEV: 2..NY-1 for the periodic y (ITYPE(4)=500, LP=0), 2..NY-2 for LP=1
-        if (J <= d.ny - 2 - d.ycopy) {
-            const double gv = bvJ[q] * (pn[q] - p0[q]) * alfxdt;
-            const double vn = v[q] - (mt.cart ? gv : gv / rpI);
-            st_off(vo, o[q], vn);
-            if (ghost) st_off(vo, o[q] + (unsigned)gofs, vn);
-        }
-        if (wface) {
-            const double wn = w[q] - cwK * (pt[q] - p0[q]) * alfxdt;
-            st_off(wo, o[q], wn);
-            if (ghost) st_off(wo, o[q] + (unsigned)gofs, wn);
-        }
-    }
-}
-
 // CORRECT along memory instead of along rows: the interior rows J = 1..L of a plane are one span
 // of L*nx consecutive elements, cut into blocks of 512 * kSpanParts elements that start on a
 // 128-byte line (when the bases do), two neighbouring elements per lane and part. Every access of
 // the six velocity fields and of dp is then a whole aligned 1 KiB per wave, where a 64-cell block of
 // a row (nx = M + 2 elements, starting one past a ghost) straddles five lines with partial lines at
 // both ends, read and written by two blocks. The ghosts inside the span (4 of nx) are loaded and
-// not stored. Needs 16-byte aligned fields (the row kernel above takes the others). HBM bound;
+// not stored. Fields and rows of any alignment take the same 16-byte accesses (d2u). HBM bound;
 // with the streamed velocities and the block order below 0.398 -> 0.343 ms at 512 x 256 x 256,
 // 0.493 -> 0.407 ms at 302 x 130 x 1026, 0.058 -> 0.044 ms at 300 x 128 x 128.
 constexpr int kSpanParts = 2;
 constexpr int kSpan = 512 * kSpanParts;  // elements per block
 
 typedef double d2 __attribute__((ext_vector_type(2)));
-typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));  // rows of odd nx
+// a pair at any element: rows of odd nx and fields that start between two 16-byte boundaries are
+// read and written with the same 16-byte instructions, which need dword alignment only
+typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));
 
 struct CorrArgs {
     Dims d;
@@ -186,18 +79,39 @@ struct CorrArgs {
     unsigned rnx;  // ceil(2^32 / nx)
 };
 
+// ceil(2^32 / nx): the quotient of an element number by nx as a high product (span_pair)
+static inline unsigned row_magic(const Dims& d) { return (unsigned)(((1ull << 32) + d.nx - 1) / d.nx); }
+
 // Blocks of a plane's span (its start rounded down to 16 elements).
 __host__ __device__ inline int span_blocks(const Dims& d) { return ceil_div(d.L * d.nx + 15, kSpan); }
 
+__device__ __forceinline__ d2 ld_pair(const double* b, unsigned off) {
+    return *reinterpret_cast<const d2u*>(reinterpret_cast<const char*>(b) + off);
+}
 // The velocities are streamed (read once, written once): non-temporal, so that they do not push
 // dp's planes out of L2 nor the solve's arrays out of the memory-side cache.
-template <typename V>
-__device__ __forceinline__ V ld_stream(const double* b, unsigned off) {
-    return __builtin_nontemporal_load(reinterpret_cast<const V*>(reinterpret_cast<const char*>(b) + off));
+__device__ __forceinline__ d2 ld_stream(const double* b, unsigned off) {
+    return __builtin_nontemporal_load(reinterpret_cast<const d2u*>(reinterpret_cast<const char*>(b) + off));
 }
-template <typename V>
-__device__ __forceinline__ void st_stream(double* b, unsigned off, V v) {
-    __builtin_nontemporal_store(v, reinterpret_cast<V*>(reinterpret_cast<char*>(b) + off));
+__device__ __forceinline__ void st_stream(double* b, unsigned off, d2 v) {
+    __builtin_nontemporal_store(v, reinterpret_cast<d2u*>(reinterpret_cast<char*>(b) + off));
+}
+
+// The pair of elements e, e + 1 of a field's plane (first element of the plane at `plane`): whether
+// it holds an interior cell of rows 1..L, and the x1 and y index of its first element.
+struct Pair {
+    int i, j;
+    bool on;
+};
+__device__ __forceinline__ Pair span_pair(const Dims& d, unsigned r, unsigned rnx) {
+    int j = (int)__umulhi(r, rnx);  // exact or one too large
+    int i = (int)r - j * d.nx;
+    if (i < 0) {
+        --j;
+        i += d.nx;
+    }
+    // (i, j), (i + 1, j), or (0, j + 1) past a row's end, which holds no interior cell
+    return Pair{i, j, j >= 1 && j <= d.L && i <= d.M};
 }
 
 // Block `b` of plane k's span (k 0-based interior).
@@ -210,38 +124,25 @@ __device__ __forceinline__ void correct_span(const CorrArgs& c, double alfxdt, i
     const bool wface = k + 1 <= d.nz - 3 + d.cyc_z;
     const int ulast = d.nx - 3 + d.cyc_x, vlast = d.ny - 2 - d.ycopy;
     unsigned o[kSpanParts];
-    int I[kSpanParts], J[kSpanParts];
-    bool on[kSpanParts];
-    d2 p0[kSpanParts], u[kSpanParts], v[kSpanParts], w[kSpanParts];
-    d2u pn[kSpanParts], pt[kSpanParts];
+    Pair pr[kSpanParts];
+    d2 p0[kSpanParts], u[kSpanParts], v[kSpanParts], w[kSpanParts], pn[kSpanParts], pt[kSpanParts];
     double pe[kSpanParts];
 #pragma unroll
     for (int q = 0; q < kSpanParts; ++q) {
-        const unsigned r = e0 + 512u * q - plane;  // element of the plane (>= nx - 15)
-        int j = (int)__umulhi(r, c.rnx);           // exact or one too large
-        int i = (int)(r - (unsigned)j * nx);
-        if (i < 0) {
-            --j;
-            i += d.nx;
-        }
-        // pairs that hold an interior cell: elements (i, j), (i + 1, j), or (0, j + 1) past a row's end
-        on[q] = j >= 1 && j <= d.L && i <= d.M;
-        I[q] = i;
-        J[q] = j;
-        o[q] = 8u * (e0 + 512u * q);
-        if (!on[q]) o[q] = 8u * (plane + nx);
-        p0[q] = ld_off(reinterpret_cast<const d2*>(c.dp), o[q] & ~15u);
-        pe[q] = ld_off(c.dp, (o[q] & ~15u) + 16u);
-        pn[q] = ld_off(reinterpret_cast<const d2u*>(c.dp), (o[q] & ~15u) + 8u * nx);
-        pt[q] = ld_off(reinterpret_cast<const d2u*>(c.dp), (o[q] & ~15u) + 8u * pl);
-        u[q] = ld_stream<d2>(c.us, o[q] & ~15u);
-        v[q] = ld_stream<d2>(c.vs, o[q] & ~15u);
-        w[q] = ld_stream<d2>(c.ws, o[q] & ~15u);
+        pr[q] = span_pair(d, e0 + 512u * q - plane, c.rnx);
+        o[q] = 8u * (pr[q].on ? e0 + 512u * q : plane + nx);
+        p0[q] = ld_pair(c.dp, o[q]);
+        pe[q] = ld_off(c.dp, o[q] + 16u);
+        pn[q] = ld_pair(c.dp, o[q] + 8u * nx);
+        pt[q] = ld_pair(c.dp, o[q] + 8u * pl);
+        u[q] = ld_stream(c.us, o[q]);
+        v[q] = ld_stream(c.vs, o[q]);
+        w[q] = ld_stream(c.ws, o[q]);
     }
 #pragma unroll
     for (int q = 0; q < kSpanParts; ++q) {
-        if (!on[q]) continue;
-        const int i = I[q], j = J[q];
+        if (!pr[q].on) continue;
+        const int i = pr[q].i, j = pr[q].j;
         const int i1 = min(i + 1, d.nx - 1);
         const double bvJ = c.mt.bv[j];
         d2 un, vn, wn;
@@ -256,14 +157,14 @@ __device__ __forceinline__ void correct_span(const CorrArgs& c, double alfxdt, i
         const bool u0 = a0 && i <= ulast, u1 = a1 && i + 1 <= ulast;
         const bool vf = j <= vlast;
         auto put = [&](double* f, unsigned at, d2 x, bool s0, bool s1) {
-            if (s0 && s1) st_stream<d2u>(f, at, x);
+            if (s0 && s1) st_stream(f, at, x);
             else if (s0) st_off(f, at, x.x);
             else if (s1) st_off(f, at + 8u, x.y);
         };
         if (a0 && a1 && u0 && u1) {
-            st_stream<d2>(c.uo, o[q], un);
-            if (vf) st_stream<d2>(c.vo, o[q], vn);
-            if (wface) st_stream<d2>(c.wo, o[q], wn);
+            st_stream(c.uo, o[q], un);
+            if (vf) st_stream(c.vo, o[q], vn);
+            if (wface) st_stream(c.wo, o[q], wn);
         } else {
             put(c.uo, o[q], un, u0, u1);
             if (vf) put(c.vo, o[q], vn, a0, a1);
@@ -302,16 +203,112 @@ __global__ void __launch_bounds__(256) k_correct_span(CorrArgs c, double alfxdt,
     correct_item(c, alfxdt, refresh, runs ? xcd_run(b, n, kCorrectRun) : xcd_tile(b, n), n / c.d.N);
 }
 
-// The bases of every field at 16 bytes, as correct_span's pairs need them.
-static bool pairs_aligned(const double* us, const double* vs, const double* ws, const double* uo, const double* vo,
-                          const double* wo, const double* dp) {
-    return (((uintptr_t)us | (uintptr_t)vs | (uintptr_t)ws | (uintptr_t)uo | (uintptr_t)vo | (uintptr_t)wo |
-             (uintptr_t)dp) & 15) == 0;
-}
-
 static CorrArgs corr_args(const Dims& d, const Metrics& mt, const double* us, const double* vs, const double* ws,
                           double* uo, double* vo, double* wo, const double* dp) {
-    return CorrArgs{d, mt, us, vs, ws, uo, vo, wo, dp, (unsigned)(((1ull << 32) + d.nx - 1) / d.nx)};
+    return CorrArgs{d, mt, us, vs, ws, uo, vo, wo, dp, row_magic(d)};
+}
+
+// SCRINFO's divergence range over the same spans (fmin / fmax as the reference's MIN / MAX). A block
+// takes the spans b, b + nbx, ... of `planes` consecutive planes and keeps w of the plane below
+// in registers on its way up, so that w is read once but for the lowest plane's neighbour. It leaves its
+// minimum at part[slot], its maximum at part[nb + slot]. 24 B/cell, HBM bound: 0.430 -> 0.360 ms at
+// 768 x 384 x 256 over a kernel of row blocks, and one fold instead of two and a log kernel after it.
+__global__ void __launch_bounds__(256) k_div_minmax(Dims d, Metrics mt, const double* __restrict__ us,
+                                                    const double* __restrict__ vs, const double* __restrict__ ws,
+                                                    double* part, unsigned rnx, int nbx, int planes, int runs) {
+    const int nb = gridDim.x;
+    const int t = runs ? xcd_run(blockIdx.x, nb, kCorrectRun) : xcd_tile(blockIdx.x, nb);
+    const int kg = t / nbx, k0 = kg * planes, k1 = min(k0 + planes, d.N);
+    const unsigned nx = (unsigned)d.nx, pl = nx * (unsigned)d.ny, nspan = (unsigned)span_blocks(d);
+    double mn = 1e300, mx = -1e300;
+    for (unsigned b = (unsigned)(t - kg * nbx); b < nspan; b += (unsigned)nbx) {
+        // the span's elements of the group's first plane; the others' are whole planes above
+        Pair pr[kSpanParts];
+        unsigned o[kSpanParts];
+        d2 wm[kSpanParts];
+        double bpj[kSpanParts];
+#pragma unroll
+        for (int q = 0; q < kSpanParts; ++q) {
+            const unsigned r = (nx & ~15u) + b * kSpan + 512u * q + 2u * threadIdx.x;
+            pr[q] = span_pair(d, r, rnx);
+            o[q] = 8u * ((pr[q].on ? r : nx) + pl * (unsigned)(k0 + 1));
+            bpj[q] = mt.bp[pr[q].on ? pr[q].j : 1];
+            wm[q] = ld_pair(ws, o[q] - 8u * pl);
+        }
+        for (int k = k0; k < k1; ++k) {
+            const double cpk = mt.cp[k + 1];
+            d2 u[kSpanParts], v[kSpanParts], vm[kSpanParts], w[kSpanParts];
+            double um[kSpanParts];
+#pragma unroll
+            for (int q = 0; q < kSpanParts; ++q) {
+                u[q] = ld_pair(us, o[q]);
+                um[q] = ld_off(us, o[q] - 8u);
+                v[q] = ld_pair(vs, o[q]);
+                vm[q] = ld_pair(vs, o[q] - 8u * nx);
+                w[q] = ld_pair(ws, o[q]);
+            }
+#pragma unroll
+            for (int q = 0; q < kSpanParts; ++q) {
+                // div_at's arithmetic
+                auto one = [&](int I, double um1, double u1, double vm1, double v1, double wm1, double w1) {
+                    if (!pr[q].on || I < 1 || I > d.M) return;
+                    const double c = cpk * (w1 - wm1);
+                    double x;
+                    if (mt.cart) {
+                        x = mt.ap[I] * (u1 - um1) + bpj[q] * (v1 - vm1) + c;
+                    } else {
+                        const double rpi = mt.rp[I];
+                        x = mt.ap[I] * (mt.ru[I] * u1 - mt.ru[I - 1] * um1) / rpi + bpj[q] * (v1 - vm1) / rpi + c;
+                    }
+                    mn = fmin(mn, x);
+                    mx = fmax(mx, x);
+                };
+                one(pr[q].i, um[q], u[q].x, vm[q].x, v[q].x, wm[q].x, w[q].x);
+                one(pr[q].i + 1, u[q].x, u[q].y, vm[q].y, v[q].y, wm[q].y, w[q].y);
+                wm[q] = w[q];
+                o[q] += 8u * pl;
+            }
+        }
+    }
+    block_partial<RED_OP_MIN>(mn, part, (int)blockIdx.x);
+    block_partial<RED_OP_MAX>(mx, part + nb, (int)blockIdx.x);
+}
+
+// red[RED_DMIN], red[RED_DMAX] from the n block minima and maxima of k_div_minmax, one workgroup of
+// 1024 threads; with a log, the step's epilogue too: log[2 s], log[2 s + 1] for s = *step < cap, then
+// *step = s + 1.
+__global__ void __launch_bounds__(1024) k_fold_minmax(const double* __restrict__ part, int n, double* red, double* log,
+                                                      int* step, int cap) {
+    double mn = 1e300, mx = -1e300;
+#pragma unroll 8
+    for (int t = threadIdx.x; t < n; t += 1024) {
+        mn = fmin(mn, part[t]);
+        mx = fmax(mx, part[n + t]);
+    }
+    __shared__ double w[2][16];
+    mn = wave_min(mn);
+    mx = wave_max(mx);
+    if ((threadIdx.x & 63) == 0) {
+        w[0][threadIdx.x >> 6] = mn;
+        w[1][threadIdx.x >> 6] = mx;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int q = 1; q < 16; ++q) {
+            mn = fmin(mn, w[0][q]);
+            mx = fmax(mx, w[1][q]);
+        }
+        red[RED_DMIN] = mn;
+        red[RED_DMAX] = mx;
+        if (log) {
+            const int s = step[0];
+            if (s >= 0 && s < cap) {
+                log[2 * s] = mn;
+                log[2 * s + 1] = mx;
+            }
+            step[0] = s + 1;
+        }
+    }
 }
 
 __global__ void __launch_bounds__(256) k_laplacian(Dims d, Op64 op, const double* __restrict__ phi,
@@ -439,33 +436,28 @@ __global__ void k_fill(double* p, size_t n, double v) {
     if (t < n) p[t] = v;
 }
 
-// out[0] (= or combined with) the reduction of part[0..n), one workgroup of 1024 threads.
-template <int OP>
-__global__ void __launch_bounds__(1024) k_fold(const double* __restrict__ part, int n, double* out, int add) {
-    const double init = (OP == RED_OP_SUM) ? 0.0 : ((OP == RED_OP_MIN) ? 1e300 : -1e300);
-    double v = init;
-    for (int t = threadIdx.x; t < n; t += blockDim.x) v = combine<OP>(v, part[t]);
+// out[0] = the sum of part[0..n), one workgroup of 1024 threads.
+__global__ void __launch_bounds__(1024) k_fold(const double* __restrict__ part, int n, double* out) {
+    double v = 0.0;
+#pragma unroll 8
+    for (int t = threadIdx.x; t < n; t += 1024) v += part[t];
     __shared__ double w[16];
-    v = wave_reduce<OP>(v);
+    v = wave_sum(v);
     if ((threadIdx.x & 63) == 0) w[threadIdx.x >> 6] = v;
     __syncthreads();
     if (threadIdx.x == 0) {
         double s = w[0];
-        for (int q = 1; q < (int)(blockDim.x >> 6); ++q) s = combine<OP>(s, w[q]);
-        *out = add ? combine<OP>(*out, s) : s;
+        for (int q = 1; q < 16; ++q) s += w[q];
+        *out = s;
     }
 }
 
 // ------------------------------------------------------------------ batched (one item per workgroup)
 struct CellArgs {
     Dims d;
-    Metrics mt;
-    const double *us, *vs, *ws;
-    double *uo, *vo, *wo;
     double* dp;
     double* rhs;
     const double* red;
-    const double* dscale;  // device {ALFXDT, 1/ALFXDT} of the projection
 };
 
 constexpr int kCellRows = 4;  // y rows per thread of a batch cell item
@@ -475,8 +467,7 @@ constexpr int kCellRows = 4;  // y rows per thread of a batch cell item
 // blocks, nty y blocks per plane). Every load of a thread is issued before its first store:
 // rows past L load a clamped in-range row and store nothing. (One row per thread left the
 // per-item set-up, the job search and argument loads, on every 256 cells: the copy stages
-// ran 1.3-1.9x slower; a loop over all of a plane's rows waited on each row's loads in turn:
-// CORRECT 1.26x slower.)
+// ran 1.3-1.9x slower.)
 template <int OP>
 __device__ __forceinline__ void cell_tile(const CellArgs& c, int t, int ntx, int nty) {
     constexpr int R = kCellRows;
@@ -491,43 +482,7 @@ __device__ __forceinline__ void cell_tile(const CellArgs& c, int t, int ntx, int
     size_t o[R];
 #pragma unroll
     for (int q = 0; q < R; ++q) o[q] = sidx(d, I, min(j0 + 4 * q, d.L - 1) + 1, K);
-    if (OP == BC_CORRECT) {
-        const size_t pl = (size_t)d.nx * d.ny;
-        const double alfxdt = c.dscale[0];
-        const double au = c.mt.au[I], cw = c.mt.cw[K], rp = c.mt.cart ? 1.0 : c.mt.rp[I];
-        double p0[R], pe[R], pn[R], pt[R], u[R], v[R], w[R], bv[R];
-#pragma unroll
-        for (int q = 0; q < R; ++q) {
-            p0[q] = c.dp[o[q]];
-            pe[q] = c.dp[o[q] + 1];
-            pn[q] = c.dp[o[q] + d.nx];
-            pt[q] = c.dp[o[q] + pl];
-            u[q] = c.us[o[q]];
-            v[q] = c.vs[o[q]];
-            w[q] = c.ws[o[q]];
-            bv[q] = c.mt.bv[min(j0 + 4 * q, d.L - 1) + 1];
-        }
-#pragma unroll
-        for (int q = 0; q < R; ++q) {
-            const int j = j0 + 4 * q;
-            if (j >= d.L) continue;
-            const long gofs = (j == d.L - 1) ? -(long)d.nx * (d.ny - 2) : ((j == 0) ? (long)d.nx * (d.ny - 2) : 0);
-            if (I <= d.nx - 3) {
-                const double uu = u[q] - au * (pe[q] - p0[q]) * alfxdt;
-                c.uo[o[q]] = uu;
-                if (gofs) c.uo[o[q] + gofs] = uu;
-            }
-            const double gv = bv[q] * (pn[q] - p0[q]) * alfxdt;
-            const double vv = v[q] - (c.mt.cart ? gv : gv / rp);
-            c.vo[o[q]] = vv;
-            if (gofs) c.vo[o[q] + gofs] = vv;
-            if (K <= d.nz - 3) {
-                const double ww = w[q] - cw * (pt[q] - p0[q]) * alfxdt;
-                c.wo[o[q]] = ww;
-                if (gofs) c.wo[o[q] + gofs] = ww;
-            }
-        }
-    } else if (OP == BC_COPY_RHS) {
+    if (OP == BC_COPY_RHS) {
         double x[R];
 #pragma unroll
         for (int q = 0; q < R; ++q) x[q] = c.dp[o[q]];
@@ -569,7 +524,7 @@ __global__ void __launch_bounds__(256) k_batch_cells(const Job<CellArgs>* jobs, 
     run_item(jobs, njobs, total, [](const Job<CellArgs>& J, int t) { cell_tile<OP>(J.a, t, J.ntx, J.aux); });
 }
 
-// CORRECT of a batch whose fields are all 16-byte aligned; alf = {ALFXDT, 1/ALFXDT} on the device.
+// CORRECT of a batch; alf = {ALFXDT, 1/ALFXDT} on the device.
 __global__ void __launch_bounds__(256) k_batch_correct(const Job<CorrArgs>* jobs, int njobs, int total,
                                                        const double* __restrict__ alf) {
     const double alfxdt = alf[0];
@@ -590,17 +545,9 @@ static int prepare_cells_t(const std::vector<BatchProblem<T>>& pr, int op, Stage
         Job<CellArgs> j{};
         CellArgs& c = j.a;
         c.d = p.d;
-        c.mt = p.mt;
-        c.us = p.us;
-        c.vs = p.vs;
-        c.ws = p.ws;
-        c.uo = p.uo;
-        c.vo = p.vo;
-        c.wo = p.wo;
         c.dp = p.dp;
         c.rhs = const_cast<double*>(p.rhs);
         c.red = p.red;
-        c.dscale = p.dscale;
         j.ntx = ceil_div(p.d.M, 64);
         j.aux = ceil_div(p.d.L, 4 * kCellRows);  // y blocks per plane
         j.ntiles = j.ntx * j.aux * p.d.N;
@@ -620,9 +567,7 @@ static int prepare_cells_t(const std::vector<BatchProblem<T>>& pr, int op, Stage
 }
 
 int prepare_cells(const std::vector<BatchProblem<double>>& pr, int op, StageLaunch& out, std::vector<void*>& owned) {
-    bool pairs = op == BC_CORRECT;
-    for (const auto& p : pr) pairs = pairs && pairs_aligned(p.us, p.vs, p.ws, p.uo, p.vo, p.wo, p.dp);
-    if (!pairs) return prepare_cells_t(pr, op, out, owned);
+    if (op != BC_CORRECT) return prepare_cells_t(pr, op, out, owned);
     std::vector<Job<CorrArgs>> jobs;
     out = StageLaunch{};
     for (const auto& p : pr) {
@@ -632,7 +577,6 @@ int prepare_cells(const std::vector<BatchProblem<double>>& pr, int op, StageLaun
         j.ntiles = j.ntx * p.d.N;
         if (!add_class_job(out, jobs, j, 0, 0)) return -1;
     }
-    out.kind = 1;
     out.alf = pr.empty() ? nullptr : pr[0].dscale;
     return upload_jobs(jobs, out, owned);
 }
@@ -642,7 +586,7 @@ int prepare_cells_f(const std::vector<BatchProblem<float>>& pr, int op, StageLau
 }
 
 void batch_cells(hipStream_t st, const StageLaunch& sl, int op) {
-    if (op == BC_CORRECT && sl.kind == 1) {
+    if (op == BC_CORRECT) {
         hipLaunchKernelGGL(k_batch_correct, dim3(std::max(sl.total, 1)), dim3(256), 0, st,
                            (const Job<CorrArgs>*)sl.jobs, sl.njobs, sl.total, sl.alf);
         return;
@@ -651,8 +595,7 @@ void batch_cells(hipStream_t st, const StageLaunch& sl, int op) {
         hipLaunchKernelGGL(fn, dim3(std::max(sl.total, 1)), dim3(256), 0, st, (const Job<CellArgs>*)sl.jobs, sl.njobs,
                            sl.total);
     };
-    if (op == BC_CORRECT) go(k_batch_cells<BC_CORRECT>);
-    else if (op == BC_COPY_RHS) go(k_batch_cells<BC_COPY_RHS>);
+    if (op == BC_COPY_RHS) go(k_batch_cells<BC_COPY_RHS>);
     else go(k_batch_cells<BC_SHIFT_GHOSTS>);
 }
 
@@ -681,12 +624,8 @@ void batch_fold(hipStream_t st, const FoldJob* jobs, int njobs) {
     if (njobs > 0) hipLaunchKernelGGL(k_batch_fold, dim3(njobs), dim3(1024), 0, st, jobs);
 }
 
-void launch_fold(hipStream_t st, const double* part, int n, double* out, int op, int add) {
-    switch (op) {
-        case RED_OP_MIN: hipLaunchKernelGGL(k_fold<RED_OP_MIN>, dim3(1), dim3(1024), 0, st, part, n, out, add); break;
-        case RED_OP_MAX: hipLaunchKernelGGL(k_fold<RED_OP_MAX>, dim3(1), dim3(1024), 0, st, part, n, out, add); break;
-        default: hipLaunchKernelGGL(k_fold<RED_OP_SUM>, dim3(1), dim3(1024), 0, st, part, n, out, add); break;
-    }
+void launch_fold(hipStream_t st, const double* part, int n, double* out) {
+    hipLaunchKernelGGL(k_fold, dim3(1), dim3(1024), 0, st, part, n, out);
 }
 
 void launch_divergence(hipStream_t st, const Dims& d, const Metrics& mt, const double* us, const double* vs,
@@ -696,31 +635,31 @@ void launch_divergence(hipStream_t st, const Dims& d, const Metrics& mt, const d
                        accumulate_compat, dscale);
     if (accumulate_compat) {
         const int nb = reduce_blocks(d);
-        launch_fold(st, rd.part, nb, rd.red + RED_VOLB, RED_OP_SUM, 0);
+        launch_fold(st, rd.part, nb, rd.red + RED_VOLB);
         launch_fill(st, rd.red + RED_VOL, 1, mt.vol_total);
     }
 }
 
 void launch_div_minmax(hipStream_t st, const Dims& d, const Metrics& mt, const double* us, const double* vs,
-                       const double* ws, const Reduce& rd) {
-    hipLaunchKernelGGL(k_div_minmax, red_grid(d), kCellBlock, 0, st, d, mt, us, vs, ws, rd.part);
-    const int nb = reduce_blocks(d);
-    launch_fold(st, rd.part, nb, rd.red + RED_DMIN, RED_OP_MIN, 0);
-    launch_fold(st, rd.part + nb, nb, rd.red + RED_DMAX, RED_OP_MAX, 0);
+                       const double* ws, const Reduce& rd, double* log, int* step, int cap) {
+    // at most M blocks a plane: the partials hold M * N of each
+    // (planes per block: as many as leave 1024 blocks, at most 8; whole calls at 768 x 384 x 256 with 1,
+    // 2, 4, 8 planes: 0.492, 0.411, 0.379, 0.370 ms, 0.436 with one row per thread; at 64 x 64 x 32: 28, 29, 30, 33 us)
+    const int nbx = std::min(span_blocks(d), d.M);
+    const int planes = std::max(1, std::min(8, (int)((long)span_blocks(d) * d.N / 1024)));
+    const int nb = nbx * ceil_div(d.N, planes);
+    const int runs = 3 * sizeof(double) * (size_t)d.nx * d.ny * d.nz > ((size_t)256 << 20);
+    hipLaunchKernelGGL(k_div_minmax, dim3(nb), dim3(256), 0, st, d, mt, us, vs, ws, rd.part, row_magic(d), nbx, planes,
+                       runs);
+    hipLaunchKernelGGL(k_fold_minmax, dim3(1), dim3(1024), 0, st, rd.part, nb, rd.red, log, step, cap);
 }
 
 void launch_correct(hipStream_t st, const Dims& d, const Metrics& mt, const double* us, const double* vs,
                     const double* ws, double* uo, double* vo, double* wo, const double* dp, double alfxdt,
                     int refresh_periodic, const double* dscale) {
-    if (pairs_aligned(us, vs, ws, uo, vo, wo, dp)) {
-        const int runs = 7 * sizeof(double) * (size_t)d.nx * d.ny * d.nz > ((size_t)256 << 20);
-        hipLaunchKernelGGL(k_correct_span, dim3(span_blocks(d) * d.N), dim3(256), 0, st,
-                           corr_args(d, mt, us, vs, ws, uo, vo, wo, dp), alfxdt, refresh_periodic, runs, dscale);
-        return;
-    }
-    const dim3 grid(ceil_div(d.M, 64), ceil_div(d.L, 4 * kCorrectRows), d.N);
-    hipLaunchKernelGGL(k_correct<kCorrectRows>, grid, kCellBlock, 0, st, d, mt, us, vs, ws, uo, vo, wo, dp, alfxdt,
-                       refresh_periodic, dscale);
+    const int runs = 7 * sizeof(double) * (size_t)d.nx * d.ny * d.nz > ((size_t)256 << 20);
+    hipLaunchKernelGGL(k_correct_span, dim3(span_blocks(d) * d.N), dim3(256), 0, st,
+                       corr_args(d, mt, us, vs, ws, uo, vo, wo, dp), alfxdt, refresh_periodic, runs, dscale);
 }
 
 void launch_laplacian(hipStream_t st, const Dims& d, const Op64& op, const double* phi, double* out) {
@@ -732,7 +671,7 @@ void launch_finalize(hipStream_t st, const Dims& d, const Op64& op, double* phi,
     // the residual reads phi's neighbours, so it runs before the shift rewrites phi
     if (rhs) {
         hipLaunchKernelGGL(k_resid_sumsq, red_grid(d), kCellBlock, 0, st, d, op, phi, rhs, rd.part);
-        launch_fold(st, rd.part, reduce_blocks(d), rd.red + RED_RNORM2, RED_OP_SUM, 0);
+        launch_fold(st, rd.part, reduce_blocks(d), rd.red + RED_RNORM2);
     }
     hipLaunchKernelGGL(k_shift_ghosts, cell_grid(d), kCellBlock, 0, st, d, phi, (const double*)rd.red);
 }
@@ -740,14 +679,14 @@ void launch_finalize(hipStream_t st, const Dims& d, const Op64& op, double* phi,
 void launch_rhs_check(hipStream_t st, const Dims& d, const Metrics& mt, const double* b, const Reduce& rd) {
     const int nb = reduce_blocks(d);
     hipLaunchKernelGGL(k_rhs_check, red_grid(d), kCellBlock, 0, st, d, mt, b, rd.part, nb);
-    launch_fold(st, rd.part, nb, rd.red + RED_CHK_VB, RED_OP_SUM, 0);
-    launch_fold(st, rd.part + nb, nb, rd.red + RED_CHK_VABS, RED_OP_SUM, 0);
-    launch_fold(st, rd.part + 2 * nb, nb, rd.red + RED_CHK_NF, RED_OP_SUM, 0);
+    launch_fold(st, rd.part, nb, rd.red + RED_CHK_VB);
+    launch_fold(st, rd.part + nb, nb, rd.red + RED_CHK_VABS);
+    launch_fold(st, rd.part + 2 * nb, nb, rd.red + RED_CHK_NF);
 }
 
 void launch_sumsq(hipStream_t st, const Dims& d, const double* a, const Reduce& rd, int slot) {
     hipLaunchKernelGGL(k_sumsq, red_grid(d), kCellBlock, 0, st, d, a, rd.part);
-    launch_fold(st, rd.part, reduce_blocks(d), rd.red + slot, RED_OP_SUM, 0);
+    launch_fold(st, rd.part, reduce_blocks(d), rd.red + slot);
 }
 
 void launch_copy_shift(hipStream_t st, const Dims& d, const double* src, double* dst, const double* red) {

@@ -722,13 +722,13 @@ void launch_yfft_fwd(hipStream_t st, const Dims& d, const FftPlan& fp, const Tab
             else go(k_yfft_fwd<T, YF_DIV_CYL, false>);
         }
         if (in.fold) {
-            launch_fold(st, rd.part, (int)(grid.x * grid.y), rd.red + RED_VOLB, RED_OP_SUM, 0);
+            launch_fold(st, rd.part, (int)(grid.x * grid.y), rd.red + RED_VOLB);
             launch_fill(st, rd.red + RED_VOL, 1, in.mt.vol_total);
         }
     } else {
         if (dense) go(k_yfft_fwd<T, YF_RESIDUAL, true>);
         else go(k_yfft_fwd<T, YF_RESIDUAL, false>);
-        launch_fold(st, rd.part, (int)(grid.x * grid.y), rd.red + RED_RNORM2, RED_OP_SUM, 0);
+        launch_fold(st, rd.part, (int)(grid.x * grid.y), rd.red + RED_RNORM2);
     }
 }
 
@@ -767,7 +767,7 @@ void launch_yfft_inv(hipStream_t st, const Dims& d, const FftPlan& fp, const Tab
         case YI_STORE:
             if (dense) go(k_yfft_inv<T, YI_STORE, true>);
             else go(k_yfft_inv<T, YI_STORE, false>);
-            launch_fold(st, rd.part, (int)(grid.x * grid.y), rd.red + RED_PHISUM, RED_OP_SUM, 0);
+            launch_fold(st, rd.part, (int)(grid.x * grid.y), rd.red + RED_PHISUM);
             break;
         case YI_UPDATE_FINAL:
             if (dense) go(k_yfft_inv<T, YI_UPDATE_FINAL, true>);
@@ -776,7 +776,7 @@ void launch_yfft_inv(hipStream_t st, const Dims& d, const FftPlan& fp, const Tab
         default:
             if (dense) go(k_yfft_inv<T, YI_UPDATE, true>);
             else go(k_yfft_inv<T, YI_UPDATE, false>);
-            launch_fold(st, rd.part, (int)(grid.x * grid.y), rd.red + RED_PHISUM, RED_OP_SUM, 0);
+            launch_fold(st, rd.part, (int)(grid.x * grid.y), rd.red + RED_PHISUM);
             break;
     }
 }

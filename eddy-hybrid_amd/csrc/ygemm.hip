@@ -219,7 +219,7 @@ void launch_ygemm_fwd(hipStream_t st, const Dims& d, const float* FT, const FwdI
     const size_t sh = (size_t)d.L * kGemmPencils * sizeof(float);
     if (in.mode == YF_RESIDUAL) {
         hipLaunchKernelGGL(k_ygemm_fwd<YF_RESIDUAL>, grid, dim3(256), sh, st, a);
-        launch_fold(st, rd.part, (int)(grid.x * grid.y), rd.red + RED_RNORM2, RED_OP_SUM, 0);
+        launch_fold(st, rd.part, (int)(grid.x * grid.y), rd.red + RED_RNORM2);
     } else {
         hipLaunchKernelGGL(k_ygemm_fwd<YF_DIRECT>, grid, dim3(256), sh, st, a);
     }
@@ -238,7 +238,7 @@ void launch_ygemm_inv(hipStream_t st, const Dims& d, const float* GT, const floa
     const size_t sh = (size_t)d.L * kGemmPencils * sizeof(float);
     if (mode == YI_STORE) hipLaunchKernelGGL(k_ygemm_inv<YI_STORE>, grid, dim3(256), sh, st, a);
     else hipLaunchKernelGGL(k_ygemm_inv<YI_UPDATE>, grid, dim3(256), sh, st, a);
-    launch_fold(st, rd.part, (int)(grid.x * grid.y), rd.red + RED_PHISUM, RED_OP_SUM, 0);
+    launch_fold(st, rd.part, (int)(grid.x * grid.y), rd.red + RED_PHISUM);
 }
 
 }  // namespace eddy
