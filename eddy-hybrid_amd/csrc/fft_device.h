@@ -207,13 +207,16 @@ __device__ void cfft_lds_ip(T* __restrict__ xr, T* __restrict__ xi, int ld, int 
 }
 
 // ------------------------------------------------------------------ compile-time radix plans
-// The same in-place passes with the length and the radices fixed at compile time, for the
-// power-of-two plans radix_plan makes with radices up to 8 (n = 16 ... 512). With n, R and the
-// span Ns constants, the butterfly's pencil, block and twiddle indices are shifts and masks,
-// and every LDS address of a butterfly is one computed base plus constant offsets: for
-// power-of-two strides the padded index pidx(base + r*s) equals pidx(base) + r*s + (r*s >> 3)
-// whenever base is aligned as the pass aligns it (the loads: base = jj < s or s % 8 == 0; the
-// stores: base = blk*Ns*R + k with k < Ns), so the offsets fold into the LDS instructions.
+// The same in-place passes with the length and the radices fixed at compile time, for the plans that
+// radix_plan makes of n = 16 ... 512 and of n = 24, 48, 96, 192 (periodic lengths and x2 counts of
+// 48 to 384) with radices up to 8. With n, R and the span Ns constants, the butterfly's pencil,
+// block and twiddle indices are shifts and masks (or one constant product), and where the strides are
+// multiples of 8 or do not carry into the padding every LDS address of a butterfly is one computed
+// base plus constant offsets: pidx(base + r*s) equals pidx(base) + r*s + (r*s >> 3) whenever
+// s % 8 == 0, or when base is a multiple of 8 and r*s < 8, so the offsets fold into the LDS
+// instructions. 768 x 384 x 256, whose x2 transforms have n = 192: 0.350 -> 0.289 ms forward and 0.367 ->
+// 0.296 inverse over the run-time passes; projections of 192 x 192 x 96 0.167 -> 0.149 ms. (Run-time
+// passes with a function per radix took 25 to 32 more registers and ran 10 % slower.)
 __device__ __forceinline__ constexpr int poff(int x) { return x + (x >> 3); }
 
 template <typename T, bool WAVE, int n, int R, int Ns>
@@ -221,17 +224,25 @@ __device__ __forceinline__ void cfft_pass_static(T* __restrict__ xr, T* __restri
                                                  const T* twr, const T* twi, T dir, int tid) {
     constexpr int nb = n / R;
     constexpr int tstep = n / (Ns * R);
+    // loads at jj + r*nb: whole padding steps apart, or jj < nb <= 8 a power of two (no carry)
+    constexpr bool lin_load = nb % 8 == 0 || 8 % nb == 0;
+    // stores at blk*Ns*R + k + r*Ns, k < Ns
+    constexpr bool lin_store = Ns % 8 == 0 || (8 % Ns == 0 && ((Ns * R) % 8 == 0 || 8 % (Ns * R) == 0));
     const bool active = tid < P * nb;
     Cx<T> v[R];
-    int oaddr = 0;
+    int orow = 0, ob = 0;
     if (active) {
-        const int pen = tid / nb;  // powers of two: shifts and masks
+        const int pen = tid / nb;  // constants: shifts and masks for powers of two
         const int jj = tid - pen * nb;
         const int blk = jj / Ns;
         const int k = jj - blk * Ns;
-        const int ia = pen * ld + pidx(jj);
+        orow = pen * ld;
+        const int ia = orow + pidx(jj);
 #pragma unroll
-        for (int r = 0; r < R; ++r) v[r] = {xr[ia + poff(r * nb)], xi[ia + poff(r * nb)]};
+        for (int r = 0; r < R; ++r) {
+            const int o = lin_load ? ia + poff(r * nb) : orow + pidx(jj + r * nb);
+            v[r] = {xr[o], xi[o]};
+        }
         if (Ns > 1) {
 #pragma unroll
             for (int r = 1; r < R; ++r) {
@@ -242,16 +253,19 @@ __device__ __forceinline__ void cfft_pass_static(T* __restrict__ xr, T* __restri
             }
         }
         if constexpr (R == 2) dft2(v);
+        else if constexpr (R == 3) dft3(v, dir);
         else if constexpr (R == 4) dft4(v, dir);
         else dft8(v, dir);
-        oaddr = pen * ld + pidx(blk * Ns * R + k);
+        ob = blk * Ns * R + k;
     }
     fft_sync<WAVE>();
     if (active) {
+        const int oa = orow + pidx(ob);
 #pragma unroll
         for (int r = 0; r < R; ++r) {
-            xr[oaddr + poff(r * Ns)] = v[r].re;
-            xi[oaddr + poff(r * Ns)] = v[r].im;
+            const int o = lin_store ? oa + poff(r * Ns) : orow + pidx(ob + r * Ns);
+            xr[o] = v[r].re;
+            xi[o] = v[r].im;
         }
     }
     fft_sync<WAVE>();
@@ -274,8 +288,7 @@ __device__ __forceinline__ bool plan_is(const FftPlan& fp) {
     return true;
 }
 
-// cfft_lds_ip with the power-of-two plans of radix_plan (largest radix 8) taken by the
-// compile-time passes; every other plan by the run-time passes. Same contract.
+// cfft_lds_ip with the plans listed above (largest radix 8) taken by the compile-time passes; every other plan by the run-time passes. Same contract.
 template <typename T, bool WAVE = false>
 __device__ __forceinline__ void cfft_lds(T* __restrict__ xr, T* __restrict__ xi, int ld, int P, const FftPlan& fp,
                                          const T* twr, const T* twi, T dir, int tid, int nthr) {
@@ -286,6 +299,11 @@ __device__ __forceinline__ void cfft_lds(T* __restrict__ xr, T* __restrict__ xi,
     else if (fp.n == 512 && plan_is<8, 8, 8>(fp))
         cfft_passes_static<T, WAVE, 512, 1, 8, 8, 8>(xr, xi, ld, P, twr, twi, dir, tid);
     else if (fp.n == 32 && plan_is<8, 4>(fp)) cfft_passes_static<T, WAVE, 32, 1, 8, 4>(xr, xi, ld, P, twr, twi, dir, tid);
+    else if (fp.n == 192 && plan_is<8, 8, 3>(fp))
+        cfft_passes_static<T, WAVE, 192, 1, 8, 8, 3>(xr, xi, ld, P, twr, twi, dir, tid);
+    else if (fp.n == 96 && plan_is<8, 4, 3>(fp)) cfft_passes_static<T, WAVE, 96, 1, 8, 4, 3>(xr, xi, ld, P, twr, twi, dir, tid);
+    else if (fp.n == 48 && plan_is<4, 4, 3>(fp)) cfft_passes_static<T, WAVE, 48, 1, 4, 4, 3>(xr, xi, ld, P, twr, twi, dir, tid);
+    else if (fp.n == 24 && plan_is<8, 3>(fp)) cfft_passes_static<T, WAVE, 24, 1, 8, 3>(xr, xi, ld, P, twr, twi, dir, tid);
     else if (fp.n == 16 && plan_is<4, 4>(fp)) cfft_passes_static<T, WAVE, 16, 1, 4, 4>(xr, xi, ld, P, twr, twi, dir, tid);
     else cfft_lds_ip<T, WAVE>(xr, xi, ld, P, fp, twr, twi, dir, tid, nthr);
 }
