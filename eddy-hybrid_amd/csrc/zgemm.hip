@@ -21,6 +21,7 @@
 #include "kernels.h"
 #include "mma_device.h"
 #include "reduce_device.h"
+#include "stencil_device.h"
 
 namespace eddy {
 
@@ -51,8 +52,8 @@ __global__ void __launch_bounds__(256) k_zgemm_delta(T* X0, const T* linesum, co
 // A[p + r*lda], Bop(p, c) = B[p + c*ldb]; the x1-form forward product) or contiguous along
 // their own index ("x-major": A[r + p*lda], B[c + p*ldb]; every other product).
 //
-// A workgroup (4 waves, 2 x 2) owns a BR x BC tile of C, each wave a (BR/2) x (BC/2) block of
-// 16 x 16 MFMA tiles (v_mfma_f64_16x16x4f64 / v_mfma_f32_16x16x4f32). The contraction runs in
+// FP32 (k_mma): a workgroup (4 waves, 2 x 2) owns a BR x BC tile of C, each wave a (BR/2) x (BC/2) block
+// of 16 x 16 MFMA tiles (v_mfma_f32_16x16x4f32; FP64 v_mfma_f64_16x16x4f64). The contraction runs in
 // chunks of KC staged in LDS, in two buffers: the next chunk's global loads are in flight
 // while the MFMAs of the current one run, one barrier per chunk.
 // MFMA 16x16x4 lane layout: lane l supplies A(l%16, l/16) and B(l/16, l%16); accumulator
@@ -535,6 +536,222 @@ static bool dma_ok(const MmArgs<double>& a) {
            (a.P % 2 == 0) && (a.R % 2 == 0) && (a.Cn % 2 == 0) && a.P >= 2 && a.R >= 2 && a.Cn >= 2;
 }
 
+// ---- FP64 products with the operands straight in registers -----------------------------------
+//
+// An FP64 16 x 16 x 4 product occupies its matrix core for 64 cycles, so a wave that owns
+// (16 NR) x (16 NC) of C needs only NR + NC 512-byte operand loads for NR * NC products of 64 cycles: little
+// enough to come from L1 and L2 without LDS. Each wave loads its own operands, eight contraction
+// indices at a time and one group ahead of the products that use them, and runs to its end without
+// a barrier or a copy to wait for together. C's edge costs what it holds: 16-row blocks wholly
+// outside run no products, and no other wave waits for the one that has fewer.
+// Operands of any alignment and length: p-major rows are read as pairs (16-byte loads at 8-byte
+// alignment), rows past the end repeat the last one, the contraction's last P mod 8 indices are
+// taken four at a time with zeros past P.
+typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));
+
+// What the zero mode adds to its operands.
+struct ZeroMode {
+    double shift, deltaA, deltaB;
+    int dnull;
+};
+
+// One wave's (16 NR) x (16 NC) of C at (r0, c0). SLOW: the tile reaches past C's end (blocks
+// nri x nci of it run) or belongs to the zero mode; the plain tile carries neither's registers.
+template <bool PM, int NR, int NC, bool SLOW>
+__device__ __forceinline__ void mma64_tile(const MmArgs<double>& a, const double* __restrict__ A,
+                                           const double* __restrict__ B, double* __restrict__ C, int r0, int c0,
+                                           int lane, const ZeroMode& z) {
+    typedef Mma<double>::v4 v4;
+    const int x = lane & 15, q = lane >> 4;
+    const int nri = SLOW ? min(NR, (a.R - r0 + 15) / 16) : NR, nci = SLOW ? min(NC, (a.Cn - c0 + 15) / 16) : NC;
+    // byte offsets of the lane's rows: of contraction index 2q (p-major) or q (x-major)
+    unsigned oa[NR], ob[NC];
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+        const unsigned r = (unsigned)min(r0 + 16 * i + x, a.R - 1);
+        oa[i] = 8u * (PM ? r * (unsigned)a.lda + 2u * q : r + (unsigned)q * (unsigned)a.lda);
+    }
+#pragma unroll
+    for (int j = 0; j < NC; ++j) {
+        const unsigned c = (unsigned)min(c0 + 16 * j + x, a.Cn - 1);
+        ob[j] = 8u * (PM ? c * (unsigned)a.ldb + 2u * q : c + (unsigned)q * (unsigned)a.ldb);
+    }
+    v4 acc[NR][NC];
+#pragma unroll
+    for (int i = 0; i < NR; ++i)
+#pragma unroll
+        for (int j = 0; j < NC; ++j) acc[i][j] = v4{0.0, 0.0, 0.0, 0.0};
+
+    // one step of four contraction indices, p the lane's
+    auto step = [&](int p, double (&av)[NR], double (&bv)[NC]) {
+        if (SLOW) {
+            const bool null = p == z.dnull;
+#pragma unroll
+            for (int i = 0; i < NR; ++i) av[i] = av[i] - z.shift + (null ? z.deltaA : 0.0);
+#pragma unroll
+            for (int j = 0; j < NC; ++j) bv[j] += null ? z.deltaB : 0.0;
+        }
+#pragma unroll
+        for (int i = 0; i < NR; ++i)
+#pragma unroll
+            for (int j = 0; j < NC; ++j)
+                if (!SLOW || (i < nri && j < nci)) acc[i][j] = Mma<double>::run(bv[j], av[i], acc[i][j]);
+    };
+    // contraction indices 8t .. 8t+7: step s of lane group q is 8t + 2q + s (p-major), 8t + 4s + q (x-major)
+    auto load = [&](int t, double (&av)[2][NR], double (&bv)[2][NC]) {
+        if (PM) {
+            const double *pa = A + 8 * (size_t)t, *pb = B + 8 * (size_t)t;
+#pragma unroll
+            for (int i = 0; i < NR; ++i) {
+                const d2u v = *reinterpret_cast<const d2u*>(reinterpret_cast<const char*>(pa) + oa[i]);
+                av[0][i] = v.x;
+                av[1][i] = v.y;
+            }
+#pragma unroll
+            for (int j = 0; j < NC; ++j) {
+                const d2u v = *reinterpret_cast<const d2u*>(reinterpret_cast<const char*>(pb) + ob[j]);
+                bv[0][j] = v.x;
+                bv[1][j] = v.y;
+            }
+        } else {
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                const double* pa = A + (size_t)(8 * t + 4 * s) * a.lda;
+                const double* pb = B + (size_t)(8 * t + 4 * s) * a.ldb;
+#pragma unroll
+                for (int i = 0; i < NR; ++i) av[s][i] = ld_off(pa, oa[i]);
+#pragma unroll
+                for (int j = 0; j < NC; ++j) bv[s][j] = ld_off(pb, ob[j]);
+            }
+        }
+    };
+    auto use = [&](int t, double (&av)[2][NR], double (&bv)[2][NC]) {
+        step(PM ? 8 * t + 2 * q : 8 * t + q, av[0], bv[0]);
+        step(PM ? 8 * t + 2 * q + 1 : 8 * t + 4 + q, av[1], bv[1]);
+    };
+    const int T = a.P >> 3;
+    if (T > 0) {
+        // one group ahead (two or three ahead measured the same: the waves of a SIMD cover the latency)
+        double a0[2][NR], b0[2][NC], a1[2][NR], b1[2][NC];
+        load(0, a0, b0);
+        for (int t = 0; t < T; t += 2) {
+            load(min(t + 1, T - 1), a1, b1);
+            use(t, a0, b0);
+            if (t + 1 == T) break;
+            load(min(t + 2, T - 1), a0, b0);
+            use(t + 1, a1, b1);
+        }
+    }
+    for (int p0 = 8 * T; p0 < a.P; p0 += 4) {
+        const int p = p0 + q, pc = min(p, a.P - 1);
+        const bool ok = p < a.P;
+        double av[NR], bv[NC];
+#pragma unroll
+        for (int i = 0; i < NR; ++i) {
+            const int r = min(r0 + 16 * i + x, a.R - 1);
+            av[i] = A[PM ? (size_t)r * a.lda + pc : (size_t)r + (size_t)pc * a.lda];
+        }
+#pragma unroll
+        for (int j = 0; j < NC; ++j) {
+            const int c = min(c0 + 16 * j + x, a.Cn - 1);
+            bv[j] = B[PM ? (size_t)c * a.ldb + pc : (size_t)c + (size_t)pc * a.ldb];
+        }
+        // past P: both operands 0 (the zero mode's shift is undone by B's 0)
+#pragma unroll
+        for (int i = 0; i < NR; ++i) av[i] = ok ? av[i] : 0.0;
+#pragma unroll
+        for (int j = 0; j < NC; ++j) bv[j] = ok ? bv[j] : 0.0;
+        step(ok ? p : -2, av, bv);
+    }
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+        const int gr = r0 + 16 * i + x;
+        if (SLOW && gr >= a.R) continue;
+#pragma unroll
+        for (int j = 0; j < NC; ++j)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int gc = c0 + 16 * j + Mma<double>::row(q, v);
+                if (!SLOW || gc < a.Cn) C[(size_t)gr + (size_t)gc * a.ldc] = acc[i][j][v];
+            }
+    }
+}
+
+template <bool PM, int NR, int NC>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NR * NC >= 16 ? 2 : (NR * NC >= 8 ? 3 : 4))))
+k_mma64(MmArgs<double> a) {
+    __shared__ double scratch[16];
+    const int tid = threadIdx.x, nthr = blockDim.x;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int tile = xcd_tile(blockIdx.x, gridDim.x);
+    const int ct = tile % a.ntc, rest = tile / a.ntc;
+    const int b = rest / a.ntr, rt = (rest - b * a.ntr) * (nthr >> 6) + wv;
+    const int r0 = rt * 16 * NR, c0 = ct * 16 * NC;
+    const double* A = a.A + (size_t)b * a.sA;
+    const double* B = a.B + (size_t)b * a.sB;
+    double* C = a.C + (size_t)b * a.sC;
+    if (b != a.zb && r0 + 16 * NR <= a.R && c0 + 16 * NC <= a.Cn) {
+        mma64_tile<PM, NR, NC, false>(a, A, B, C, r0, c0, tid & 63, ZeroMode{});
+        return;
+    }
+    // the zero mode: shift and delta (the same for every workgroup of that batch)
+    ZeroMode z{0.0, 0.0, 0.0, -1};
+    if (b == a.zb) {
+        z.shift = a.shiftL * mean_shift(a.shift, scratch);
+        if (a.linesum) {
+            double s = 0.0;
+            for (int m = tid; m < a.dn; m += nthr) s += a.wsum[m] * a.linesum[m];
+            s = wave_sum(s);
+            if ((tid & 63) == 0) scratch[wv] = s;
+            __syncthreads();
+            double tot = 0.0;
+            for (int w = 0; w < nthr >> 6; ++w) tot += scratch[w];
+            const double delta = -tot / (a.wsum[a.dnull] * a.dnorm);
+            z.dnull = a.dnull;
+            (a.dop == 0 ? z.deltaA : z.deltaB) = delta;
+        }
+    }
+    if (r0 < a.R) mma64_tile<PM, NR, NC, true>(a, A, B, C, r0, c0, tid & 63, z);
+}
+
+template <bool PM, int NR, int NC>
+static void launch_mma64_tiles(hipStream_t st, MmArgs<double> a) {
+    const int wr = ceil_div(a.R, 16 * NR);  // wave tiles along r
+    // waves of a workgroup: consecutive row tiles, as many as divide them evenly
+    const int nw = wr % 4 == 0 ? 4 : (wr % 2 == 0 ? 2 : 1);
+    a.ntr = wr / nw;
+    a.ntc = ceil_div(a.Cn, 16 * NC);
+    hipLaunchKernelGGL((k_mma64<PM, NR, NC>), dim3((unsigned)((long)a.ntr * a.ntc * a.nb)), dim3(64 * nw), 0, st, a);
+}
+
+// Tiles of 16 nr x 16 nc of all products, and the product steps of a SIMD that runs its share of them
+// one after another (1024 SIMDs).
+static long mma64_tiles(const MmArgs<double>& a, int nr, int nc) {
+    return (long)ceil_div(a.R, 16 * nr) * ceil_div(a.Cn, 16 * nc) * a.nb;
+}
+static long mma64_steps(const MmArgs<double>& a, int nr, int nc) {
+    return ((mma64_tiles(a, nr, nc) + 1023) / 1024) * nr * nc;
+}
+
+// The FP64 products. Two tiles of 64 x 64 per SIMD or more: the LDS-staged kernel where its copies
+// are aligned (302 x 130 x 1026: 0.432 + 0.429 ms a pair of products, 0.446 + 0.423 straight from registers;
+// 512 x 256 x 64 0.174 and 0.170), else 64 x 64 tiles from registers (301 x 501 x 64: 0.289 against 0.302 ms of
+// the register-staged LDS kernel they replace). Fewer: the register kernel with the tile that gives
+// every SIMD at least two waves in the fewest steps (a pair of products, LDS-staged before and now:
+// 256 x 192 x 128 0.114 -> 0.106 ms with 32 x 64, 150 x 150 x 150 0.088 -> 0.068, 203 x 101 x 90 0.0445 -> 0.0402,
+// 395 x 161 x 24 0.0527 -> 0.0473 and 128 x 179 x 10 0.0283 -> 0.0251 with 32 x 32; all at stretched or odd x2).
+template <bool PM>
+static void launch_mma64(hipStream_t st, const MmArgs<double>& a) {
+    if (mma64_tiles(a, 4, 4) >= 2048) {
+        if (dma_ok(a)) launch_mma_dma<PM>(st, a);
+        else launch_mma64_tiles<PM, 4, 4>(st, a);
+    } else if (mma64_tiles(a, 2, 4) >= 2048 && mma64_steps(a, 2, 4) <= mma64_steps(a, 2, 2)) {
+        launch_mma64_tiles<PM, 2, 4>(st, a);
+    } else {
+        launch_mma64_tiles<PM, 2, 2>(st, a);
+    }
+}
+
 template <typename T, bool PM, int BR, int BC>
 static void launch_mma_tiles(hipStream_t st, MmArgs<T> a) {
     a.ntr = ceil_div(a.R, BR);
@@ -545,18 +762,15 @@ static void launch_mma_tiles(hipStream_t st, MmArgs<T> a) {
     hipLaunchKernelGGL((k_mma<T, PM, BR, BC>), dim3((unsigned)nwg), dim3(256), sh, st, a);
 }
 
-// 64 x 64 tiles; FP64 with the DMA-staged kernel where its copies are aligned
 template <typename T>
 static void launch_mma(hipStream_t st, bool pmajor, const MmArgs<T>& a) {
     if constexpr (std::is_same<T, double>::value) {
-        if (dma_ok(a)) {
-            if (pmajor) launch_mma_dma<true>(st, a);
-            else launch_mma_dma<false>(st, a);
-            return;
-        }
+        if (pmajor) launch_mma64<true>(st, a);
+        else launch_mma64<false>(st, a);
+    } else {
+        if (pmajor) launch_mma_tiles<T, true, 64, 64>(st, a);
+        else launch_mma_tiles<T, false, 64, 64>(st, a);
     }
-    if (pmajor) launch_mma_tiles<T, true, 64, 64>(st, a);
-    else launch_mma_tiles<T, false, 64, 64>(st, a);
 }
 
 template <typename T>
