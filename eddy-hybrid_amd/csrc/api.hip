@@ -86,6 +86,7 @@ static bool radix_plan(int n, FftPlan& fp, int maxr = 8) {
             r /= f;
         }
     }
+    fp.fixed = fixed_plan(fp);
     return r == 1;
 }
 
@@ -683,11 +684,7 @@ static int create_plan(eddy_plan_s** out, int nx, int ny, int nz, double delysq,
     P->np = np;
     P->delysq = delysq;
     P->stream = static_cast<hipStream_t>(stream);
-    // y-transform tiles of at least 4096 elements where M allows: L/2-point FFTs over TI
-    // pencils then give every one of the 256 threads a radix-8 butterfly in each pass
     P->tune.yfft_pencils = 16;
-    while (P->tune.yfft_pencils < 64 && P->tune.yfft_pencils < M && (long)P->tune.yfft_pencils * L < 4096)
-        P->tune.yfft_pencils *= 2;
     P->tune.ztrans_pencils = 16;
     P->tune.xsolve_chunk = 12;
     P->tune.use_dense_z = 0;
@@ -720,22 +717,32 @@ static int create_plan(eddy_plan_s** out, int nx, int ny, int nz, double delysq,
     }
     HIP_TRY(hipGetDevice(&P->device));
     // Keep every kernel's LDS within the 160 KiB of a gfx950 CU (FP64 sizes bound FP32), and
-    // the in-place FFTs at one butterfly per thread and pass (tile width x half-length /
-    // smallest radix <= kFftThreads = 512).
+    // the in-place FFTs at the butterflies that 512 threads hold in a pass (fft_tile_ok).
     const size_t lds_cap = 160 * 1024;
+    // Transform tiles start at 16 pencils (a row of a tile is a full 128-byte line) and double, up to
+    // 64, while they hold fewer than 4096 elements and three workgroups of the doubled tile still share
+    // a CU's LDS: 32 pencils of 144 to 160 elements run 2 to 13 % faster than 16, but 32 of 192 (two
+    // workgroups) 11 % slower in the inverse y transform and 9 % in the forward x2 transform.
+    auto tile_grows = [&](int ti, long len, size_t doubled) {
+        return ti < 64 && ti < M && ti * len < 4096 && 3 * doubled <= lds_cap;
+    };
     // the y transform: the radix FFT of L/2 complex points for an even L whose half factors
     // into 2, 3 and 5; any other periodic length (fftpack's general odd factors, fftpack.f:2096-
     // 2123) takes the dense real DFT, marked by a radix plan of length 0
     const bool ydense = (L % 2) || !radix_plan(L / 2, P->fpy, P->tune.fft_radix);
-    if (ydense) P->fpy = FftPlan{0, 0, {}};
+    if (ydense) P->fpy = FftPlan{0, 0, {}, 0};
     {
         auto ylds = [&](int ti) {
             return ydense ? (size_t)ti * dft_pitch(L) * sizeof(double)
                           : (2 * (size_t)ti * fft_ld(L / 2) + 4 * (size_t)fft_ld(L / 2)) * sizeof(double);
         };
         auto yok = [&](int ti) {
-            return ylds(ti) <= lds_cap && (ydense || (long)ti * (L / 2) <= (long)min_radix(P->fpy) * kFftThreads);
+            return ylds(ti) <= lds_cap && (ydense || (L / 2 <= min_radix(P->fpy) * kFftThreads &&
+                                                      fft_tile_ok(P->fpy, ti, kFftThreads)));
         };
+        if (!(tuning && tuning->yfft_pencils > 0))
+            while (tile_grows(P->tune.yfft_pencils, L, ydense ? 0 : ylds(2 * P->tune.yfft_pencils)))
+                P->tune.yfft_pencils *= 2;
         while (P->tune.yfft_pencils > 1 && !yok(P->tune.yfft_pencils)) P->tune.yfft_pencils /= 2;
         // (the dense DFT's matrices grow with L^2: lengths above 6500 or so stay refused)
         if (!yok(P->tune.yfft_pencils) || (ydense && (fft_ld(L) + 2 * (size_t)L) * sizeof(double) > lds_cap)) {
@@ -862,17 +869,16 @@ static int create_plan(eddy_plan_s** out, int nx, int ny, int nz, double delysq,
     // x2 tile width: the DCT's in-place FFT as above; the dense transform works on groups of
     // 4 lines staged whole in LDS.
     {
+        auto zlds = [&](int ti) { return (2 * (size_t)ti * fft_ld(N / 2) + 4 * (size_t)N + 2) * sizeof(double); };
         auto zok = [&](int ti) {
             if (P->dense) return (size_t)N * ti * sizeof(double) <= lds_cap;
-            return (2 * (size_t)ti * fft_ld(N / 2) + 4 * (size_t)N + 2) * sizeof(double) <= lds_cap &&
-                   (long)ti * (N / 2) <= (long)min_radix(P->fpz) * kFftThreads;
+            return zlds(ti) <= lds_cap && N / 2 <= min_radix(P->fpz) * kFftThreads &&
+                   fft_tile_ok(P->fpz, ti, kFftThreads);
         };
         const int zmin = P->dense ? 4 : 1;
-        // the DCT of a short x2 takes more pencils per tile (at least 4096 elements where M
-        // allows), as the y transform does
         if (!P->dense && !(tuning && tuning->ztrans_pencils > 0))
-            while (P->tune.ztrans_pencils < 64 && P->tune.ztrans_pencils < M &&
-                   (long)P->tune.ztrans_pencils * N < 4096 && zok(2 * P->tune.ztrans_pencils))
+            while (tile_grows(P->tune.ztrans_pencils, N, zlds(2 * P->tune.ztrans_pencils)) &&
+                   zok(2 * P->tune.ztrans_pencils))
                 P->tune.ztrans_pencils *= 2;
         while (P->tune.ztrans_pencils > zmin && !zok(P->tune.ztrans_pencils)) P->tune.ztrans_pencils /= 2;
         if (!zok(P->tune.ztrans_pencils)) {
@@ -958,7 +964,7 @@ static int create_plan(eddy_plan_s** out, int nx, int ny, int nz, double delysq,
                 h.qiT[(size_t)m * N + k] = u * sq[k];  // A[s=m][o=k] = Qinv(k,m)
                 h.wsum[m] += u * sq[k];
             }
-        P->fpz = FftPlan{1, 0, {}};
+        P->fpz = FftPlan{1, 0, {}, 0};
     }
     // y real FFT tables (L = 2H; radix plan made above), or the dense DFT's matrices
     if (ydense) {

@@ -15,6 +15,7 @@ struct FftPlan {
     int n;
     int count;
     int rad[kMaxRadices];
+    int fixed;  // n where the compile-time passes take the plan, else 0
 };
 
 // Operator and transform tables of one plan, in the precision T of the kernels that read

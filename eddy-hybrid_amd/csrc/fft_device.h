@@ -8,6 +8,9 @@
 // tw[t] = exp(-2 pi i t / n), t < n (conjugated for the inverse).
 #pragma once
 
+#include <algorithm>
+#include <initializer_list>
+
 #include "common.h"
 
 namespace eddy {
@@ -109,6 +112,15 @@ __device__ __forceinline__ void dft8(Cx<T>* v, T dir) {
     v[7] = {e[3].re - o3.re, e[3].im - o3.im};
 }
 
+template <int R, typename T>
+__device__ __forceinline__ void dft(Cx<T>* v, T dir) {
+    if constexpr (R == 2) dft2(v);
+    else if constexpr (R == 3) dft3(v, dir);
+    else if constexpr (R == 4) dft4(v, dir);
+    else if constexpr (R == 5) dft5(v, dir);
+    else dft8(v, dir);
+}
+
 // Exact quotient and remainder of small non-negative integers (x < 2^22, d >= 1) through a
 // float reciprocal rd = 1/d and one correction step: a few VALU ops instead of the ~25 of a
 // generic 32-bit division.
@@ -140,68 +152,86 @@ __device__ __forceinline__ void fft_sync() {
     }
 }
 
+// Butterflies of radix R that a thread holds in one pass: what fits 8 complex registers. With one
+// butterfly per thread whatever the radix, a tile was as narrow as its plan's smallest radix left it
+// (half-length 120 = 8 * 5 * 3: 8 pencils, 150 with a 2: 4), and rows of 64 or 32 bytes ran the
+// transforms at half the rate or less: along y at 256 x 128 cells per plane, forward and inverse, 240 2.04 ->
+// 3.38 and 2.29 -> 3.21 TB/s, 300 1.33 -> 2.90 and 1.56 -> 2.97, 180 1.62 -> 2.73 and 1.73 -> 2.45; along x2
+// alike (300 1.59 -> 3.00 both ways).
+__host__ __device__ constexpr int fft_hold(int R) { return R >= 5 ? 1 : 8 / R; }
+
+// One run-time pass of radix R over P sequences of length n = nb*R, span Ns (cfft_lds_ip).
+template <typename T, bool WAVE, int R>
+__device__ __forceinline__ void cfft_pass_rt(T* __restrict__ xr, T* __restrict__ xi, int ld, int P, int n, int Ns,
+                                             const T* twr, const T* twi, T dir, int tid, int nthr) {
+    constexpr int U = fft_hold(R);
+    const int nb = n / R, tstep = nb / Ns, tasks = P * nb;
+    const float rnb = 1.0f / (float)nb, rNs = 1.0f / (float)Ns;
+    Cx<T> v[U][R];
+    int orow[U], ob[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int t = tid + u * nthr;
+        if (t < tasks) {
+            int jj, k;
+            orow[u] = udiv_small(t, nb, rnb, jj) * ld;
+            const int blk = udiv_small(jj, Ns, rNs, k);
+            ob[u] = blk * Ns * R + k;
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const int o = orow[u] + pidx(jj + r * nb);
+                v[u][r] = {xr[o], xi[o]};
+            }
+            if (Ns > 1) {
+                int w = 0;
+#pragma unroll
+                for (int r = 1; r < R; ++r) {
+                    w += k * tstep;
+                    // table holds exp(-2 pi i t/n); forward (dir=-1) uses it as is, inverse conj
+                    v[u][r] = cmul(v[u][r], Cx<T>{twr[w], (dir < 0) ? twi[w] : -twi[w]});
+                }
+            }
+            dft<R>(v[u], dir);
+        }
+    }
+    fft_sync<WAVE>();
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        if (tid + u * nthr < tasks) {
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const int o = orow[u] + pidx(ob[u] + r * Ns);
+                xr[o] = v[u][r].re;
+                xi[o] = v[u][r].im;
+            }
+        }
+    }
+    fft_sync<WAVE>();
+}
+
 // In-place complex FFT of P sequences of length fp.n held in ONE buffer (split re/im, row
-// stride ld). Each radix pass: every thread loads at most one butterfly (up to 8 points, the
-// radix chosen at run time with predicated loads/stores so that all radices share the same
-// registers), the workgroup synchronises, then every thread stores. Needs
-// P * n / (smallest radix of the plan) <= nthr. The caller synchronises before (data
-// ready); the result is visible on return. WAVE: tid is the lane of the one wave that owns the P
-// sequences, nthr = 64.
+// stride ld). Each radix pass: every thread loads its butterflies (fft_hold of them at most: 8
+// complex values), the workgroup synchronises, then every thread stores. Needs
+// P * n <= R * fft_hold(R) * nthr for every radix R of the plan (fft_tile_ok). The caller
+// synchronises before (data ready); the result is visible on return. WAVE: tid is the lane of the
+// one wave that owns the P sequences, nthr = 64.
 template <typename T, bool WAVE = false>
 __device__ void cfft_lds_ip(T* __restrict__ xr, T* __restrict__ xi, int ld, int P, const FftPlan& fp,
                             const T* twr, const T* twi, T dir, int tid, int nthr) {
-    const int n = fp.n;
     int Ns = 1;
     for (int p = 0; p < fp.count; ++p) {
         const int R = fp.rad[p];
-        const int nb = n / R;
-        const int tstep = n / (Ns * R);
-        const bool active = tid < P * nb;
-        Cx<T> v[8];
-        int orow = 0, obase = 0;
-        if (active) {
-            int jj, k;
-            const int pen = udiv_small(tid, nb, 1.0f / (float)nb, jj);
-            const int blk = udiv_small(jj, Ns, 1.0f / (float)Ns, k);
-            const T* pr = xr + pen * ld;
-            const T* pi = xi + pen * ld;
-#pragma unroll
-            for (int r = 0; r < 8; ++r)
-                if (r < R) v[r] = {pr[pidx(jj + r * nb)], pi[pidx(jj + r * nb)]};
-            if (Ns > 1) {
-#pragma unroll
-                for (int r = 1; r < 8; ++r) {
-                    if (r < R) {
-                        const int t = k * r * tstep;
-                        // table holds exp(-2 pi i t/n); forward (dir=-1) uses it as is, inverse conj
-                        Cx<T> w = {twr[t], (dir < 0) ? twi[t] : -twi[t]};
-                        v[r] = cmul(v[r], w);
-                    }
-                }
-            }
-            switch (R) {
-                case 2: dft2(v); break;
-                case 3: dft3(v, dir); break;
-                case 4: dft4(v, dir); break;
-                case 5: dft5(v, dir); break;
-                default: dft8(v, dir); break;
-            }
-            orow = pen;
-            obase = blk * Ns * R + k;
+        // opaque: nothing of a pass is hoisted out of the loop over them, where the values of all
+        // radices would hold registers together
+        int t = tid;
+        asm volatile("" : "+v"(t));
+        switch (R) {
+            case 2: cfft_pass_rt<T, WAVE, 2>(xr, xi, ld, P, fp.n, Ns, twr, twi, dir, t, nthr); break;
+            case 3: cfft_pass_rt<T, WAVE, 3>(xr, xi, ld, P, fp.n, Ns, twr, twi, dir, t, nthr); break;
+            case 4: cfft_pass_rt<T, WAVE, 4>(xr, xi, ld, P, fp.n, Ns, twr, twi, dir, t, nthr); break;
+            case 5: cfft_pass_rt<T, WAVE, 5>(xr, xi, ld, P, fp.n, Ns, twr, twi, dir, t, nthr); break;
+            default: cfft_pass_rt<T, WAVE, 8>(xr, xi, ld, P, fp.n, Ns, twr, twi, dir, t, nthr); break;
         }
-        fft_sync<WAVE>();
-        if (active) {
-            T* qr = xr + orow * ld;
-            T* qi = xi + orow * ld;
-#pragma unroll
-            for (int r = 0; r < 8; ++r) {
-                if (r < R) {
-                    qr[pidx(obase + r * Ns)] = v[r].re;
-                    qi[pidx(obase + r * Ns)] = v[r].im;
-                }
-            }
-        }
-        fft_sync<WAVE>();
         Ns *= R;
     }
 }
@@ -215,57 +245,60 @@ __device__ void cfft_lds_ip(T* __restrict__ xr, T* __restrict__ xi, int ld, int 
 // base plus constant offsets: pidx(base + r*s) equals pidx(base) + r*s + (r*s >> 3) whenever
 // s % 8 == 0, or when base is a multiple of 8 and r*s < 8, so the offsets fold into the LDS
 // instructions. 768 x 384 x 256, whose x2 transforms have n = 192: 0.350 -> 0.289 ms forward and 0.367 ->
-// 0.296 inverse over the run-time passes; projections of 192 x 192 x 96 0.167 -> 0.149 ms. (Run-time
-// passes with a function per radix took 25 to 32 more registers and ran 10 % slower.)
+// 0.296 inverse over the run-time passes; projections of 192 x 192 x 96 0.167 -> 0.149 ms.
 __device__ __forceinline__ constexpr int poff(int x) { return x + (x >> 3); }
 
 template <typename T, bool WAVE, int n, int R, int Ns>
 __device__ __forceinline__ void cfft_pass_static(T* __restrict__ xr, T* __restrict__ xi, int ld, int P,
-                                                 const T* twr, const T* twi, T dir, int tid) {
+                                                 const T* twr, const T* twi, T dir, int tid, int nthr) {
     constexpr int nb = n / R;
     constexpr int tstep = n / (Ns * R);
     // loads at jj + r*nb: whole padding steps apart, or jj < nb <= 8 a power of two (no carry)
     constexpr bool lin_load = nb % 8 == 0 || 8 % nb == 0;
     // stores at blk*Ns*R + k + r*Ns, k < Ns
     constexpr bool lin_store = Ns % 8 == 0 || (8 % Ns == 0 && ((Ns * R) % 8 == 0 || 8 % (Ns * R) == 0));
-    const bool active = tid < P * nb;
-    Cx<T> v[R];
-    int orow = 0, ob = 0;
-    if (active) {
-        const int pen = tid / nb;  // constants: shifts and masks for powers of two
-        const int jj = tid - pen * nb;
-        const int blk = jj / Ns;
-        const int k = jj - blk * Ns;
-        orow = pen * ld;
-        const int ia = orow + pidx(jj);
+    // powers of two take one butterfly per thread: their tiles fill the workgroup so
+    constexpr int U = (n & (n - 1)) == 0 ? 1 : fft_hold(R);
+    Cx<T> v[U][R];
+    int orow[U], ob[U];
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const int o = lin_load ? ia + poff(r * nb) : orow + pidx(jj + r * nb);
-            v[r] = {xr[o], xi[o]};
-        }
-        if (Ns > 1) {
+    for (int u = 0; u < U; ++u) {
+        const int t = tid + u * nthr;
+        if (t < P * nb) {
+            const int pen = t / nb;  // constants: shifts and masks for powers of two
+            const int jj = t - pen * nb;
+            const int blk = jj / Ns;
+            const int k = jj - blk * Ns;
+            orow[u] = pen * ld;
+            const int ia = orow[u] + pidx(jj);
 #pragma unroll
-            for (int r = 1; r < R; ++r) {
-                const int t = k * (r * tstep);
-                // table holds exp(-2 pi i t/n); forward (dir=-1) uses it as is, inverse conj
-                Cx<T> w = {twr[t], (dir < 0) ? twi[t] : -twi[t]};
-                v[r] = cmul(v[r], w);
+            for (int r = 0; r < R; ++r) {
+                const int o = lin_load ? ia + poff(r * nb) : orow[u] + pidx(jj + r * nb);
+                v[u][r] = {xr[o], xi[o]};
             }
+            if (Ns > 1) {
+#pragma unroll
+                for (int r = 1; r < R; ++r) {
+                    const int w = k * (r * tstep);
+                    // table holds exp(-2 pi i t/n); forward (dir=-1) uses it as is, inverse conj
+                    v[u][r] = cmul(v[u][r], Cx<T>{twr[w], (dir < 0) ? twi[w] : -twi[w]});
+                }
+            }
+            dft<R>(v[u], dir);
+            ob[u] = blk * Ns * R + k;
         }
-        if constexpr (R == 2) dft2(v);
-        else if constexpr (R == 3) dft3(v, dir);
-        else if constexpr (R == 4) dft4(v, dir);
-        else dft8(v, dir);
-        ob = blk * Ns * R + k;
     }
     fft_sync<WAVE>();
-    if (active) {
-        const int oa = orow + pidx(ob);
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const int o = lin_store ? oa + poff(r * Ns) : orow + pidx(ob + r * Ns);
-            xr[o] = v[r].re;
-            xi[o] = v[r].im;
+    for (int u = 0; u < U; ++u) {
+        if (tid + u * nthr < P * nb) {
+            const int oa = orow[u] + pidx(ob[u]);
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const int o = lin_store ? oa + poff(r * Ns) : orow[u] + pidx(ob[u] + r * Ns);
+                xr[o] = v[u][r].re;
+                xi[o] = v[u][r].im;
+            }
         }
     }
     fft_sync<WAVE>();
@@ -273,39 +306,43 @@ __device__ __forceinline__ void cfft_pass_static(T* __restrict__ xr, T* __restri
 
 template <typename T, bool WAVE, int n, int Ns, int R, int... Rest>
 __device__ __forceinline__ void cfft_passes_static(T* xr, T* xi, int ld, int P, const T* twr, const T* twi, T dir,
-                                                   int tid) {
-    cfft_pass_static<T, WAVE, n, R, Ns>(xr, xi, ld, P, twr, twi, dir, tid);
-    if constexpr (sizeof...(Rest) > 0) cfft_passes_static<T, WAVE, n, Ns * R, Rest...>(xr, xi, ld, P, twr, twi, dir, tid);
+                                                   int tid, int nthr) {
+    cfft_pass_static<T, WAVE, n, R, Ns>(xr, xi, ld, P, twr, twi, dir, tid, nthr);
+    if constexpr (sizeof...(Rest) > 0) cfft_passes_static<T, WAVE, n, Ns * R, Rest...>(xr, xi, ld, P, twr, twi, dir, tid, nthr);
 }
 
-template <int... Rs>
-__device__ __forceinline__ bool plan_is(const FftPlan& fp) {
-    constexpr int rs[] = {Rs...};
-    if (fp.count != (int)sizeof...(Rs)) return false;
-#pragma unroll
-    for (int p = 0; p < (int)sizeof...(Rs); ++p)
-        if (fp.rad[p] != rs[p]) return false;
-    return true;
-}
-
-// cfft_lds_ip with the plans listed above (largest radix 8) taken by the compile-time passes; every other plan by the run-time passes. Same contract.
+// cfft_lds_ip with the plans listed above taken by the compile-time passes (fp.fixed, which the plan
+// sets), every other plan by the run-time passes. Same contract. One switch on the length: its compares
+// lie together, where a chain of tests would step over each body on the way to the next and wait for
+// its instructions (a small kernel is bound by that).
 template <typename T, bool WAVE = false>
 __device__ __forceinline__ void cfft_lds(T* __restrict__ xr, T* __restrict__ xi, int ld, int P, const FftPlan& fp,
                                          const T* twr, const T* twi, T dir, int tid, int nthr) {
-    if (fp.n == 128 && plan_is<8, 4, 4>(fp)) cfft_passes_static<T, WAVE, 128, 1, 8, 4, 4>(xr, xi, ld, P, twr, twi, dir, tid);
-    else if (fp.n == 64 && plan_is<8, 8>(fp)) cfft_passes_static<T, WAVE, 64, 1, 8, 8>(xr, xi, ld, P, twr, twi, dir, tid);
-    else if (fp.n == 256 && plan_is<8, 8, 4>(fp))
-        cfft_passes_static<T, WAVE, 256, 1, 8, 8, 4>(xr, xi, ld, P, twr, twi, dir, tid);
-    else if (fp.n == 512 && plan_is<8, 8, 8>(fp))
-        cfft_passes_static<T, WAVE, 512, 1, 8, 8, 8>(xr, xi, ld, P, twr, twi, dir, tid);
-    else if (fp.n == 32 && plan_is<8, 4>(fp)) cfft_passes_static<T, WAVE, 32, 1, 8, 4>(xr, xi, ld, P, twr, twi, dir, tid);
-    else if (fp.n == 192 && plan_is<8, 8, 3>(fp))
-        cfft_passes_static<T, WAVE, 192, 1, 8, 8, 3>(xr, xi, ld, P, twr, twi, dir, tid);
-    else if (fp.n == 96 && plan_is<8, 4, 3>(fp)) cfft_passes_static<T, WAVE, 96, 1, 8, 4, 3>(xr, xi, ld, P, twr, twi, dir, tid);
-    else if (fp.n == 48 && plan_is<4, 4, 3>(fp)) cfft_passes_static<T, WAVE, 48, 1, 4, 4, 3>(xr, xi, ld, P, twr, twi, dir, tid);
-    else if (fp.n == 24 && plan_is<8, 3>(fp)) cfft_passes_static<T, WAVE, 24, 1, 8, 3>(xr, xi, ld, P, twr, twi, dir, tid);
-    else if (fp.n == 16 && plan_is<4, 4>(fp)) cfft_passes_static<T, WAVE, 16, 1, 4, 4>(xr, xi, ld, P, twr, twi, dir, tid);
-    else cfft_lds_ip<T, WAVE>(xr, xi, ld, P, fp, twr, twi, dir, tid, nthr);
+    switch (fp.fixed) {
+        case 16: cfft_passes_static<T, WAVE, 16, 1, 4, 4>(xr, xi, ld, P, twr, twi, dir, tid, nthr); break;
+        case 24: cfft_passes_static<T, WAVE, 24, 1, 8, 3>(xr, xi, ld, P, twr, twi, dir, tid, nthr); break;
+        case 32: cfft_passes_static<T, WAVE, 32, 1, 8, 4>(xr, xi, ld, P, twr, twi, dir, tid, nthr); break;
+        case 48: cfft_passes_static<T, WAVE, 48, 1, 4, 4, 3>(xr, xi, ld, P, twr, twi, dir, tid, nthr); break;
+        case 64: cfft_passes_static<T, WAVE, 64, 1, 8, 8>(xr, xi, ld, P, twr, twi, dir, tid, nthr); break;
+        case 96: cfft_passes_static<T, WAVE, 96, 1, 8, 4, 3>(xr, xi, ld, P, twr, twi, dir, tid, nthr); break;
+        case 128: cfft_passes_static<T, WAVE, 128, 1, 8, 4, 4>(xr, xi, ld, P, twr, twi, dir, tid, nthr); break;
+        case 192: cfft_passes_static<T, WAVE, 192, 1, 8, 8, 3>(xr, xi, ld, P, twr, twi, dir, tid, nthr); break;
+        case 256: cfft_passes_static<T, WAVE, 256, 1, 8, 8, 4>(xr, xi, ld, P, twr, twi, dir, tid, nthr); break;
+        case 512: cfft_passes_static<T, WAVE, 512, 1, 8, 8, 8>(xr, xi, ld, P, twr, twi, dir, tid, nthr); break;
+        default: cfft_lds_ip<T, WAVE>(xr, xi, ld, P, fp, twr, twi, dir, tid, nthr);
+    }
+}
+
+// Whether the compile-time passes of cfft_lds take the plan: its length, else 0.
+inline int fixed_plan(const FftPlan& fp) {
+    auto is = [&](std::initializer_list<int> rad) {
+        return fp.count == (int)rad.size() && std::equal(rad.begin(), rad.end(), fp.rad);
+    };
+    const bool listed = (fp.n == 16 && is({4, 4})) || (fp.n == 24 && is({8, 3})) || (fp.n == 32 && is({8, 4})) ||
+                        (fp.n == 48 && is({4, 4, 3})) || (fp.n == 64 && is({8, 8})) || (fp.n == 96 && is({8, 4, 3})) ||
+                        (fp.n == 128 && is({8, 4, 4})) || (fp.n == 192 && is({8, 8, 3})) ||
+                        (fp.n == 256 && is({8, 8, 4})) || (fp.n == 512 && is({8, 8, 8}));
+    return listed ? fp.n : 0;
 }
 
 // Smallest radix of a plan (bounds the butterflies per pass of cfft_lds_ip).
@@ -315,9 +352,17 @@ __host__ __device__ inline int min_radix(const FftPlan& fp) {
     return fp.count ? r : 8;
 }
 
+// Whether nthr threads hold P sequences of the plan in one pass of each radix (powers of two at one
+// butterfly per thread: theirs are compile-time passes, whose 16 pencils need no more).
+inline bool fft_tile_ok(const FftPlan& fp, long P, int nthr) {
+    const bool pow2 = (fp.n & (fp.n - 1)) == 0;
+    for (int p = 0; p < fp.count; ++p)
+        if (P * fp.n > (long)fp.rad[p] * (pow2 ? 1 : fft_hold(fp.rad[p])) * nthr) return false;
+    return true;
+}
+
 // Workgroup size of the transform kernels: 512 threads hold 16 pencils of a length-256 real
-// transform at one butterfly per thread and pass, so every HBM row access of a tile covers a
-// full 128-byte line.
+// transform in one pass, so every HBM row access of a tile covers a full 128-byte line.
 constexpr int kFftThreads = 512;
 
 }  // namespace eddy
