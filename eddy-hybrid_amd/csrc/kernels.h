@@ -164,7 +164,7 @@ struct BatchProblem {
 
 // A prepared batched stage: the job array (device), its size, the item count and the LDS
 // bytes the stage kernel needs.
-constexpr int kMaxClasses = 12;  // kernel templates of a stage
+constexpr int kMaxClasses = 16;  // kernel templates of a stage
 struct StageLaunch {
     void* jobs = nullptr;
     int njobs = 0;

@@ -31,9 +31,10 @@
 namespace eddy {
 
 // One block of 256/P lines (logical line block `lb`), 64/P lines per wave.
-template <typename T, int QMAX, bool FIXED, bool CYC = false>
+template <typename T, int QMAX, int ROWS, bool CYC = false>
 __device__ __forceinline__ void xsolve_tile(const XArgs<T>& a, int lb) {
     extern __shared__ unsigned char smem_raw[];
+    constexpr bool FIXED = ROWS != XR_ANY, PADDED = ROWS == XR_PADDED;
     const Dims d = a.d;
     const int P = a.P, Q = FIXED ? QMAX : a.Q, M = d.M, N = d.N;
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
@@ -51,9 +52,22 @@ __device__ __forceinline__ void xsolve_tile(const XArgs<T>& a, int lb) {
     T* const blk = a.S + (size_t)line0 * (size_t)M;
     const int nel = nl * M;
     const int wi = lane + (lane >> 3);
+    // PADDED (LW <= 4): where element el of the wave's lines lies when each takes P*Q elements, so that a
+    // lane's rows are Q consecutive ones as in an exact split (slots past M hold no row of the line)
+    const int pad = P * Q - M;
+    auto place = [&](int el) {
+        int e = el;
+        if (LW > 1) e += el >= M ? pad : 0;
+        if (LW > 2) e += (el >= 2 * M ? pad : 0) + (el >= 3 * M ? pad : 0);
+        return e + (e >> 3);
+    };
     {
         T v[QMAX];
-        if (nel == 64 * QMAX) {  // wave-uniform
+        if (PADDED && nl == LW) {  // M > P (Q - 1): only the last round reaches past the lines
+#pragma unroll
+            for (int u = 0; u < QMAX - 1; ++u) v[u] = blk[lane + 64 * u];
+            v[QMAX - 1] = blk[min(lane + 64 * (QMAX - 1), nel - 1)];
+        } else if (nel == 64 * QMAX) {  // wave-uniform
 #pragma unroll
             for (int u = 0; u < QMAX; ++u) v[u] = blk[lane + 64 * u];
         } else {
@@ -63,7 +77,11 @@ __device__ __forceinline__ void xsolve_tile(const XArgs<T>& a, int lb) {
         }
 #pragma unroll
         for (int u = 0; u < QMAX; ++u)
-            if (FIXED || u < Q) tile[wi + 72 * u] = v[u];
+            if (PADDED) {
+                if (lane + 64 * u < nel) tile[place(lane + 64 * u)] = v[u];
+            } else if (FIXED || u < Q) {
+                tile[wi + 72 * u] = v[u];
+            }
     }
     // the wave's LDS operations complete in order; this only keeps the compiler from moving them
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -91,7 +109,7 @@ __device__ __forceinline__ void xsolve_tile(const XArgs<T>& a, int lb) {
     // the lane's rows: elements e0 + r of the wave's region
     const int e0 = FIXED ? lane * QMAX : lw * M + p * Q;
     auto at = [&](int r) { return e0 + r + ((e0 + r) >> 3); };
-    T part = xsolve_lines<T, QMAX, FIXED, CYC>(
+    T part = xsolve_lines<T, QMAX, ROWS, CYC>(
         a, p, lane, akj, lam, pin,
         [&](int r) { return tile[FIXED ? at(r) : min(at(r), xlds_wave(Q) - 1)]; },
         [&](int r, T x) {
@@ -105,7 +123,12 @@ __device__ __forceinline__ void xsolve_tile(const XArgs<T>& a, int lb) {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    if (nel == 64 * QMAX) {
+    if (PADDED) {
+#pragma unroll
+        for (int u = 0; u < QMAX; ++u)
+            if (lane + 64 * u < nel)
+                st_off(blk, (unsigned)sizeof(T) * (unsigned)(lane + 64 * u), tile[place(lane + 64 * u)]);
+    } else if (nel == 64 * QMAX) {
 #pragma unroll
         for (int u = 0; u < QMAX; ++u) blk[lane + 64 * u] = tile[wi + 72 * u];
     } else {
@@ -119,11 +142,11 @@ __device__ __forceinline__ void xsolve_tile(const XArgs<T>& a, int lb) {
 // sides: each then starts on what the pass before it left in the 256 MiB memory-side cache. At
 // 768 x 384 x 256 (a spectrum of 604 MB) this solve takes 0.284 ms instead of 0.310 and the inverse
 // x2 transform 0.369 instead of 0.387; nothing changes at 512 x 256 x 256 (268 MB) and below.
-template <typename T, int QMAX, bool FIXED, bool CYC>
+template <typename T, int QMAX, int ROWS, bool CYC>
 __global__ void __launch_bounds__(256)
-__attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 && FIXED ? (QMAX <= 8 ? 6 : 4) : 1)))
+__attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 && ROWS != XR_ANY ? (QMAX <= 8 ? 6 : 4) : 1)))
 k_xsolve(XArgs<T> a) {
-    xsolve_tile<T, QMAX, FIXED, CYC>(a, xcd_tile(gridDim.x - 1 - blockIdx.x, gridDim.x));
+    xsolve_tile<T, QMAX, ROWS, CYC>(a, xcd_tile(gridDim.x - 1 - blockIdx.x, gridDim.x));
 }
 
 // Pick P (threads per line, a power of two <= 64) and Q (rows per thread, 3 <= Q <= qmax):
@@ -171,14 +194,15 @@ int launch_xsolve(hipStream_t st, const Dims& d, const Tables<T>& tb, T* S, T* l
     const long nlines = a.lend - a.lbeg;
     dim3 grid((unsigned)((nlines + LPW - 1) / LPW));
     const size_t sh = 4 * (size_t)xlds_wave(Q) * sizeof(T);
-    xsolve_dispatch(xsolve_class(d.M, P, Q, cyc != 0), [&](auto qmax, auto fixed) {
+    xsolve_dispatch(xsolve_class(d.M, P, Q, cyc != 0), [&](auto qmax, auto rows) {
+        constexpr int ROWS = decltype(rows)::value;
         auto go = [&](auto fn) {
             (void)hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sh);
             hipLaunchKernelGGL(fn, grid, dim3(256), sh, st, a);
         };
-        if constexpr (decltype(fixed)::value) go(k_xsolve<T, decltype(qmax)::value, true, false>);
-        else if (cyc) go(k_xsolve<T, decltype(qmax)::value, false, true>);
-        else go(k_xsolve<T, decltype(qmax)::value, false, false>);
+        if constexpr (ROWS != XR_ANY) go(k_xsolve<T, decltype(qmax)::value, ROWS, false>);
+        else if (cyc) go(k_xsolve<T, decltype(qmax)::value, XR_ANY, true>);
+        else go(k_xsolve<T, decltype(qmax)::value, XR_ANY, false>);
     });
     return 0;
 }
@@ -188,11 +212,11 @@ int launch_xsolve(hipStream_t st, const Dims& d, const Tables<T>& tb, T* S, T* l
 // registers of the largest (QMAX = 32) for all problems.
 // Bounds where the unbounded kernel sits just above an occupancy step (8 rows: 86 VGPRs, 6 waves
 // per SIMD at 80; 16 rows: 148, 4 waves at 128).
-template <typename T, int QMAX, bool FIXED>
+template <typename T, int QMAX, int ROWS>
 __global__ void __launch_bounds__(256)
-__attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 && FIXED ? (QMAX <= 8 ? 6 : 4) : 1)))
+__attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 && ROWS != XR_ANY ? (QMAX <= 8 ? 6 : 4) : 1)))
 k_batch_xsolve(const Job<XArgs<T>>* jobs, int njobs, int total) {
-    run_item(jobs, njobs, total, [](const Job<XArgs<T>>& J, int t) { xsolve_tile<T, QMAX, FIXED>(J.a, t); });
+    run_item(jobs, njobs, total, [](const Job<XArgs<T>>& J, int t) { xsolve_tile<T, QMAX, ROWS>(J.a, t); });
 }
 
 template <typename T>
@@ -210,7 +234,7 @@ int prepare_xsolve(const std::vector<BatchProblem<T>>& pr, StageLaunch& out, std
     // grouped by template class (most rows first); the tiles of most LDS first, then the
     // longest x1 lines
     std::stable_sort(items.begin(), items.end(), [&](const Item& x, const Item& y) {
-        if (x.cls % kFixed != y.cls % kFixed) return x.cls % kFixed > y.cls % kFixed;
+        if (x.cls % kExact != y.cls % kExact) return x.cls % kExact > y.cls % kExact;
         if (x.cls != y.cls) return x.cls > y.cls;
         const int ox = lds_occupancy(lds_of(x)), oy = lds_occupancy(lds_of(y));
         return ox != oy ? ox < oy : pr[x.idx].d.M > pr[y.idx].d.M;
@@ -241,8 +265,8 @@ int prepare_xsolve(const std::vector<BatchProblem<T>>& pr, StageLaunch& out, std
 template <typename T>
 void batch_xsolve(hipStream_t st, const StageLaunch& sl) {
     for (int c = 0; c < sl.ncls; ++c) {
-        xsolve_dispatch(sl.cls_q[c], [&](auto qmax, auto fixed) {
-            auto fn = k_batch_xsolve<T, decltype(qmax)::value, decltype(fixed)::value>;
+        xsolve_dispatch(sl.cls_q[c], [&](auto qmax, auto rows) {
+            auto fn = k_batch_xsolve<T, decltype(qmax)::value, decltype(rows)::value>;
             const size_t lds = sl.cls_lds[c];
             (void)hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
             const int total = sl.cls_total[c];

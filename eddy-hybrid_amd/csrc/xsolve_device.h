@@ -59,17 +59,21 @@ __host__ __device__ inline int xlds_wave(int Q) { return 72 * Q + 2; }
 // two or three of the log2 P steps are left over.
 constexpr double kDecoupled = 0x1p-80;
 
-// Solve the wave's 64/P lines, P lanes and Q rows per lane (FIXED: Q = QMAX and M = P*Q, no row
-// checks). get(r) is the right-hand side of this lane's row r, put(r, x) takes its solution.
+// How a line-solve template takes its rows: any Q <= QMAX; Q = QMAX with lines that end in padding
+// (M <= P*Q); Q = QMAX and M = P*Q (no row checks).
+enum XRows { XR_ANY = 0, XR_PADDED = 1, XR_EXACT = 2 };
+
+// Solve the wave's 64/P lines, P lanes and Q rows per lane. get(r) is the right-hand side of this lane's row r, put(r, x) takes its solution.
 // Returns the sum of the lane's solution rows. CYC: periodic lines, solved as the tridiagonal
 // part T' plus a rank-one correction (Sherman-Morrison, the method of the reference's CYCLIC,
 // numrec.f:754-781): T = T' + u v^T with u = (g, 0, ..., 0, alpha), v = (1, 0, ..., 0, beta/g),
 // g = -b(0); the elimination carries the second right-hand side u beside d, and
 // x = y - z (y_0 + beta y_{M-1}/g) / (1 + z_0 + beta z_{M-1}/g). The singular line is pinned at
 // x(0) = 0 and solved without the correction (its corner couplings act on x(0) = 0).
-template <typename T, int QMAX, bool FIXED, bool CYC, typename Get, typename Put>
+template <typename T, int QMAX, int ROWS, bool CYC, typename Get, typename Put>
 __device__ __forceinline__ T xsolve_lines(const XArgs<T>& a, int p, int lane, T akj, T lam, bool pin, Get get,
                                           Put put) {
+    constexpr bool FIXED = ROWS != XR_ANY;
     const int P = a.P, Q = FIXED ? QMAX : a.Q, M = a.d.M;
     // periodic line: the corrected diagonals of rows 0 and M-1 and the second right-hand side
     const bool cyc = CYC && !pin;
@@ -99,7 +103,7 @@ __device__ __forceinline__ T xsolve_lines(const XArgs<T>& a, int p, int lane, T 
             const int r = r0 + u;
             if (!FIXED && r >= Q) continue;
             T av = ta[u], cv = tc[u], bv = tb[u] - akj * tr[u] + lam;
-            T dv = (FIXED || ib + r < M) ? td[u] : T(0);
+            T dv = (ROWS == XR_EXACT || ib + r < M) ? td[u] : T(0);
             if (r == 0) {  // the singular line: x(0) = 0
                 const bool z = pin && p == 0;
                 av = z ? T(0) : av;
@@ -238,27 +242,43 @@ __device__ __forceinline__ T xsolve_lines(const XArgs<T>& a, int p, int lane, T 
 }
 
 // Kernel template of a line length: the exact splits M = P*Q with Q of the usual grids have their
-// own (kFixed + Q: no row checks, constant LDS offsets), every other split runs the smallest
-// template of at least Q rows.
-constexpr int kFixed = 64;
+// own (kExact + Q: no row checks), as have the other splits into 7 to 12 rows (all that the default
+// partition makes of M > 96; kPadded + Q: constant loops, the lines staged at P*Q elements each so that LDS
+// offsets are constant too); every other split runs the smallest template of at least Q rows. At
+// 128 x 128 lines, against the next larger of 8 or 16 rows with its row checks: 300 rows 2.27 -> 2.87 TB/s,
+// 350 2.62 -> 3.21, 528 2.45 -> 3.29, 576 2.58 -> 3.60, 700 3.04 -> 3.84, 200 2.31 -> 2.44, 450 3.10 -> 3.19. P < 16
+// (M <= 96) has 8 lines and more to a wave, whose staging would look their bounds up one by one.
+constexpr int kExact = 64, kPadded = 128;
 inline int xsolve_class(int M, int P, int Q, bool cyc) {
-    if (!cyc && P * Q == M && (Q == 6 || Q == 8 || Q == 10 || Q == 12 || Q == 16)) return kFixed + Q;
+    if (!cyc && P * Q == M && (Q == 6 || Q == 8 || Q == 10 || Q == 12 || Q == 16)) return kExact + Q;
+    if (!cyc && P >= 16 && Q >= 7 && Q <= 12) return kPadded + Q;
     return Q <= 4 ? 4 : (Q <= 8 ? 8 : (Q <= 16 ? 16 : 32));
 }
 
-// go(integral QMAX, FIXED) of a class
+template <int QMAX, int ROWS, typename Go>
+void xsolve_go(Go go) {
+    go(std::integral_constant<int, QMAX>{}, std::integral_constant<int, ROWS>{});
+}
+
+// go(integral QMAX, integral XRows) of a class
 template <typename Go>
 void xsolve_dispatch(int cls, Go go) {
     switch (cls) {
-        case kFixed + 6: go(std::integral_constant<int, 6>{}, std::true_type{}); break;
-        case kFixed + 8: go(std::integral_constant<int, 8>{}, std::true_type{}); break;
-        case kFixed + 10: go(std::integral_constant<int, 10>{}, std::true_type{}); break;
-        case kFixed + 12: go(std::integral_constant<int, 12>{}, std::true_type{}); break;
-        case kFixed + 16: go(std::integral_constant<int, 16>{}, std::true_type{}); break;
-        case 4: go(std::integral_constant<int, 4>{}, std::false_type{}); break;
-        case 8: go(std::integral_constant<int, 8>{}, std::false_type{}); break;
-        case 16: go(std::integral_constant<int, 16>{}, std::false_type{}); break;
-        default: go(std::integral_constant<int, 32>{}, std::false_type{}); break;
+        case kExact + 6: xsolve_go<6, XR_EXACT>(go); break;
+        case kExact + 8: xsolve_go<8, XR_EXACT>(go); break;
+        case kExact + 10: xsolve_go<10, XR_EXACT>(go); break;
+        case kExact + 12: xsolve_go<12, XR_EXACT>(go); break;
+        case kExact + 16: xsolve_go<16, XR_EXACT>(go); break;
+        case kPadded + 7: xsolve_go<7, XR_PADDED>(go); break;
+        case kPadded + 8: xsolve_go<8, XR_PADDED>(go); break;
+        case kPadded + 9: xsolve_go<9, XR_PADDED>(go); break;
+        case kPadded + 10: xsolve_go<10, XR_PADDED>(go); break;
+        case kPadded + 11: xsolve_go<11, XR_PADDED>(go); break;
+        case kPadded + 12: xsolve_go<12, XR_PADDED>(go); break;
+        case 4: xsolve_go<4, XR_ANY>(go); break;
+        case 8: xsolve_go<8, XR_ANY>(go); break;
+        case 16: xsolve_go<16, XR_ANY>(go); break;
+        default: xsolve_go<32, XR_ANY>(go); break;
     }
 }
 

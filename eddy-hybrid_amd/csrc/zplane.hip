@@ -50,10 +50,10 @@ __device__ __forceinline__ int opaque(int lane) {
 
 // The line solves of the plane; at(m, i) is the LDS element of x2 mode m and x1 row i. The line
 // sums go to lsum when it is not null.
-template <typename T, int QMAX, bool FIXED, typename At>
+template <typename T, int QMAX, int ROWS, typename At>
 __device__ __forceinline__ void plane_solve(const XArgs<T>& x, int j, T* lsum, At at) {
     const int w = threadIdx.x >> 6, nw = blockDim.x >> 6;
-    const int P = x.P, Q = FIXED ? QMAX : x.Q, LW = 64 / P, N = x.d.N;
+    const int P = x.P, Q = ROWS != XR_ANY ? QMAX : x.Q, LW = 64 / P, N = x.d.N;
     const T akj = x.tb.akj[j];
     for (int b = __builtin_amdgcn_readfirstlane(w); b * LW < N; b += nw) {
         const int lane = opaque(threadIdx.x & 63);
@@ -61,11 +61,11 @@ __device__ __forceinline__ void plane_solve(const XArgs<T>& x, int j, T* lsum, A
         const int m = min(b * LW + lw, N - 1);
         const bool own = b * LW + lw < N;
         const T lam = x.tb.lam[m];
-        T part = xsolve_lines<T, QMAX, FIXED, false>(
+        T part = xsolve_lines<T, QMAX, ROWS, false>(
             x, p, lane, akj, lam, j == 0 && m == x.d.null_m,
-            [&](int r) { return at(m, FIXED ? p * Q + r : min(p * Q + r, x.d.M - 1)); },
+            [&](int r) { return at(m, ROWS == XR_EXACT ? p * Q + r : min(p * Q + r, x.d.M - 1)); },
             [&](int r, T v) {
-                if (own && (FIXED || p * Q + r < x.d.M)) at(m, p * Q + r) = v;
+                if (own && (ROWS == XR_EXACT || p * Q + r < x.d.M)) at(m, p * Q + r) = v;
             });
         if (lsum) {
             for (int off = P >> 1; off > 0; off >>= 1) part += __shfl_xor(part, off, 64);
@@ -88,7 +88,7 @@ __device__ __forceinline__ T plane_delta(const XArgs<T>& x, const T* lsum, doubl
     return T(-tot / ((double)x.tb.wsum[x.d.null_m] * (double)x.d.M));
 }
 
-template <typename T, int QMAX, bool FIXED>
+template <typename T, int QMAX, int ROWS>
 __global__ void __launch_bounds__(kPlaneThreads) k_zplane_dct(PlaneArgs<T> a) {
     extern __shared__ __align__(16) unsigned char plane_lds[];
     __shared__ double scratch[16];
@@ -171,7 +171,7 @@ __global__ void __launch_bounds__(kPlaneThreads) k_zplane_dct(PlaneArgs<T> a) {
     }
     __syncthreads();
 
-    plane_solve<T, QMAX, FIXED>(a.x, j, j == 0 ? lsum : nullptr, [&](int m, int i) -> T& {
+    plane_solve<T, QMAX, ROWS>(a.x, j, j == 0 ? lsum : nullptr, [&](int m, int i) -> T& {
         return m < H ? Ar[i * ld + pidx(m)] : Ai[i * ld + (m == H ? 0 : pidx(N - m))];
     });
     __syncthreads();
@@ -262,7 +262,7 @@ __device__ __forceinline__ void dense_block(const T* __restrict__ A, int N, int 
     }
 }
 
-template <typename T, int QMAX, bool FIXED>
+template <typename T, int QMAX, int ROWS>
 __global__ void __launch_bounds__(kPlaneThreads) k_zplane_dense(PlaneArgs<T> a) {
     extern __shared__ __align__(16) unsigned char plane_lds[];
     __shared__ double scratch[16];
@@ -295,7 +295,7 @@ __global__ void __launch_bounds__(kPlaneThreads) k_zplane_dense(PlaneArgs<T> a) 
                 }
     }
     __syncthreads();
-    plane_solve<T, QMAX, FIXED>(a.x, j, j == 0 ? lsum : nullptr, [&](int m, int i) -> T& { return Y[m * ld + i]; });
+    plane_solve<T, QMAX, ROWS>(a.x, j, j == 0 ? lsum : nullptr, [&](int m, int i) -> T& { return Y[m * ld + i]; });
     __syncthreads();
     T delta = T(0);
     if (j == 0) delta = plane_delta(a.x, lsum, scratch);
@@ -366,15 +366,15 @@ void launch_zplane(hipStream_t st, const Dims& d, const FftPlan& fpz, const Tabl
     // 512 threads for the small planes (64 x 64 x 32: 0.0353 ms, 0.0360 with 1024)
     const int nthr = d.M * d.N <= 6144 ? 512 : kPlaneThreads;
     a.pw = dense ? 1 : std::max(1, 64 / std::max(1, fpz.n / min_radix(fpz)));
-    xsolve_dispatch(xsolve_class(d.M, a.x.P, a.x.Q, false), [&](auto qmax, auto fixed) {
+    xsolve_dispatch(xsolve_class(d.M, a.x.P, a.x.Q, false), [&](auto qmax, auto rows) {
         constexpr int QMAX = decltype(qmax)::value;
         if constexpr (QMAX <= 16) {
             auto go = [&](auto fn) {
                 (void)hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
                 hipLaunchKernelGGL(fn, dim3(nj), dim3(nthr), lds, st, a);
             };
-            if (dense) go(k_zplane_dense<T, QMAX, decltype(fixed)::value>);
-            else go(k_zplane_dct<T, QMAX, decltype(fixed)::value>);
+            if (dense) go(k_zplane_dense<T, QMAX, decltype(rows)::value>);
+            else go(k_zplane_dct<T, QMAX, decltype(rows)::value>);
         }
     });
 }
