@@ -72,6 +72,7 @@ struct MmArgs {
     int lda, ldb, ldc;
     int R, Cn, P, nb;
     int ntr, ntc;     // tiles along r and along c
+    int flat;         // k_mma64: a workgroup's waves take consecutive tiles of a batch (else of a column)
     int zb;           // batch of the zero y-mode (-1: not in this launch)
     // forward: operand A of the zero mode minus shiftL times this mean
     MeanShift shift;
@@ -684,8 +685,21 @@ k_mma64(MmArgs<double> a) {
     const int tid = threadIdx.x, nthr = blockDim.x;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int tile = xcd_tile(blockIdx.x, gridDim.x);
-    const int ct = tile % a.ntc, rest = tile / a.ntc;
-    const int b = rest / a.ntr, rt = (rest - b * a.ntr) * (nthr >> 6) + wv;
+    const int nt = a.ntr * a.ntc;  // flat: wave tiles of a batch; else its workgroups
+    int b, rt, ct;
+    if (a.flat) {
+        const int nwg = (nt + 3) >> 2;
+        b = tile / nwg;
+        const int t = 4 * (tile - b * nwg) + wv;
+        rt = t / a.ntc;  // past the last row tile: nothing to do
+        ct = t - rt * a.ntc;
+    } else {
+        b = tile / nt;
+        const int t = tile - b * nt;
+        rt = t / a.ntc;
+        ct = t - rt * a.ntc;
+        rt = rt * (nthr >> 6) + wv;
+    }
     const int r0 = rt * 16 * NR, c0 = ct * 16 * NC;
     const double* A = a.A + (size_t)b * a.sA;
     const double* B = a.B + (size_t)b * a.sB;
@@ -717,10 +731,25 @@ k_mma64(MmArgs<double> a) {
 template <bool PM, int NR, int NC>
 static void launch_mma64_tiles(hipStream_t st, MmArgs<double> a) {
     const int wr = ceil_div(a.R, 16 * NR);  // wave tiles along r
+    a.ntc = ceil_div(a.Cn, 16 * NC);
+    const long tiles = (long)wr * a.ntc * a.nb, rounds = (tiles + 1023) / 1024;
+    const long nwg = (long)ceil_div(wr * a.ntc, 4) * a.nb;
+    // Row tiles that four waves do not divide left workgroups of one or two waves, which spread unevenly
+    // over the SIMDs: with the last of several rounds of waves a fifth full or more, a third one landed on
+    // SIMDs that should run two (a pair of products: 220 x 260 x 48 0.084 -> 0.074 ms, 170 x 250 x 56 0.066 ->
+    // 0.060, 144 x 246 x 50 0.0504 -> 0.0457, 395 x 161 x 24 0.0488 -> 0.0445, 160 x 160 x 64 0.0435 -> 0.0419). Not where
+    // filling up to four adds a round (150 x 150 x 150 0.072 -> 0.076) or the last is nearly empty
+    // (200 x 200 x 64 0.0743 -> 0.0766) or the first not full (128 x 179 x 10 0.0253 -> 0.0265).
+    if (wr % 4 && rounds > 1 && 10 * tiles >= 1024 * (10 * rounds - 8) && 4 * nwg <= 1024 * rounds) {
+        a.flat = 1;
+        a.ntr = wr;
+        hipLaunchKernelGGL((k_mma64<PM, NR, NC>), dim3((unsigned)nwg), dim3(256), 0, st, a);
+        return;
+    }
     // waves of a workgroup: consecutive row tiles, as many as divide them evenly
     const int nw = wr % 4 == 0 ? 4 : (wr % 2 == 0 ? 2 : 1);
+    a.flat = 0;
     a.ntr = wr / nw;
-    a.ntc = ceil_div(a.Cn, 16 * NC);
     hipLaunchKernelGGL((k_mma64<PM, NR, NC>), dim3((unsigned)((long)a.ntr * a.ntc * a.nb)), dim3(64 * nw), 0, st, a);
 }
 
