@@ -44,7 +44,7 @@ enum YfftFwdMode { YF_DIRECT = 0, YF_RESIDUAL = 1, YF_DIVERGENCE = 2 };
 
 // What the forward y-FFT reads: YF_DIRECT the RHS in src (minus the solvability shift
 // red[RED_VOLB]/red[RED_VOL] when shift != 0); YF_RESIDUAL r = (src - that shift when
-// shift != 0) - L(phi) in FP64 (src is the RHS; sum r^2 -> red[RED_RNORM2]); YF_DIVERGENCE
+// shift != 0) - L(phi) in FP64 (src is the RHS); YF_DIVERGENCE
 // b = DIV(us, vs, ws) * scale formed on the fly (sum vol*b -> red[RED_VOLB], sum vol ->
 // red[RED_VOL]; the solvability shift is then applied to the zero y-mode by the x2 transform;
 // the FP32 transform also stores b in FP64 at rhs_out, the RHS of the defect correction).
@@ -79,7 +79,7 @@ void launch_yfft_fwd(hipStream_t st, const Dims& d, const FftPlan& fp, const Tab
 // red[RED_PHISUM]; YI_UPDATE adds into phi's interior and adds sum(new phi).
 template <typename T>
 void launch_yfft_inv(hipStream_t st, const Dims& d, const FftPlan& fp, const Tables<T>& tb,
-                     const T* S, double* dp, const Reduce& rd, int TI, int mode);
+                     const T* S, double* dp, const Reduce& rd, int TI, int mode, bool fold = true);
 
 // The y real DFT as FP32 matrix-core products (ygemm.hip), for L % 16 == 0, L <= 512:
 // forward from the YF_DIRECT / YF_RESIDUAL input into S, inverse (YI_STORE / YI_UPDATE)
@@ -88,7 +88,7 @@ bool ygemm_supported(const Dims& d);
 void launch_ygemm_fwd(hipStream_t st, const Dims& d, const float* FT, const FwdInput& in, const Op64& op,
                       const Reduce& rd, float* S);
 void launch_ygemm_inv(hipStream_t st, const Dims& d, const float* GT, const float* S, double* dp, const Reduce& rd,
-                      int mode);
+                      int mode, bool fold);
 
 // Forward x2 transform (DCT-II when uniform, dense eigenvectors otherwise), in place on S.
 // The zero y-mode first loses L times the mean `shift` (the volume-weighted solvability shift of
@@ -264,7 +264,8 @@ void batch_fold(hipStream_t st, const FoldJob* jobs, int njobs);
 
 // Stencils (FP64).
 int reduce_blocks(const Dims& d);
-void launch_fold(hipStream_t st, const double* part, int n, double* out);
+// out[b] = sum of part[b*n .. b*n + n), b < count; next != 0 (count 1): out[1] = next
+void launch_fold(hipStream_t st, const double* part, int n, double* out, int count = 1, double next = 0.0);
 // red[RED_CHK_VB] = sum vol*b, red[RED_CHK_VABS] = sum vol*|b| over the finite interior values
 // of b, red[RED_CHK_NF] = the count of non-finite ones.
 void launch_rhs_check(hipStream_t st, const Dims& d, const Metrics& mt, const double* b, const Reduce& rd);

@@ -436,8 +436,10 @@ __global__ void k_fill(double* p, size_t n, double v) {
     if (t < n) p[t] = v;
 }
 
-// out[0] = the sum of part[0..n), one workgroup of 1024 threads.
-__global__ void __launch_bounds__(1024) k_fold(const double* __restrict__ part, int n, double* out) {
+// out[b] = the sum of part[b*n .. b*n + n) for workgroup b of 1024 threads; out[1] = next where next is
+// not 0 (one workgroup).
+__global__ void __launch_bounds__(1024) k_fold(const double* __restrict__ part, int n, double* out, double next) {
+    part += (size_t)blockIdx.x * n;
     double v = 0.0;
 #pragma unroll 8
     for (int t = threadIdx.x; t < n; t += 1024) v += part[t];
@@ -448,7 +450,8 @@ __global__ void __launch_bounds__(1024) k_fold(const double* __restrict__ part, 
     if (threadIdx.x == 0) {
         double s = w[0];
         for (int q = 1; q < 16; ++q) s += w[q];
-        *out = s;
+        out[blockIdx.x] = s;
+        if (next != 0.0) out[1] = next;
     }
 }
 
@@ -624,8 +627,8 @@ void batch_fold(hipStream_t st, const FoldJob* jobs, int njobs) {
     if (njobs > 0) hipLaunchKernelGGL(k_batch_fold, dim3(njobs), dim3(1024), 0, st, jobs);
 }
 
-void launch_fold(hipStream_t st, const double* part, int n, double* out) {
-    hipLaunchKernelGGL(k_fold, dim3(1), dim3(1024), 0, st, part, n, out);
+void launch_fold(hipStream_t st, const double* part, int n, double* out, int count, double next) {
+    hipLaunchKernelGGL(k_fold, dim3(count), dim3(1024), 0, st, part, n, out, next);
 }
 
 void launch_divergence(hipStream_t st, const Dims& d, const Metrics& mt, const double* us, const double* vs,
@@ -635,8 +638,7 @@ void launch_divergence(hipStream_t st, const Dims& d, const Metrics& mt, const d
                        accumulate_compat, dscale);
     if (accumulate_compat) {
         const int nb = reduce_blocks(d);
-        launch_fold(st, rd.part, nb, rd.red + RED_VOLB);
-        launch_fill(st, rd.red + RED_VOL, 1, mt.vol_total);
+        launch_fold(st, rd.part, nb, rd.red + RED_VOLB, 1, mt.vol_total);
     }
 }
 
@@ -679,9 +681,7 @@ void launch_finalize(hipStream_t st, const Dims& d, const Op64& op, double* phi,
 void launch_rhs_check(hipStream_t st, const Dims& d, const Metrics& mt, const double* b, const Reduce& rd) {
     const int nb = reduce_blocks(d);
     hipLaunchKernelGGL(k_rhs_check, red_grid(d), kCellBlock, 0, st, d, mt, b, rd.part, nb);
-    launch_fold(st, rd.part, nb, rd.red + RED_CHK_VB);
-    launch_fold(st, rd.part + nb, nb, rd.red + RED_CHK_VABS);
-    launch_fold(st, rd.part + 2 * nb, nb, rd.red + RED_CHK_NF);
+    launch_fold(st, rd.part, nb, rd.red + RED_CHK_VB, 3);  // RED_CHK_VB, RED_CHK_VABS, RED_CHK_NF
 }
 
 void launch_sumsq(hipStream_t st, const Dims& d, const double* a, const Reduce& rd, int slot) {

@@ -138,13 +138,13 @@ __device__ __forceinline__ void divergence_rows(const Dims& d, const Metrics& mt
     }
 }
 
-// B cells of the residual r = src - L(phi) (lap_at's arithmetic), sum r^2 into rsum; loads
-// first, as in divergence_rows. The x and x2 neighbours at the walls are ghosts (in range)
+// B cells of the residual r = src - L(phi) (lap_at's arithmetic); loads first, as in
+// divergence_rows. The x and x2 neighbours at the walls are ghosts (in range)
 // whose terms are dropped, as lap_at drops them.
 template <int B>
 __device__ __forceinline__ void residual_rows(const Dims& d, const Op64& op, const double* __restrict__ src,
                                               const double* __restrict__ phi, int gi, bool iok, int j0, int jstep,
-                                              int k, double* v, double& rsum, double shift) {
+                                              int k, double* v, double shift) {
     const int I = gi + 1, K = k + 1;
     // 32-bit byte offsets from the field bases (fields below 4 GiB); a neighbour step is added
     // modulo 2^32, so a negative step is its two's complement. Across a wall the neighbour is
@@ -189,7 +189,6 @@ __device__ __forceinline__ void residual_rows(const Dims& d, const Op64& op, con
         if (zhi) sz += cn * pzp[u];
         const bool ok = iok && j0 + u * jstep < d.L;
         v[u] = ok ? (s[u] - shift) - (sx + sy + sz) : 0.0;
-        rsum += v[u] * v[u];
     }
 }
 
@@ -322,7 +321,7 @@ __device__ __forceinline__ void yfft_fwd_tile(const YArgs<T>& a, int tile, int n
             for (int h = 0; h < kLoadBatch / kDivRows; ++h) {  // sub-batches as for the divergence below
                 const int jh = j0 + h * kDivRows * jstep;
                 double v[kDivRows];
-                residual_rows<kDivRows>(d, a.op, a.src, a.phi, gi, iok, jh, jstep, k, v, rsq, shift);
+                residual_rows<kDivRows>(d, a.op, a.src, a.phi, gi, iok, jh, jstep, k, v, shift);
 #pragma unroll
                 for (int r = 0; r < kDivRows; ++r) put(v[r], jh + r * jstep);
                 __builtin_amdgcn_sched_barrier(0);
@@ -361,7 +360,6 @@ __device__ __forceinline__ void yfft_fwd_tile(const YArgs<T>& a, int tile, int n
             }
         }
     }
-    if (MODE == YF_RESIDUAL) block_partial<RED_OP_SUM>(rsq, a.part, slot);
     if (MODE == YF_DIVERGENCE || MODE == YF_DIV_CART || MODE == YF_DIV_CYL)
         block_partial<RED_OP_SUM>(rsq, a.part, slot);
     __syncthreads();
@@ -722,22 +720,20 @@ void launch_yfft_fwd(hipStream_t st, const Dims& d, const FftPlan& fp, const Tab
             else go(k_yfft_fwd<T, YF_DIV_CYL, false>);
         }
         if (in.fold) {
-            launch_fold(st, rd.part, (int)(grid.x * grid.y), rd.red + RED_VOLB);
-            launch_fill(st, rd.red + RED_VOL, 1, in.mt.vol_total);
+            launch_fold(st, rd.part, (int)(grid.x * grid.y), rd.red + RED_VOLB, 1, in.mt.vol_total);
         }
     } else {
         if (dense) go(k_yfft_fwd<T, YF_RESIDUAL, true>);
         else go(k_yfft_fwd<T, YF_RESIDUAL, false>);
-        launch_fold(st, rd.part, (int)(grid.x * grid.y), rd.red + RED_RNORM2);
     }
 }
 
 template <typename T>
 void launch_yfft_inv(hipStream_t st, const Dims& d, const FftPlan& fp, const Tables<T>& tb,
-                     const T* S, double* dp, const Reduce& rd, int TI, int mode) {
+                     const T* S, double* dp, const Reduce& rd, int TI, int mode, bool fold) {
     if constexpr (std::is_same<T, float>::value) {
         if (tb.ydft_b && (mode == YI_STORE || mode == YI_UPDATE)) {
-            launch_ygemm_inv(st, d, tb.ydft_b, S, dp, rd, mode);
+            launch_ygemm_inv(st, d, tb.ydft_b, S, dp, rd, mode, fold);
             return;
         }
     }
@@ -767,7 +763,7 @@ void launch_yfft_inv(hipStream_t st, const Dims& d, const FftPlan& fp, const Tab
         case YI_STORE:
             if (dense) go(k_yfft_inv<T, YI_STORE, true>);
             else go(k_yfft_inv<T, YI_STORE, false>);
-            launch_fold(st, rd.part, (int)(grid.x * grid.y), rd.red + RED_PHISUM);
+            if (fold) launch_fold(st, rd.part, (int)(grid.x * grid.y), rd.red + RED_PHISUM);
             break;
         case YI_UPDATE_FINAL:
             if (dense) go(k_yfft_inv<T, YI_UPDATE_FINAL, true>);
@@ -776,7 +772,7 @@ void launch_yfft_inv(hipStream_t st, const Dims& d, const FftPlan& fp, const Tab
         default:
             if (dense) go(k_yfft_inv<T, YI_UPDATE, true>);
             else go(k_yfft_inv<T, YI_UPDATE, false>);
-            launch_fold(st, rd.part, (int)(grid.x * grid.y), rd.red + RED_PHISUM);
+            if (fold) launch_fold(st, rd.part, (int)(grid.x * grid.y), rd.red + RED_PHISUM);
             break;
     }
 }
@@ -906,8 +902,8 @@ template void launch_yfft_fwd<double>(hipStream_t, const Dims&, const FftPlan&, 
 template void launch_yfft_fwd<float>(hipStream_t, const Dims&, const FftPlan&, const Tables<float>&,
                                      const FwdInput&, const Op64&, const Reduce&, float*, int, int);
 template void launch_yfft_inv<double>(hipStream_t, const Dims&, const FftPlan&, const Tables<double>&,
-                                      const double*, double*, const Reduce&, int, int);
+                                      const double*, double*, const Reduce&, int, int, bool);
 template void launch_yfft_inv<float>(hipStream_t, const Dims&, const FftPlan&, const Tables<float>&,
-                                     const float*, double*, const Reduce&, int, int);
+                                     const float*, double*, const Reduce&, int, int, bool);
 
 }  // namespace eddy

@@ -84,7 +84,6 @@ __global__ void __launch_bounds__(256) k_ygemm_fwd(GArgs a) {
     const int tid = threadIdx.x;
     double shift = 0.0;
     if (a.shift) shift = a.red[RED_VOLB] / a.red[RED_VOL];
-    double rsq = 0.0;
     const int total = kGemmPencils * L;
     constexpr int U = 8;
     for (int e0 = tid; e0 < total; e0 += 256 * U) {
@@ -101,7 +100,6 @@ __global__ void __launch_bounds__(256) k_ygemm_fwd(GArgs a) {
                     v[u] = a.src[sidx(d, gi + 1, j + 1, k + 1)] - shift;
                 } else {
                     v[u] = (a.src[sidx(d, gi + 1, j + 1, k + 1)] - shift) - lap_at(d, a.op, a.phi, gi, j, k);
-                    rsq += v[u] * v[u];
                 }
             }
         }
@@ -111,7 +109,6 @@ __global__ void __launch_bounds__(256) k_ygemm_fwd(GArgs a) {
             if (e < total) X[e] = (float)v[u];
         }
     }
-    if (MODE == YF_RESIDUAL) block_partial<RED_OP_SUM>(rsq, a.part, linear_bid());
     __syncthreads();
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform: scalar branches
@@ -219,14 +216,13 @@ void launch_ygemm_fwd(hipStream_t st, const Dims& d, const float* FT, const FwdI
     const size_t sh = (size_t)d.L * kGemmPencils * sizeof(float);
     if (in.mode == YF_RESIDUAL) {
         hipLaunchKernelGGL(k_ygemm_fwd<YF_RESIDUAL>, grid, dim3(256), sh, st, a);
-        launch_fold(st, rd.part, (int)(grid.x * grid.y), rd.red + RED_RNORM2);
     } else {
         hipLaunchKernelGGL(k_ygemm_fwd<YF_DIRECT>, grid, dim3(256), sh, st, a);
     }
 }
 
 void launch_ygemm_inv(hipStream_t st, const Dims& d, const float* GT, const float* S, double* dp, const Reduce& rd,
-                      int mode) {
+                      int mode, bool fold) {
     GArgs a{};
     a.part = rd.part;
     a.red = rd.red;
@@ -238,7 +234,7 @@ void launch_ygemm_inv(hipStream_t st, const Dims& d, const float* GT, const floa
     const size_t sh = (size_t)d.L * kGemmPencils * sizeof(float);
     if (mode == YI_STORE) hipLaunchKernelGGL(k_ygemm_inv<YI_STORE>, grid, dim3(256), sh, st, a);
     else hipLaunchKernelGGL(k_ygemm_inv<YI_UPDATE>, grid, dim3(256), sh, st, a);
-    launch_fold(st, rd.part, (int)(grid.x * grid.y), rd.red + RED_PHISUM);
+    if (fold) launch_fold(st, rd.part, (int)(grid.x * grid.y), rd.red + RED_PHISUM);
 }
 
 }  // namespace eddy
