@@ -81,13 +81,14 @@ int eddy_direct_release(void);
  * Plans (explicit form of the SAVEd state of direct.f:121-585).
  * ------------------------------------------------------------------------------------- */
 typedef struct {
-    /* Zero fields take the defaults. The plan lowers the two tile widths until the in-place
-       FFTs hold one butterfly per thread and pass (width * transform/2 / smallest radix <= 512)
-       and the LDS fits; eddy_plan_get_tuning reports what the plan uses. */
+    /* Zero fields take the defaults. The plan lowers the two tile widths until one pass of the
+       in-place FFTs fits 512 threads of up to 8 complex points each and the LDS fits;
+       eddy_plan_get_tuning reports what the plan uses. */
     int yfft_pencils;   /* pencils (consecutive x1 lines) per workgroup in the y-FFT: power of 2
-                           <= 64 (default: the smallest of 16, 32, 64 with pencils x L >= 4096,
-                           at most the next power of 2 of M) */
-    int ztrans_pencils; /* lines per workgroup in the x2 transform: power of 2, >= 4 (default 16) */
+                           <= 64 (default: 16, doubled while pencils x L < 4096, three of the
+                           doubled tiles fit a CU's LDS and pencils < M) */
+    int ztrans_pencils; /* lines per workgroup in the x2 transform: power of 2, >= 4 (default 16,
+                           the DCT's doubled as for the y-FFT) */
     int xsolve_chunk;   /* max rows per thread in the x1 solve: the PCR-to-Thomas switch (3..32,
                            default 12; EDDY_ERR_ARG outside) */
     int use_dense_z;    /* 1: force the dense x2 eigen-transform even on a uniform x2 grid */
@@ -328,7 +329,9 @@ int eddy_iovector_write_dev(const char* path, const double* d_u, const double* d
                             void* stream);
 
 /* ---------------------------------------------------------------------------------------
- * Kernel timing (hipEvents around each launch on the plan's stream).
+ * Kernel timing (hipEvents around each launch on the plan's stream). While it is on, a plan whose
+ * planes go through one kernel runs the x2 transform, x1 solve and inverse transform as kernels of
+ * their own, each with its time.
  * ------------------------------------------------------------------------------------- */
 enum {
     EDDY_K_YFFT_FWD = 0, EDDY_K_ZTRANS_FWD, EDDY_K_XSOLVE, EDDY_K_ZTRANS_INV, EDDY_K_YFFT_INV,
