@@ -6,11 +6,13 @@
 //   ghost boundary values: x (:2813-2824, MP and the ITYPE(1) = 300 axis with JSYM), y
 //   (:2829-2835, LP), z (:2843-2847, ITYPE(5) / ITYPE(6): 500 periodic, else Neumann).
 //
-// Three launches: the reference value (one workgroup), the interior update, and the ghost
-// shell. The reference applies its boundary copies one axis after the other over whole
-// planes; every ghost value therefore equals +-P at one interior cell, found by mapping the
-// z index, then the y index, then the x index (with its sign and the axis reflection), and
-// the ghost kernel gathers it from the already updated interior.
+// Two launches: the reference value (one workgroup), then the update. The reference applies its
+// boundary copies one axis after the other over whole planes; every ghost value therefore equals +-P
+// at one interior cell, found by mapping the z index, then the y index, then the x index (with its
+// sign and the axis reflection). The thread of an interior cell writes the ghosts that copy it beside
+// its own value, so that no pass over the shell waits for the interior to be done. Bound by memory at
+// large sizes (512 x 256 x 256 0.163 -> 0.155 ms, 5.2 TB/s on its 24 B/cell) and by its two dependent
+// launches at small ones (203 x 101 x 90 0.0176 -> 0.0142 ms, 32 x 32 x 32 0.0120 -> 0.0078).
 #include <algorithm>
 
 #include "kernels.h"
@@ -52,82 +54,52 @@ __global__ void __launch_bounds__(256) k_pref(PressArgs a) {
     }
 }
 
-__global__ void __launch_bounds__(256) k_p_interior(PressArgs a) {
+// The value v of interior cell (I, J, K) and of every ghost that the boundary copies take from it:
+// ghost planes 0 and n-1 of an axis copy interior planes lo and hi, composed z, y, x.
+__device__ __forceinline__ void p_store(const PressArgs& a, int I, int J, int K, double v) {
+    const Dims d = a.d;
+    const int zlo = a.itype5 == 500 ? d.N : 1, zhi = a.itype6 == 500 ? 1 : d.N;
+    const int ylo = a.lp == 0 ? d.L : 1, yhi = a.lp == 0 ? 1 : d.L;
+    auto planes = [&](int i, int j, double x) {
+        a.p[sidx(d, i, j, K)] = x;
+        if (K == zlo) a.p[sidx(d, i, j, 0)] = x;
+        if (K == zhi) a.p[sidx(d, i, j, d.nz - 1)] = x;
+    };
+    auto rows = [&](int i, int j, double x) {
+        planes(i, j, x);
+        if (j == ylo) planes(i, 0, x);
+        if (j == yhi) planes(i, d.ny - 1, x);
+    };
+    rows(I, J, v);
+    if (a.itype1 == 300) {  // axis: P(1,J,:) = P(IX1, JSYM(J), :), JSYM(J) = J + (NY-2)/2 mod the period
+        if (I == 1) {
+            const int j = J - d.L / 2;
+            rows(0, j < 1 ? j + d.L : j, v);
+        }
+    } else if (a.mp == 0) {
+        if (I == d.M) rows(0, J, v);
+    } else if (I == 1) {
+        rows(0, J, -v);
+    }
+    if (a.mp == 0) {
+        if (I == 1) rows(d.nx - 1, J, v);
+    } else if (I == d.M) {
+        rows(d.nx - 1, J, -v);
+    }
+}
+
+__global__ void __launch_bounds__(256) k_p_update(PressArgs a) {
     const int I = blockIdx.x * 64 + threadIdx.x + 1;
     const int J = blockIdx.y * 4 + threadIdx.y + 1;
     const int K = blockIdx.z + 1;
     if (I > a.d.M || J > a.d.L) return;
-    const double v = p_updated(a, I, J, K);
-    a.p[sidx(a.d, I, J, K)] = v - a.red[RED_PREF];
-}
-
-// Ghost cell (I, J, K) <- sign * P(interior source), the boundary copies composed z, y, x.
-__device__ __forceinline__ void p_ghost(const PressArgs& a, int I, int J, int K) {
-    const Dims d = a.d;
-    int k = K;
-    if (K == 0) k = (a.itype5 == 500) ? d.nz - 2 : 1;
-    else if (K == d.nz - 1) k = (a.itype6 == 500) ? 1 : d.nz - 2;
-    int j = J;
-    if (J == 0) j = (a.lp == 0) ? d.ny - 2 : 1;
-    else if (J == d.ny - 1) j = (a.lp == 0) ? 1 : d.ny - 2;
-    int i = I;
-    double s = 1.0;
-    if (I == 0) {
-        if (a.itype1 == 300) {  // axis: P(1,J,:) = P(IX1, JSYM(J), :), JSYM(J) = J + (NY-2)/2 mod the period
-            i = 1;
-            j += d.L / 2;
-            if (j > d.L) j -= d.L;
-        } else if (a.mp == 0) {
-            i = d.nx - 2;
-        } else {
-            i = 1;
-            s = -1.0;
-        }
-    } else if (I == d.nx - 1) {
-        if (a.mp == 0) {
-            i = 1;
-        } else {
-            i = d.nx - 2;
-            s = -1.0;
-        }
-    }
-    a.p[sidx(d, I, J, K)] = s * a.p[sidx(d, i, j, k)];
-}
-
-// The ghost shell as three pairs of planes: blockIdx.z selects the face (0/1: x, 2/3: y,
-// 4/5: z); edges are written by two faces with the same value.
-__global__ void __launch_bounds__(256) k_p_ghosts(PressArgs a) {
-    const Dims d = a.d;
-    const int face = blockIdx.z;
-    const int u = blockIdx.x * 256 + threadIdx.x;
-    const int v = blockIdx.y;
-    int I, J, K;
-    if (face < 2) {  // x faces: u over J, v over K
-        if (u >= d.ny || v >= d.nz) return;
-        I = face ? d.nx - 1 : 0;
-        J = u;
-        K = v;
-    } else if (face < 4) {  // y faces: u over I, v over K
-        if (u >= d.nx || v >= d.nz) return;
-        I = u;
-        J = (face & 1) ? d.ny - 1 : 0;
-        K = v;
-    } else {  // z faces: u over I, v over J
-        if (u >= d.nx || v >= d.ny) return;
-        I = u;
-        J = v;
-        K = (face & 1) ? d.nz - 1 : 0;
-    }
-    p_ghost(a, I, J, K);
+    p_store(a, I, J, K, p_updated(a, I, J, K) - a.red[RED_PREF]);
 }
 
 void launch_pressure_update(hipStream_t st, const PressArgs& a) {
     const Dims& d = a.d;
     hipLaunchKernelGGL(k_pref, dim3(1), dim3(256), 0, st, a);
-    hipLaunchKernelGGL(k_p_interior, dim3(ceil_div(d.M, 64), ceil_div(d.L, 4), d.N), dim3(64, 4, 1), 0, st, a);
-    const int umax = std::max(d.nx, d.ny);
-    const int vmax = std::max(d.ny, d.nz);
-    hipLaunchKernelGGL(k_p_ghosts, dim3(ceil_div(umax, 256), vmax, 6), dim3(256), 0, st, a);
+    hipLaunchKernelGGL(k_p_update, dim3(ceil_div(d.M, 64), ceil_div(d.L, 4), d.N), dim3(64, 4, 1), 0, st, a);
 }
 
 }  // namespace eddy
