@@ -721,8 +721,15 @@ static int create_plan(eddy_plan_s** out, int nx, int ny, int nz, double delysq,
     // 64, while they hold fewer than 4096 elements and three workgroups of the doubled tile still share
     // a CU's LDS: 32 pencils of 144 to 160 elements run 2 to 13 % faster than 16, but 32 of 192 (two
     // workgroups) 11 % slower in the inverse y transform and 9 % in the forward x2 transform.
-    auto tile_grows = [&](int ti, long len, size_t doubled) {
-        return ti < 64 && ti < M && ti * len < 4096 && 3 * doubled <= lds_cap;
+    // A plan that runs alone also keeps enough workgroups for the 256 CUs: 160 of the doubled tile along y,
+    // 256 along x2 (projections with 16, 32, 64 pencils along y: 64 x 64 x 64 36.0, 37.4, 40.8 us with 256, 128 and
+    // 64 workgroups; 96 x 64 x 32 37.7, 36.3, 39.9 with 384, 192, 128; 64 x 200 x 64 71.3, 64.0, 63.1 with
+    // 800, 400, 200), and stops at 2048 elements where the y transform is the dense one, whose waves
+    // have products to hide latency with (160 x 96 x 112 109.6, 98.4, 118.3; 100 x 100 x 77 73.3, 70.7, 73.9). Among the
+    // problems of a batch throughput counts, and the others fill the CUs.
+    auto tile_grows = [&](int ti, long len, size_t doubled, int planes, int least, long enough) {
+        if (ti >= 64 || ti >= M || 3 * doubled > lds_cap) return false;
+        return batch ? ti * len < 4096 : ti * len < enough && ceil_div(M, 2 * ti) * planes >= least;
     };
     // the y transform: the radix FFT of L/2 complex points for an even L whose half factors
     // into 2, 3 and 5; any other periodic length (fftpack's general odd factors, fftpack.f:2096-
@@ -739,7 +746,8 @@ static int create_plan(eddy_plan_s** out, int nx, int ny, int nz, double delysq,
                                                       fft_tile_ok(P->fpy, ti, kFftThreads)));
         };
         if (!(tuning && tuning->yfft_pencils > 0))
-            while (tile_grows(P->tune.yfft_pencils, L, ydense ? 0 : ylds(2 * P->tune.yfft_pencils)))
+            while (tile_grows(P->tune.yfft_pencils, L, ydense ? 0 : ylds(2 * P->tune.yfft_pencils), N, 160,
+                              ydense ? 2048 : 4096))
                 P->tune.yfft_pencils *= 2;
         while (P->tune.yfft_pencils > 1 && !yok(P->tune.yfft_pencils)) P->tune.yfft_pencils /= 2;
         // (the dense DFT's matrices grow with L^2: lengths above 6500 or so stay refused)
@@ -875,7 +883,7 @@ static int create_plan(eddy_plan_s** out, int nx, int ny, int nz, double delysq,
         };
         const int zmin = P->dense ? 4 : 1;
         if (!P->dense && !(tuning && tuning->ztrans_pencils > 0))
-            while (tile_grows(P->tune.ztrans_pencils, N, zlds(2 * P->tune.ztrans_pencils)) &&
+            while (tile_grows(P->tune.ztrans_pencils, N, zlds(2 * P->tune.ztrans_pencils), L, 256, 4096) &&
                    zok(2 * P->tune.ztrans_pencils))
                 P->tune.ztrans_pencils *= 2;
         while (P->tune.ztrans_pencils > zmin && !zok(P->tune.ztrans_pencils)) P->tune.ztrans_pencils /= 2;

@@ -20,7 +20,7 @@ import numpy as np
 from . import Plan, EddyError, to_device
 
 # yfft_pencils / ztrans_pencils 0: the plan's own choice (16, doubled while a tile holds fewer than
-# 4096 elements and three of the doubled ones fit a CU; 16 for the dense x2 transform)
+# 4096 elements, three of the doubled ones fit a CU and enough are left; 16 for the dense x2 transform)
 DEFAULT = {"yfft_pencils": 0, "ztrans_pencils": 0, "xsolve_chunk": 12, "use_dense_z": 0, "fft_radix": 8,
            "yfft_gemm": 0}
 

@@ -85,8 +85,9 @@ typedef struct {
        in-place FFTs fits 512 threads of up to 8 complex points each and the LDS fits;
        eddy_plan_get_tuning reports what the plan uses. */
     int yfft_pencils;   /* pencils (consecutive x1 lines) per workgroup in the y-FFT: power of 2
-                           <= 64 (default: 16, doubled while pencils x L < 4096, three of the
-                           doubled tiles fit a CU's LDS and pencils < M) */
+                           <= 64 (default: 16, doubled while pencils x L < 4096, pencils < M, three
+                           of the doubled tiles fit a CU's LDS and, outside batches, enough of them
+                           are left for the CUs) */
     int ztrans_pencils; /* lines per workgroup in the x2 transform: power of 2, >= 4 (default 16,
                            the DCT's doubled as for the y-FFT) */
     int xsolve_chunk;   /* max rows per thread in the x1 solve: the PCR-to-Thomas switch (3..32,
