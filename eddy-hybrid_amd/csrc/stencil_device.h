@@ -20,6 +20,20 @@ __device__ __forceinline__ void st_off(V* base, unsigned byte_off, V v) {
     *reinterpret_cast<V*>(reinterpret_cast<char*>(base) + byte_off) = v;
 }
 
+// The same past the caches where NT (values read or written once, in fields larger than the caches).
+template <bool NT, typename V>
+__device__ __forceinline__ V ld_once(const V* base, unsigned byte_off) {
+    const V* p = reinterpret_cast<const V*>(reinterpret_cast<const char*>(base) + byte_off);
+    if constexpr (NT) return __builtin_nontemporal_load(p);
+    else return *p;
+}
+template <bool NT, typename V>
+__device__ __forceinline__ void st_once(V* base, unsigned byte_off, V v) {
+    V* p = reinterpret_cast<V*>(reinterpret_cast<char*>(base) + byte_off);
+    if constexpr (NT) __builtin_nontemporal_store(v, p);
+    else *p = v;
+}
+
 __device__ __forceinline__ size_t sidx(const Dims& d, int I, int J, int K) {
     return (size_t)I + (size_t)d.nx * ((size_t)J + (size_t)d.ny * (size_t)K);
 }

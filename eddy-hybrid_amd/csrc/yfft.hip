@@ -27,6 +27,7 @@
 
 namespace eddy {
 
+constexpr size_t kCacheBytes = (size_t)256 << 20;  // memory-side cache
 constexpr int kLoadBatch = 8;
 constexpr int kInvTasks = 2;  // packing tasks (4 coefficient rows each) per thread and load batch
 constexpr int kDivRows = 4;  // rows per load sub-batch of the fused divergence and residual
@@ -254,7 +255,7 @@ __device__ __forceinline__ void dft_zero_pads(T* rows, int pitch, int L, int TI,
 
 // One tile (TI pencils at one x2 index) of the forward transform; `tile` is the logical tile,
 // ntx the tiles per x2 row, `slot`/`nslots` the reduction partial index and count.
-template <typename T, int MODE, bool DENSE = false>
+template <typename T, int MODE, bool DENSE = false, bool NT = false>
 __device__ __forceinline__ void yfft_fwd_tile(const YArgs<T>& a, int tile, int ntx, int slot, int nslots) {
     extern __shared__ unsigned char smem_raw[];
     T* smem = reinterpret_cast<T*>(smem_raw);
@@ -410,35 +411,39 @@ __device__ __forceinline__ void yfft_fwd_tile(const YArgs<T>& a, int tile, int n
                 const T wdr = wr * dr - wi * di, wdi = wr * di + wi * dr;
                 const T xr = er + wdi, xi = ei - wdr;
                 if (kk == 0) {
-                    out[0] = xr;
+                    st_once<NT>(out, 0u, xr);
                 } else if (kk == H) {
-                    st_off(out, jsb * (unsigned)(L - 1), xr);
+                    st_once<NT>(out, jsb * (unsigned)(L - 1), xr);
                 } else {
-                    st_off(out, jsb * (unsigned)(2 * kk - 1), xr);
-                    st_off(out, jsb * (unsigned)(2 * kk), xi);
+                    st_once<NT>(out, jsb * (unsigned)(2 * kk - 1), xr);
+                    st_once<NT>(out, jsb * (unsigned)(2 * kk), xi);
                 }
             }
         }
     }
 }
 
-template <typename T, int MODE, bool DENSE>
+// NT: the spectrum's rows are whole lines (M a multiple of 16) and it exceeds the 256 MiB memory-side
+// cache, which non-temporal stores leave to the velocities (512 x 256 x 256: this kernel 0.2746 -> 0.2727 ms,
+// the line solve 0.1148 -> 0.1097). Rows that begin inside a line lose by it (500 x 256 x 256 0.278 -> 0.327),
+// and smaller spectra are read back from the cache (256 x 192 x 128: x2 transform 0.0284 -> 0.0320).
+template <typename T, int MODE, bool DENSE, bool NT = false>
 __global__ void __launch_bounds__(kFftThreads) k_yfft_fwd(YArgs<T> a) {
     const int nb = gridDim.x * gridDim.y;
     const int t = iblock_tile(xcd_tile(blockIdx.x + gridDim.x * blockIdx.y, nb), gridDim.x, gridDim.y, a.iblk);
-    yfft_fwd_tile<T, MODE, DENSE>(a, t, gridDim.x, linear_bid(), nb);
+    yfft_fwd_tile<T, MODE, DENSE, NT>(a, t, gridDim.x, linear_bid(), nb);
 }
 
 // The forward transform of a stored RHS at no more than 80 VGPRs: with its 42 KB LDS tile
 // (L = 256, 16 pencils) three workgroups of 8 waves then share a CU (6 waves per SIMD).
-template <typename T, bool DENSE>
+template <typename T, bool DENSE, bool NT = false>
 __global__ void __launch_bounds__(kFftThreads) __attribute__((amdgpu_waves_per_eu(6))) k_yfft_fwd_rhs(YArgs<T> a) {
     const int nb = gridDim.x * gridDim.y;
     const int t = iblock_tile(xcd_tile(blockIdx.x + gridDim.x * blockIdx.y, nb), gridDim.x, gridDim.y, a.iblk);
-    yfft_fwd_tile<T, YF_DIRECT, DENSE>(a, t, gridDim.x, linear_bid(), nb);
+    yfft_fwd_tile<T, YF_DIRECT, DENSE, NT>(a, t, gridDim.x, linear_bid(), nb);
 }
 
-template <typename T, int MODE, bool DENSE = false>
+template <typename T, int MODE, bool DENSE = false, bool NT = false>
 __device__ __forceinline__ void yfft_inv_tile(const YArgs<T>& a, int tile, int ntx, int slot) {
     extern __shared__ unsigned char smem_raw[];
     T* smem = reinterpret_cast<T*>(smem_raw);
@@ -523,10 +528,10 @@ __device__ __forceinline__ void yfft_inv_tile(const YArgs<T>& a, int tile, int n
             const unsigned qo = (q0 + u * qstep <= half) ? qo0 + (unsigned)(u * qstep) * q2 : qcap;
             const bool q0row = qo == 0;
             const unsigned ob = lm1 - qo;
-            xa_r[u] = ld_off(col, q0row ? 0u : qo - rs);
-            xa_i[u] = ld_off(col, q0row ? rs : qo);
-            xb_r[u] = ld_off(col, ob);
-            xb_i[u] = ld_off(col, q0row ? lm1 : ob + rs);
+            xa_r[u] = ld_once<NT>(col, q0row ? 0u : qo - rs);
+            xa_i[u] = ld_once<NT>(col, q0row ? rs : qo);
+            xb_r[u] = ld_once<NT>(col, ob);
+            xb_i[u] = ld_once<NT>(col, q0row ? lm1 : ob + rs);
         }
 #pragma unroll
         for (int u = 0; u < UB; ++u) {
@@ -647,11 +652,16 @@ __device__ __forceinline__ void yfft_inv_tile(const YArgs<T>& a, int tile, int n
     }
 }
 
-template <typename T, int MODE, bool DENSE>
+// NT: the spectrum's rows are whole lines and it fills the memory-side cache with the pressure; its
+// last read, past the caches, leaves them the pressure for CORRECT (512 x 256 x 256: this kernel 0.137 -> 0.131 ms
+// and CORRECT 0.343 -> 0.330; 512 x 256 x 192 0.100 -> 0.089 and 0.256 -> 0.244; 768 x 384 x 256 0.278 -> 0.259 but
+// CORRECT 0.777 -> 0.795). A smaller spectrum comes from the caches, and lines that two tiles share would be
+// read twice (300 x 256 x 250: 0.084 -> 0.097 and 0.195 -> 0.187; 300 x 128 x 128 0.0252 -> 0.0280).
+template <typename T, int MODE, bool DENSE, bool NT = false>
 // at most 80 VGPRs (the last defect-correction update needs 82 unbounded): with its 42 KB LDS
 // tile (L = 256, 16 pencils) three workgroups of 8 waves share a CU (6 waves per SIMD)
 __global__ void __launch_bounds__(kFftThreads) __attribute__((amdgpu_waves_per_eu(6))) k_yfft_inv(YArgs<T> a) {
-    yfft_inv_tile<T, MODE, DENSE>(a, xcd_tile(blockIdx.x + gridDim.x * blockIdx.y, gridDim.x * gridDim.y), gridDim.x,
+    yfft_inv_tile<T, MODE, DENSE, NT>(a, xcd_tile(blockIdx.x + gridDim.x * blockIdx.y, gridDim.x * gridDim.y), gridDim.x,
                                   linear_bid());
 }
 
@@ -702,8 +712,12 @@ void launch_yfft_fwd(hipStream_t st, const Dims& d, const FftPlan& fp, const Tab
         (void)hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sh);
         hipLaunchKernelGGL(fn, grid, dim3(kFftThreads), sh, st, a);
     };
+    constexpr bool F64 = std::is_same<T, double>::value;
+    const size_t spectrum = sizeof(T) * (size_t)d.M * d.N * d.L;
+    const bool once = F64 && d.M % 16 == 0 && spectrum > kCacheBytes;
     if (mode == YF_DIRECT) {
         if (dense) go(k_yfft_fwd<T, YF_DIRECT, true>);
+        else if (once) go(k_yfft_fwd_rhs<T, false, F64>);
         else go(k_yfft_fwd_rhs<T, false>);
     } else if (mode == YF_DIVERGENCE) {
         a.us = in.us;
@@ -716,7 +730,9 @@ void launch_yfft_fwd(hipStream_t st, const Dims& d, const FftPlan& fp, const Tab
             if (in.mt.cart) go(k_yfft_fwd<T, YF_DIV_CART, true>);
             else go(k_yfft_fwd<T, YF_DIV_CYL, true>);
         } else {
-            if (in.mt.cart) go(k_yfft_fwd<T, YF_DIV_CART, false>);
+            if (in.mt.cart && once) go(k_yfft_fwd<T, YF_DIV_CART, false, F64>);
+            else if (in.mt.cart) go(k_yfft_fwd<T, YF_DIV_CART, false>);
+            else if (once) go(k_yfft_fwd<T, YF_DIV_CYL, false, F64>);
             else go(k_yfft_fwd<T, YF_DIV_CYL, false>);
         }
         if (in.fold) {
@@ -755,9 +771,12 @@ void launch_yfft_inv(hipStream_t st, const Dims& d, const FftPlan& fp, const Tab
         (void)hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sh);
         hipLaunchKernelGGL(fn, grid, dim3(kFftThreads), sh, st, a);
     };
+    constexpr bool F64 = std::is_same<T, double>::value;
+    const size_t spectrum = sizeof(T) * (size_t)d.M * d.N * d.L;
     switch (mode) {
         case YI_DIRECT:
             if (dense) go(k_yfft_inv<T, YI_DIRECT, true>);
+            else if (F64 && d.M % 16 == 0 && 2 * spectrum >= kCacheBytes) go(k_yfft_inv<T, YI_DIRECT, false, F64>);
             else go(k_yfft_inv<T, YI_DIRECT, false>);
             break;
         case YI_STORE:
