@@ -423,7 +423,7 @@ __device__ __forceinline__ void yfft_fwd_tile(const YArgs<T>& a, int tile, int n
     }
 }
 
-// NT: the spectrum's rows are whole lines (M a multiple of 16) and it exceeds the 256 MiB memory-side
+// NT: the spectrum's rows are whole lines (M a multiple of 16) and it fills the 256 MiB memory-side
 // cache, which non-temporal stores leave to the velocities (512 x 256 x 256: this kernel 0.2746 -> 0.2727 ms,
 // the line solve 0.1148 -> 0.1097). Rows that begin inside a line lose by it (500 x 256 x 256 0.278 -> 0.327),
 // and smaller spectra are read back from the cache (256 x 192 x 128: x2 transform 0.0284 -> 0.0320).
@@ -714,7 +714,7 @@ void launch_yfft_fwd(hipStream_t st, const Dims& d, const FftPlan& fp, const Tab
     };
     constexpr bool F64 = std::is_same<T, double>::value;
     const size_t spectrum = sizeof(T) * (size_t)d.M * d.N * d.L;
-    const bool once = F64 && d.M % 16 == 0 && spectrum > kCacheBytes;
+    const bool once = F64 && d.M % 16 == 0 && spectrum >= kCacheBytes;
     if (mode == YF_DIRECT) {
         if (dense) go(k_yfft_fwd<T, YF_DIRECT, true>);
         else if (once) go(k_yfft_fwd_rhs<T, false, F64>);
