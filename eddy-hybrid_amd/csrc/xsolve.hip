@@ -47,8 +47,11 @@ __device__ __forceinline__ void xsolve_tile(const XArgs<T>& a, int lb) {
     if (nl <= 0) return;
 
     // The wave's lines, contiguous in S, into its LDS: element lane + 64 u, every load in flight
-    // together; elements past the last line read the last one (finite values for lanes whose
-    // results are not stored)
+    // together. Every slot that a lane reads as a row of its line is written, also for lanes without a
+    // line: their results are not stored, but the reduction's wrapped shuffles carry their values, times
+    // 0, into the lines that are there, so those must be finite. Elements past the last line take the
+    // last one's value; in the padded layout, where they fall elsewhere, a lane without a line zeroes
+    // its own rows.
     T* const blk = a.S + (size_t)line0 * (size_t)M;
     const int nel = nl * M;
     const int wi = lane + (lane >> 3);
@@ -82,6 +85,11 @@ __device__ __forceinline__ void xsolve_tile(const XArgs<T>& a, int lb) {
             } else if (FIXED || u < Q) {
                 tile[wi + 72 * u] = v[u];
             }
+        if (PADDED && nl < LW && lane >= nl * P) {
+            const int e0 = lane * QMAX;
+#pragma unroll
+            for (int r = 0; r < QMAX; ++r) tile[e0 + r + ((e0 + r) >> 3)] = T(0);
+        }
     }
     // the wave's LDS operations complete in order; this only keeps the compiler from moving them
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");

@@ -63,11 +63,12 @@ constexpr double kDecoupled = 0x1p-80;
 // (M <= P*Q); Q = QMAX and M = P*Q (no row checks).
 enum XRows { XR_ANY = 0, XR_PADDED = 1, XR_EXACT = 2 };
 
-// Solve the wave's 64/P lines, P lanes and Q rows per lane. get(r) is the right-hand side of this lane's row r, put(r, x) takes its solution.
-// Returns the sum of the lane's solution rows. CYC: periodic lines, solved as the tridiagonal
-// part T' plus a rank-one correction (Sherman-Morrison, the method of the reference's CYCLIC,
-// numrec.f:754-781): T = T' + u v^T with u = (g, 0, ..., 0, alpha), v = (1, 0, ..., 0, beta/g),
-// g = -b(0); the elimination carries the second right-hand side u beside d, and
+// Solve the wave's 64/P lines, P lanes and Q rows per lane. get(r) is the right-hand side of this lane's
+// row r (any finite value in lanes without a line), put(r, x) takes its solution. Returns the sum of
+// the lane's solution rows. CYC: periodic lines, solved as the tridiagonal part T' plus a rank-one
+// correction (Sherman-Morrison, the method of the reference's CYCLIC, numrec.f:754-781):
+// T = T' + u v^T with u = (g, 0, ..., 0, alpha), v = (1, 0, ..., 0, beta/g), g = -b(0); the
+// elimination carries the second right-hand side u beside d, and
 // x = y - z (y_0 + beta y_{M-1}/g) / (1 + z_0 + beta z_{M-1}/g). The singular line is pinned at
 // x(0) = 0 and solved without the correction (its corner couplings act on x(0) = 0).
 template <typename T, int QMAX, int ROWS, bool CYC, typename Get, typename Put>
@@ -170,8 +171,8 @@ __device__ __forceinline__ T xsolve_lines(const XArgs<T>& a, int p, int lane, T 
     // (wave shuffles), and each odd unknown follows from its own row:
     // y_2p+1 = d1 - a1 y_2p - c1 y_2p+2. Rows at a line end have the coupling to the missing
     // side at exactly 0 (AM(1) = CM(M) = 0 at the walls, identity padding rows), so the
-    // neighbours fetched across a line end (wrapping inside the wave) are finite values
-    // multiplied by 0.
+    // neighbours fetched across a line end (wrapping inside the wave) are multiplied by 0; they are
+    // finite in lanes without a line too, as get() is (0 * NaN would be NaN).
     T a0 = aa[0], c0 = cc[0], d0 = dd[0], e0 = CYC ? ee[0] : T(0);
     const T a1 = lastA, c1 = lastC, d1 = lastD, e1 = lastE;
     {  // even row 2p minus a0 * row 2p-1 (lane p-1's odd row) minus c0 * row 2p+1 (own odd row)
