@@ -6,6 +6,8 @@
 #include <cstddef>
 #include <cstdint>
 
+#include "index_map.h"
+
 namespace eddy {
 
 constexpr int kMaxRadices = 16;
@@ -96,16 +98,6 @@ struct MeanShift {
 };
 
 __host__ __device__ inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
-
-// Workgroups are dispatched round-robin over the 8 XCDs (workgroup b runs on XCD b % 8) and
-// each XCD has its own L2. Give workgroups b, b+8, b+16, ... (one XCD) consecutive logical
-// tiles, so neighbouring tiles -- which share cache lines at their edges and, for stencils,
-// neighbouring planes -- meet in the same L2. Bijective on [0, n).
-__device__ __forceinline__ int xcd_tile(int b, int n) {
-    const int q = n >> 3, r = n & 7;
-    const int x = b & 7;
-    return x * q + (x < r ? x : r) + (b >> 3);
-}
 
 // Item of workgroup b when runs of C consecutive items share an XCD. Workgroups are dealt
 // to the 8 XCDs in turn (XCD b % 8), so workgroup b takes item ((s / C) * 8 + b % 8) * C + s % C

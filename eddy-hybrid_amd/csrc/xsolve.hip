@@ -146,15 +146,18 @@ __device__ __forceinline__ void xsolve_tile(const XArgs<T>& a, int lb) {
     }
 }
 
-// The lines are walked from the last to the first, against the order of the x2 transforms on both
-// sides: each then starts on what the pass before it left in the 256 MiB memory-side cache. At
-// 768 x 384 x 256 (a spectrum of 604 MB) this solve takes 0.284 ms instead of 0.310 and the inverse
-// x2 transform 0.369 instead of 0.387; nothing changes at 512 x 256 x 256 (268 MB) and below.
+// Each XCD walks its lines from the last to the first, against the order of the x2 transforms on both
+// sides: every pass then starts on what the pass before it left in the caches. The eighth of the lines
+// that an XCD takes is the eighth of the x2 transforms' tiles that it took, so that spectra that fit the
+// L2s are found there (128 x 128 x 128, 17 MB: this solve 0.0137 ms and the inverse x2 transform 0.0139; 0.0167 and
+// 0.0137 in forward order; 0.0205 and 0.0204 where reversing the whole order gives an XCD another's eighth), and
+// larger ones in the memory-side cache (768 x 384 x 256, 604 MB: 0.284 instead of 0.310 in forward order and
+// 0.369 instead of 0.387).
 template <typename T, int QMAX, int ROWS, bool CYC>
 __global__ void __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 && ROWS != XR_ANY ? (QMAX <= 8 ? 6 : 4) : 1)))
 k_xsolve(XArgs<T> a) {
-    xsolve_tile<T, QMAX, ROWS, CYC>(a, xcd_tile(gridDim.x - 1 - blockIdx.x, gridDim.x));
+    xsolve_tile<T, QMAX, ROWS, CYC>(a, xcd_tile_back(blockIdx.x, gridDim.x));
 }
 
 // Pick P (threads per line, a power of two <= 64) and Q (rows per thread, 3 <= Q <= qmax):

@@ -1,0 +1,40 @@
+"""The index maps of csrc/index_map.h, compiled for the host."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CSRC = os.path.join(ROOT, "eddy-hybrid_amd", "csrc")
+
+
+def run(tmp_path, body, flags=()):
+    cxx = shutil.which("g++")
+    if cxx is None:
+        pytest.skip("no host C++ compiler")
+    src, exe = str(tmp_path / "t.cpp"), str(tmp_path / "t")
+    with open(src, "w") as f:
+        f.write('#define __host__\n#define __device__\n#include "index_map.h"\n#include <cstdio>\n#include <vector>\n'
+                "using namespace eddy;\n" + body)
+    subprocess.run([cxx, "-std=c++17", "-O1", *flags, "-I", CSRC, src, "-o", exe], check=True)
+    return subprocess.run([exe], capture_output=True, text=True, timeout=300)
+
+
+def test_line_solve_order_keeps_each_xcds_eighth(tmp_path):
+    """Every tile once, and each on the XCD (workgroup number modulo 8) that takes it in the forward order."""
+    r = run(tmp_path, """
+int main() {
+    for (int n = 1; n < 3000; ++n) {
+        std::vector<int> xcd(n), seen(n, 0);
+        for (int b = 0; b < n; ++b) xcd[xcd_tile(b, n)] = b % 8;
+        int last[8] = {n, n, n, n, n, n, n, n};
+        for (int b = 0; b < n; ++b) {
+            const int t = xcd_tile_back(b, n);
+            if (t < 0 || t >= n || seen[t]++ || xcd[t] != b % 8 || t >= last[b % 8]) return printf("n %d b %d\\n", n, b), 1;
+            last[b % 8] = t;
+        }
+    }
+}
+""")
+    assert r.returncode == 0, r.stdout
