@@ -37,6 +37,7 @@ struct PlaneArgs {
 };
 
 constexpr int kPlaneThreads = 1024;
+constexpr int kPlaneSmall = 6144;  // planes up to this take 512 threads, two to a CU
 constexpr size_t kPlaneLds = 160 * 1024 - 512;  // beside the static reduction scratch
 
 // The lane index as a value the compiler cannot see through: inside the loops over a wave's pencils
@@ -330,14 +331,19 @@ static size_t plane_lds_bytes(const Dims& d, int dense, size_t tsz) {
 }
 
 // When the planes go through one workgroup each. The dense transform always gains where it fits
-// (whole FP64 projections, three kernels against one: 32 x 16 x 24 0.0373 -> 0.0257 ms, 120 x 101 x 64
-// 0.129 -> 0.093, 64 x 100 x 256 0.173 -> 0.085: its products move from the vector ALUs to the matrix
-// cores too). The cosine form's work is bound by the issue of the one CU a plane runs on, so
-// it pays where there are planes for half the CUs (L >= 128: 128 x 128 x 256 0.156 -> 0.141, 64 x 128 x 192
-// 0.091 -> 0.078, 96 x 64 x 128 0.0587 -> 0.0543, but 128 x 128 x 96 0.091 -> 0.093) or where the planes are so
-// small that launches and latency rule (64 x 64 x 32 0.0380 -> 0.0353, 48 x 32 x 32 0.0355 -> 0.0303; N/2
-// not a power of two: 30 x 90 x 64 0.0450 -> 0.0400, but 100 x 40 x 48 0.0463 -> 0.0488; 128 x 64 x 32 0.0405 ->
-// 0.0459). The FP32 sweeps follow the FP64 rule and its LDS.
+// (solves, three kernels against one: 32 x 24 x 96 0.034 -> 0.019 ms, 100 x 60 x 128 0.088 -> 0.044, 127 x 127 x 16 0.087 ->
+// 0.080: its products move from the vector ALUs to the matrix cores too). The cosine form's work is bound by the
+// issue of the one CU a plane runs on, so it pays where launches and latency rule or where the planes fill the CUs.
+// Solves with the three kernels and with the one, ratio of the times:
+//   planes up to 3072, any L: 48 x 48 0.85 to 0.95, 30 x 90 0.87 to 0.96, 96 x 32 0.90 to 0.97, 48 x 64 0.91 to 0.99; past it
+//   64 x 64 x 32 1.09, 32 x 128 x 16 1.03;
+//   larger ones from the L where they break even, 48 + plane / 86 (a line through 64 x 64 x 80 1.02, x 96 0.99,
+//   x 144 0.90; 96 x 64 x 112 1.02, x 144 0.90; 64 x 128 x 112 1.05, x 144 0.91; 128 x 96 x 176 1.00, x 208 0.94;
+//   128 x 128 x 192 1.01, x 240 0.90; 120 x 120 x 192 1.05, x 240 0.93);
+//   planes past 6144 run on 1024 threads, one to a CU, and a second round of them loses: L = 288 1.07 to 1.23
+//   (96 x 64 x 640, two to a CU, 0.94);
+//   run-time FFT passes that hold a radix of 2 lose: 100 x 60 (N/2 = 30) x 128 1.17, x 208 1.00; 160 x 100 x 256 1.11.
+// The FP32 sweeps follow the FP64 rule and its LDS (0.87 to 1.05 on the taken side).
 bool zplane_fits(const Dims& d, const FftPlan& fpz, int dense, int chunk) {
     int P = 0, Q = 0;
     if (d.cyc_x || !xsolve_partition(d.M, chunk, P, Q) || Q > 16) return false;
@@ -345,8 +351,10 @@ bool zplane_fits(const Dims& d, const FftPlan& fpz, int dense, int chunk) {
     if (dense) return d.M < 128 && d.N < 128;
     // a wave's FFT call holds whole pencils, one butterfly per lane and pass
     if (fpz.n / min_radix(fpz) > 64) return false;
-    const bool pow2 = (fpz.n & (fpz.n - 1)) == 0;
-    return d.L >= 128 || d.M * d.N <= (pow2 ? 4096 : 3072);
+    const int plane = d.M * d.N;
+    if (plane <= 3072) return true;
+    if (min_radix(fpz) < 3 && fpz.n > 8) return false;
+    return plane <= 86 * (d.L - 48) && (plane <= kPlaneSmall || d.L <= 256);
 }
 
 template <typename T>
@@ -364,7 +372,7 @@ void launch_zplane(hipStream_t st, const Dims& d, const FftPlan& fpz, const Tabl
     a.rM = (unsigned)(((1ull << 32) + d.M - 1) / d.M);
     const size_t lds = plane_lds_bytes(d, dense, sizeof(T));
     // 512 threads for the small planes (64 x 64 x 32: 0.0353 ms, 0.0360 with 1024)
-    const int nthr = d.M * d.N <= 6144 ? 512 : kPlaneThreads;
+    const int nthr = d.M * d.N <= kPlaneSmall ? 512 : kPlaneThreads;
     a.pw = dense ? 1 : std::max(1, 64 / std::max(1, fpz.n / min_radix(fpz)));
     xsolve_dispatch(xsolve_class(d.M, a.x.P, a.x.Q, false), [&](auto qmax, auto rows) {
         constexpr int QMAX = decltype(qmax)::value;
