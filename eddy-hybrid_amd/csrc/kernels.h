@@ -179,7 +179,7 @@ struct StageLaunch {
     int cls_total[kMaxClasses] = {};
     size_t cls_lds[kMaxClasses] = {};
     // the forward y transform with the divergence: 1 every problem Cartesian, 2 every one
-    // cylindrical (a kernel with only that metric's registers), 0 mixed
+    // cylindrical (a kernel with only that metric's registers), 0 mixed; CORRECT: 1 streamed loads
     int kind = 0;
     const double* alf = nullptr;  // CORRECT: device {ALFXDT, 1/ALFXDT}
 };

@@ -88,10 +88,21 @@ __host__ __device__ inline int span_blocks(const Dims& d) { return ceil_div(d.L 
 __device__ __forceinline__ d2 ld_pair(const double* b, unsigned off) {
     return *reinterpret_cast<const d2u*>(reinterpret_cast<const char*>(b) + off);
 }
-// The velocities are streamed (read once, written once): non-temporal, so that they do not push
-// dp's planes out of L2 nor the solve's arrays out of the memory-side cache.
-__device__ __forceinline__ d2 ld_stream(const double* b, unsigned off) {
-    return __builtin_nontemporal_load(reinterpret_cast<const d2u*>(reinterpret_cast<const char*>(b) + off));
+// The velocities are streamed (read once, written once): non-temporal, so that they do not push dp's
+// planes out of L2 nor the solve's arrays out of the memory-side cache. Small fields (kCorrectCached) are
+// read through the caches: the forward y transform has just read u*, and what it left there is lost to a
+// non-temporal load (projections on the same fields again, and on others each time, read past the caches and
+// through them: 128 x 96 x 64 0.0540 -> 0.0501 ms and 0.0558 -> 0.0548, 120 x 90 x 80 0.0704 -> 0.0661 and 0.0723 ->
+// 0.0715; CORRECT alone 0.0109 -> 0.0072 and 0.0126 -> 0.0137 at the first). Larger fields gain in the second case
+// what they lose in the first (203 x 101 x 90 0.1091 -> 0.1029 and 0.1112 -> 0.1121; its four calls of a substep
+// 0.131 -> 0.136; 240 x 128 x 128 0.1418 -> 0.1339 and 0.1474 -> 0.1578) and stay streamed; CORRECT alone on the same
+// fields again is then slower than through the caches (128 x 128 x 128 0.0235 and 0.0197), on others faster (0.0249
+// and 0.0279).
+template <bool STREAM>
+__device__ __forceinline__ d2 ld_velocity(const double* b, unsigned off) {
+    const d2u* p = reinterpret_cast<const d2u*>(reinterpret_cast<const char*>(b) + off);
+    if constexpr (STREAM) return __builtin_nontemporal_load(p);
+    else return *p;
 }
 __device__ __forceinline__ void st_stream(double* b, unsigned off, d2 v) {
     __builtin_nontemporal_store(v, reinterpret_cast<d2u*>(reinterpret_cast<char*>(b) + off));
@@ -114,7 +125,12 @@ __device__ __forceinline__ Pair span_pair(const Dims& d, unsigned r, unsigned rn
     return Pair{i, j, j >= 1 && j <= d.L && i <= d.M};
 }
 
+// Whether the seven fields of CORRECT exceed `mib` MiB together.
+static inline bool correct_exceeds(size_t cells, size_t mib) { return 7 * sizeof(double) * cells > (mib << 20); }
+constexpr size_t kCorrectCached = 64;  // MiB up to which the velocities are read through the caches
+
 // Block `b` of plane k's span (k 0-based interior).
+template <bool STREAM>
 __device__ __forceinline__ void correct_span(const CorrArgs& c, double alfxdt, int refresh, int k, int b, int tid) {
     const Dims& d = c.d;
     const unsigned nx = (unsigned)d.nx, pl = nx * (unsigned)d.ny;
@@ -135,9 +151,9 @@ __device__ __forceinline__ void correct_span(const CorrArgs& c, double alfxdt, i
         pe[q] = ld_off(c.dp, o[q] + 16u);
         pn[q] = ld_pair(c.dp, o[q] + 8u * nx);
         pt[q] = ld_pair(c.dp, o[q] + 8u * pl);
-        u[q] = ld_stream(c.us, o[q]);
-        v[q] = ld_stream(c.vs, o[q]);
-        w[q] = ld_stream(c.ws, o[q]);
+        u[q] = ld_velocity<STREAM>(c.us, o[q]);
+        v[q] = ld_velocity<STREAM>(c.vs, o[q]);
+        w[q] = ld_velocity<STREAM>(c.ws, o[q]);
     }
 #pragma unroll
     for (int q = 0; q < kSpanParts; ++q) {
@@ -183,10 +199,11 @@ __device__ __forceinline__ void correct_span(const CorrArgs& c, double alfxdt, i
 
 // Item t of a problem's nb x N blocks, the planes in pairs (dp's plane k + 1, read with plane k, is
 // then read again by the block after it).
+template <bool STREAM>
 __device__ __forceinline__ void correct_item(const CorrArgs& c, double alfxdt, int refresh, int t, int nb) {
     const int c0 = t / (2 * nb), r = t - c0 * 2 * nb, kc = min(2, c.d.N - 2 * c0);
     const int b = r / kc;
-    correct_span(c, alfxdt, refresh, 2 * c0 + r - b * kc, b, (int)threadIdx.x);
+    correct_span<STREAM>(c, alfxdt, refresh, 2 * c0 + r - b * kc, b, (int)threadIdx.x);
 }
 
 // The XCDs share the field in runs of kCorrectRun blocks, so that the eight of them work within a
@@ -196,11 +213,13 @@ __device__ __forceinline__ void correct_item(const CorrArgs& c, double alfxdt, i
 // fields come out of the cache and take the eighths (256 x 128 x 128: 0.0385 against 0.0397 ms).
 constexpr int kCorrectRun = 16;
 
+template <bool STREAM>
 __global__ void __launch_bounds__(256) k_correct_span(CorrArgs c, double alfxdt, int refresh, int runs,
                                                       const double* __restrict__ dscale) {
     const int b = blockIdx.x, n = gridDim.x;
     if (dscale) alfxdt = dscale[0];
-    correct_item(c, alfxdt, refresh, runs ? xcd_run(b, n, kCorrectRun) : xcd_tile(b, n), n / c.d.N);
+    const int t = runs ? xcd_run(b, n, kCorrectRun) : xcd_tile(b, n);
+    correct_item<STREAM>(c, alfxdt, refresh, t, n / c.d.N);
 }
 
 static CorrArgs corr_args(const Dims& d, const Metrics& mt, const double* us, const double* vs, const double* ws,
@@ -528,11 +547,12 @@ __global__ void __launch_bounds__(256) k_batch_cells(const Job<CellArgs>* jobs, 
 }
 
 // CORRECT of a batch; alf = {ALFXDT, 1/ALFXDT} on the device.
+template <bool STREAM>
 __global__ void __launch_bounds__(256) k_batch_correct(const Job<CorrArgs>* jobs, int njobs, int total,
                                                        const double* __restrict__ alf) {
     const double alfxdt = alf[0];
     run_item<kCorrectRun>(jobs, njobs, total,
-                          [=](const Job<CorrArgs>& J, int t) { correct_item(J.a, alfxdt, 1, t, J.ntx); });
+                          [=](const Job<CorrArgs>& J, int t) { correct_item<STREAM>(J.a, alfxdt, 1, t, J.ntx); });
 }
 
 template <typename T>
@@ -573,7 +593,9 @@ int prepare_cells(const std::vector<BatchProblem<double>>& pr, int op, StageLaun
     if (op != BC_CORRECT) return prepare_cells_t(pr, op, out, owned);
     std::vector<Job<CorrArgs>> jobs;
     out = StageLaunch{};
+    size_t cells = 0;
     for (const auto& p : pr) {
+        cells += (size_t)p.d.nx * p.d.ny * p.d.nz;
         Job<CorrArgs> j{};
         j.a = corr_args(p.d, p.mt, p.us, p.vs, p.ws, p.uo, p.vo, p.wo, p.dp);
         j.ntx = span_blocks(p.d);
@@ -581,6 +603,7 @@ int prepare_cells(const std::vector<BatchProblem<double>>& pr, int op, StageLaun
         if (!add_class_job(out, jobs, j, 0, 0)) return -1;
     }
     out.alf = pr.empty() ? nullptr : pr[0].dscale;
+    out.kind = correct_exceeds(cells, kCorrectCached);
     return upload_jobs(jobs, out, owned);
 }
 int prepare_cells_f(const std::vector<BatchProblem<float>>& pr, int op, StageLaunch& out,
@@ -590,8 +613,12 @@ int prepare_cells_f(const std::vector<BatchProblem<float>>& pr, int op, StageLau
 
 void batch_cells(hipStream_t st, const StageLaunch& sl, int op) {
     if (op == BC_CORRECT) {
-        hipLaunchKernelGGL(k_batch_correct, dim3(std::max(sl.total, 1)), dim3(256), 0, st,
-                           (const Job<CorrArgs>*)sl.jobs, sl.njobs, sl.total, sl.alf);
+        auto go = [&](auto fn) {
+            hipLaunchKernelGGL(fn, dim3(std::max(sl.total, 1)), dim3(256), 0, st, (const Job<CorrArgs>*)sl.jobs,
+                               sl.njobs, sl.total, sl.alf);
+        };
+        if (sl.kind) go(k_batch_correct<true>);
+        else go(k_batch_correct<false>);
         return;
     }
     auto go = [&](auto fn) {
@@ -659,9 +686,15 @@ void launch_div_minmax(hipStream_t st, const Dims& d, const Metrics& mt, const d
 void launch_correct(hipStream_t st, const Dims& d, const Metrics& mt, const double* us, const double* vs,
                     const double* ws, double* uo, double* vo, double* wo, const double* dp, double alfxdt,
                     int refresh_periodic, const double* dscale) {
-    const int runs = 7 * sizeof(double) * (size_t)d.nx * d.ny * d.nz > ((size_t)256 << 20);
-    hipLaunchKernelGGL(k_correct_span, dim3(span_blocks(d) * d.N), dim3(256), 0, st,
-                       corr_args(d, mt, us, vs, ws, uo, vo, wo, dp), alfxdt, refresh_periodic, runs, dscale);
+    const CorrArgs c = corr_args(d, mt, us, vs, ws, uo, vo, wo, dp);
+    const size_t cells = (size_t)d.nx * d.ny * d.nz;
+    const int runs = correct_exceeds(cells, 256);
+    auto go = [&](auto fn) {
+        hipLaunchKernelGGL(fn, dim3(span_blocks(d) * d.N), dim3(256), 0, st, c, alfxdt, refresh_periodic, runs,
+                           dscale);
+    };
+    if (correct_exceeds(cells, kCorrectCached)) go(k_correct_span<true>);
+    else go(k_correct_span<false>);
 }
 
 void launch_laplacian(hipStream_t st, const Dims& d, const Op64& op, const double* phi, double* out) {
