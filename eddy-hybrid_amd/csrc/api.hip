@@ -856,11 +856,11 @@ static int create_plan(eddy_plan_s** out, int nx, int ny, int nz, double delysq,
             const double s = std::sin(M_PI * (double)m / (2.0 * N));
             h.lam[m] = -4.0 * c * s * s;
         }
-        h.wsum[0] = 1.0;
         P->d.null_m = 0;
         if (!radix_plan(N / 2, P->fpz, P->tune.fft_radix)) {
-            P->dense = 1;
+            P->dense = 1;  // its column sums are added up below
         } else {
+            h.wsum[0] = 1.0;
             twiddles(N / 2, N / 2, h.ztwc_re, h.ztwc_im);
             twiddles(N, N / 2 + 1, h.ztwr_re, h.ztwr_im);
             h.zdct_re.resize(N);
