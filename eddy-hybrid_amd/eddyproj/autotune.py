@@ -7,9 +7,10 @@ Picks, per grid, the launch parameters the kernels expose (include/eddyproj.h, e
                       hands over to Thomas elimination (P = M / chunk threads per line do PCR
                       on the 2P chunk ends, each thread runs Thomas on its chunk),
   * fft_radix      -- the largest radix of the FFT radix plan (8, 4 or 2).
-Each parameter only changes its own kernels, so the search is coordinate-wise: every
-candidate value is timed with the HIP-event kernel timers of the plan (median of several
-solves), and the best value is kept before the next parameter is searched. Results are
+The search is coordinate-wise: every candidate value is timed on whole solves (median of several),
+and the best value is kept before the next parameter is searched. Whole solves, as the plan runs
+them: its kernel timers split the fused plane kernel into the three that it replaces, and a
+parameter can change which of them run (a chunk that leaves a lane more than 16 rows). Results are
 cached in a JSON table keyed by the grid shape and x2 transform kind.
 """
 import json
@@ -25,11 +26,12 @@ DEFAULT = {"yfft_pencils": 0, "ztrans_pencils": 0, "xsolve_chunk": 12, "use_dens
            "yfft_gemm": 0}
 
 SEARCH = (
-    ("yfft_pencils", (4, 8, 16, 32, 64), ("yfft_fwd", "yfft_inv")),
-    ("ztrans_pencils", (4, 8, 16, 32, 64), ("ztrans_fwd", "ztrans_inv")),
-    ("xsolve_chunk", (4, 6, 8, 12, 16, 24, 32), ("xsolve",)),
-    ("fft_radix", (8, 4, 2), ("yfft_fwd", "yfft_inv", "ztrans_fwd", "ztrans_inv")),
+    ("yfft_pencils", (4, 8, 16, 32, 64)),
+    ("ztrans_pencils", (4, 8, 16, 32, 64)),
+    ("xsolve_chunk", (4, 6, 8, 12, 16, 24, 32)),
+    ("fft_radix", (8, 4, 2)),
 )
+CALLS = 4  # solves per sample
 
 TABLE = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "lib", "tuning.json")
 
@@ -39,23 +41,24 @@ def key(g):
 
 
 def _time(g, tuning, rhs, reps):
+    """(ms per solve, effective tuning) of a plan with this tuning."""
     import torch
     plan = Plan(g, tuning=tuning, stream=torch.cuda.current_stream())  # ordered with the copies below
     effective = plan.tuning()
     d = rhs.clone()
     plan.direct(d)
-    samples = {}
+    samples = []
     for _ in range(reps):
-        plan.enable_timing(True)
-        plan.reset_timing()
         d.copy_(rhs)
-        plan.direct(d)
-        kt = plan.kernel_times()
-        for k, (n, ms) in kt.items():
-            samples.setdefault(k, []).append(ms / max(n, 1))
+        start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        start.record()
+        for _ in range(CALLS):
+            plan.direct(d)
+        end.record()
+        end.synchronize()
+        samples.append(start.elapsed_time(end) / CALLS)
     plan.close()
-    torch.cuda.synchronize()
-    return {k: float(np.median(v)) for k, v in samples.items()}, effective
+    return float(np.median(samples)), effective
 
 
 def autotune(g, reps=5, seed=0, log=None):
@@ -65,13 +68,13 @@ def autotune(g, reps=5, seed=0, log=None):
     rhs = to_device(configs.rhs_from_velocity(g, us, vs, ws))
     best = dict(DEFAULT)
     trace = []
-    for param, values, kernels in SEARCH:
+    for param, values in SEARCH:
         scores = {}
         for v in values:
             t = dict(best)
             t[param] = v
             try:
-                times, eff = _time(g, t, rhs, reps)
+                ms, eff = _time(g, t, rhs, reps)
             except EddyError as e:  # candidate not valid for this grid (LDS, divisibility)
                 trace.append({"param": param, "value": v, "error": str(e)})
                 continue
@@ -79,7 +82,7 @@ def autotune(g, reps=5, seed=0, log=None):
             if ev in scores:
                 trace.append({"param": param, "value": v, "same_as": ev})
                 continue
-            scores[ev] = sum(times[k] for k in kernels)
+            scores[ev] = ms
             trace.append({"param": param, "value": ev, "ms": round(scores[ev], 5)})
             if log:
                 log("autotune %s=%s: %.4f ms" % (param, ev, scores[ev]))
