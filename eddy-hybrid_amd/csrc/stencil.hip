@@ -76,11 +76,10 @@ struct CorrArgs {
     const double *us, *vs, *ws;
     double *uo, *vo, *wo;
     const double* dp;
-    unsigned rnx;  // ceil(2^32 / nx)
+    unsigned rnx;  // row_reciprocal(nx)
 };
 
-// ceil(2^32 / nx): the quotient of an element number by nx as a high product (span_pair)
-static inline unsigned row_magic(const Dims& d) { return (unsigned)(((1ull << 32) + d.nx - 1) / d.nx); }
+static inline unsigned row_magic(const Dims& d) { return row_reciprocal(d.nx); }
 
 // Blocks of a plane's span (its start rounded down to 16 elements).
 __host__ __device__ inline int span_blocks(const Dims& d) { return ceil_div(d.L * d.nx + 15, kSpan); }
@@ -108,21 +107,8 @@ __device__ __forceinline__ void st_stream(double* b, unsigned off, d2 v) {
     __builtin_nontemporal_store(v, reinterpret_cast<d2u*>(reinterpret_cast<char*>(b) + off));
 }
 
-// The pair of elements e, e + 1 of a field's plane (first element of the plane at `plane`): whether
-// it holds an interior cell of rows 1..L, and the x1 and y index of its first element.
-struct Pair {
-    int i, j;
-    bool on;
-};
 __device__ __forceinline__ Pair span_pair(const Dims& d, unsigned r, unsigned rnx) {
-    int j = (int)__umulhi(r, rnx);  // exact or one too large
-    int i = (int)r - j * d.nx;
-    if (i < 0) {
-        --j;
-        i += d.nx;
-    }
-    // (i, j), (i + 1, j), or (0, j + 1) past a row's end, which holds no interior cell
-    return Pair{i, j, j >= 1 && j <= d.L && i <= d.M};
+    return plane_pair(d.nx, d.M, d.L, r, rnx);
 }
 
 // Whether the seven fields of CORRECT exceed `mib` MiB together.

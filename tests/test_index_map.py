@@ -38,3 +38,32 @@ int main() {
 }
 """)
     assert r.returncode == 0, r.stdout
+
+
+def test_plane_pairs(tmp_path):
+    """Every element number that CORRECT's and the divergence range's spans produce, and those that wrap below the
+    plane's start (rows shorter than 16), against the division; without undefined arithmetic."""
+    r = run(tmp_path, """
+static bool check(int nx, int ny, unsigned r) {
+    const int M = nx - 2, L = ny - 2;
+    const Pair p = plane_pair(nx, M, L, r, row_reciprocal(nx));
+    const unsigned i = r % (unsigned)nx, j = r / (unsigned)nx;
+    const bool on = r < (unsigned)(nx * ny) && j >= 1 && j <= (unsigned)L && i <= (unsigned)M;
+    if (p.on == on && (!on || (p.i == (int)i && p.j == (int)j))) return true;
+    printf("nx %d ny %d r %u: %d %d %d\\n", nx, ny, r, p.i, p.j, (int)p.on);
+    return false;
+}
+int main() {
+    for (int nx = 4; nx < 1100; nx += nx < 80 ? 1 : 17)
+        for (int ny = 4; ny < 40; ny += 5) {
+            for (unsigned r = 0; r < (unsigned)(nx * ny) + 2048; ++r)
+                if (!check(nx, ny, r)) return 1;
+            for (unsigned below = 1; below <= 16; ++below)
+                if (!check(nx, ny, 0u - below)) return 1;
+        }
+    for (unsigned r = 0; r < 1u << 29; r += 65521)  // the largest fields: rows and planes of 2^29 elements
+        for (int nx : {4, 5, 66, 771, 2050, 130000})
+            if (!check(nx, (1 << 29) / nx, r)) return 1;
+}
+""", ["-fsanitize=undefined", "-fno-sanitize-recover=all"])
+    assert r.returncode == 0, r.stdout + r.stderr
