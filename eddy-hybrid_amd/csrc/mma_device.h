@@ -14,7 +14,6 @@ struct Mma;
 template <>
 struct Mma<double> {
     typedef double v4 __attribute__((ext_vector_type(4)));
-    typedef double v16b __attribute__((ext_vector_type(2)));
     static __device__ __forceinline__ v4 run(double a, double b, v4 c) {
         return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
     }
@@ -23,7 +22,6 @@ struct Mma<double> {
 template <>
 struct Mma<float> {
     typedef float v4 __attribute__((ext_vector_type(4)));
-    typedef float v16b __attribute__((ext_vector_type(4)));
     static __device__ __forceinline__ v4 run(float a, float b, v4 c) {
         return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
     }

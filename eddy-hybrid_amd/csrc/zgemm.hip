@@ -10,8 +10,9 @@
 // A product costs 2 x (the diagonalised length) flops per element, so the plan picks the
 // shorter axis (the production grid: M = 300 against N = 1024). Either way it is one batched
 // product over the y-modes (out of place, S <-> S2) on the matrix cores: the library's own
-// MFMA kernel (k_mma below), or a strided-batched rocBLAS GEMM when the plan asks for it.
-// The MFMA kernel applies, inside its operand loads, what the fused kernel of small N does
+// MFMA kernels (FP64 k_mma_dma and k_mma64, FP32 k_mma), or a strided-batched rocBLAS GEMM when
+// the plan asks for it.
+// The MFMA kernels apply, inside their operand loads, what the fused kernel of small N does
 // inside its tiles (rocBLAS needs two small kernels for it):
 //   forward: the solvability shift of the zero y-mode (L * VOLB/VOL subtracted from slab 0);
 //   inverse: the plain-mean correction of direct.f:894-898, delta added to the null mode's
@@ -52,17 +53,16 @@ __global__ void __launch_bounds__(256) k_zgemm_delta(T* X0, const T* linesum, co
 // A[p + r*lda], Bop(p, c) = B[p + c*ldb]; the x1-form forward product) or contiguous along
 // their own index ("x-major": A[r + p*lda], B[c + p*ldb]; every other product).
 //
+// In all three kernels the MFMA (16 x 16 x 4; lane layout in mma_device.h) takes Bop^T as its A
+// input and Aop^T as its B input, so lane x + 16q holds C(r0 + x, c0 + row(q, v)): 16 lanes store
+// 16 consecutive rows of a column of C.
+//
 // FP32 (k_mma): a workgroup (4 waves, 2 x 2) owns a BR x BC tile of C, each wave a (BR/2) x (BC/2) block
-// of 16 x 16 MFMA tiles (v_mfma_f32_16x16x4f32; FP64 v_mfma_f64_16x16x4f64). The contraction runs in
-// chunks of KC staged in LDS, in two buffers: the next chunk's global loads are in flight
-// while the MFMAs of the current one run, one barrier per chunk.
-// MFMA 16x16x4 lane layout: lane l supplies A(l%16, l/16) and B(l/16, l%16); accumulator
-// element v of lane l is D(4*(l/16) + v, l%16) for f32 and D(l/16 + 4v, l%16) for f64 (the
-// f64 rows interleave across the four lane groups; checked on the device). The MFMA takes
-// Bop^T as its A input and Aop^T as its B input, so lane x + 16q holds C(r0 + x, c0 + row(q,
-// v)): 16 lanes store 16 consecutive rows of a column of C. The MFMA's k index 4s + q (step s of a chunk, lane
-// group q) stands for chunk offset q*(KC/4) + s -- a permutation of the contraction, exact
-// in any order -- so that a lane reads KC/4 consecutive p of a p-major operand at once.
+// of 16 x 16 MFMA tiles. The contraction runs in chunks of KC staged in LDS, in two buffers: the next
+// chunk's global loads are in flight while the MFMAs of the current one run, one barrier per chunk.
+// The MFMA's k index 4s + q (step s of a chunk, lane group q) stands for chunk offset q*(KC/4) + s --
+// a permutation of the contraction, exact in any order -- so that a lane reads KC/4 consecutive p of a
+// p-major operand at once.
 template <typename T>
 struct MmArgs {
     const T* A;
@@ -85,15 +85,14 @@ struct MmArgs {
     double dnorm;
 };
 
-template <typename T>
 struct MmShape {
-    static constexpr int KC = sizeof(T) == 8 ? 16 : 32;  // contraction chunk: 128 B of p
-    static constexpr int KS = KC / 4;                    // MFMA steps per chunk
-    static constexpr int QP = KC + 16 / (int)sizeof(T);  // p-major LDS row pitch
-    static constexpr int XPAD = sizeof(T) == 8 ? 4 : 2;  // x-major LDS row pad
+    static constexpr int KC = 32;      // contraction chunk: 128 B of p
+    static constexpr int KS = KC / 4;  // MFMA steps per chunk
+    static constexpr int QP = KC + 4;  // p-major LDS row pitch
+    static constexpr int XPAD = 2;     // x-major LDS row pad
 };
 
-// LDS: p-major operands as rows X[x][p'] (pitch QP: a lane's KS consecutive p' are one or two
+// LDS: p-major operands as rows X[x][p'] (pitch QP: a lane's KS consecutive p' are two
 // 16-byte reads, and the 16 rows a read touches fall in distinct banks); x-major operands as
 // rows X[p'][x] (pitch BX + XPAD: the four lane groups of a read fall in distinct banks).
 // Thread tid's LOADS slots of a chunk: p-major, p = tid % KC (every slot) and x = tid / KC +
@@ -101,9 +100,9 @@ struct MmShape {
 // offset from the chunk's (uniform) base; rows past the operand's end read its last row
 // instead (they feed only entries of C that are never stored), and only the last chunk checks
 // the contraction bound (zeros past P).
-template <typename T, bool PM, int BX>
+template <bool PM, int BX>
 struct MmOperand {
-    typedef MmShape<T> S;
+    typedef MmShape S;
     static constexpr int ELEMS = PM ? BX * S::QP : S::KC * (BX + S::XPAD);
     static constexpr int LOADS = BX * S::KC / 256;  // global loads per thread and chunk
     static constexpr int XSTEP = PM ? 256 / S::KC : 0;
@@ -121,40 +120,40 @@ struct MmOperand {
 #pragma unroll
             for (int u = 0; u < LOADS; ++u) {
                 const int gx = min(x0 + xt + u * XSTEP, Xn - 1);
-                off[u] = (unsigned)(((size_t)p + (size_t)gx * ld) * sizeof(T));
+                off[u] = (unsigned)(((size_t)p + (size_t)gx * ld) * sizeof(float));
             }
-            cstride = (size_t)S::KC * sizeof(T);
+            cstride = (size_t)S::KC * sizeof(float);
         } else {
             p = tid / BX;
             xt = tid % BX;
             const int gx = min(x0 + xt, Xn - 1);
 #pragma unroll
-            for (int u = 0; u < LOADS; ++u) off[u] = (unsigned)(((size_t)gx + (size_t)(p + u * PSTEP) * ld) * sizeof(T));
-            cstride = (size_t)S::KC * ld * sizeof(T);
+            for (int u = 0; u < LOADS; ++u) off[u] = (unsigned)(((size_t)gx + (size_t)(p + u * PSTEP) * ld) * sizeof(float));
+            cstride = (size_t)S::KC * ld * sizeof(float);
         }
     }
     __device__ __forceinline__ int slot_p(int u) const { return p + u * PSTEP; }
     // global -> registers, chunk c
-    __device__ __forceinline__ void load(const T* X, int c, int P, T (&r)[LOADS]) const {
+    __device__ __forceinline__ void load(const float* X, int c, int P, float (&r)[LOADS]) const {
         const char* base = reinterpret_cast<const char*>(X) + (size_t)c * cstride;
         const int p0 = c * S::KC;
         if (p0 + S::KC <= P) {
 #pragma unroll
-            for (int u = 0; u < LOADS; ++u) r[u] = *reinterpret_cast<const T*>(base + off[u]);
+            for (int u = 0; u < LOADS; ++u) r[u] = *reinterpret_cast<const float*>(base + off[u]);
         } else {
 #pragma unroll
             for (int u = 0; u < LOADS; ++u)
-                r[u] = (p0 + slot_p(u) < P) ? *reinterpret_cast<const T*>(base + off[u]) : T(0);
+                r[u] = (p0 + slot_p(u) < P) ? *reinterpret_cast<const float*>(base + off[u]) : 0.0f;
         }
     }
     // the zero mode's adjustments: every element minus `shift` (the other operand is zero past
     // P), and `delta` where p == dnull
-    __device__ __forceinline__ void adjust(int c, T shift, T delta, int dnull, T (&r)[LOADS]) const {
+    __device__ __forceinline__ void adjust(int c, float shift, float delta, int dnull, float (&r)[LOADS]) const {
         const int p0 = c * S::KC;
 #pragma unroll
-        for (int u = 0; u < LOADS; ++u) r[u] = r[u] - shift + (p0 + slot_p(u) == dnull ? delta : T(0));
+        for (int u = 0; u < LOADS; ++u) r[u] = r[u] - shift + (p0 + slot_p(u) == dnull ? delta : 0.0f);
     }
-    __device__ __forceinline__ void store(T* lds, const T (&r)[LOADS]) const {
+    __device__ __forceinline__ void store(float* lds, const float (&r)[LOADS]) const {
 #pragma unroll
         for (int u = 0; u < LOADS; ++u) {
             if (PM) lds[(xt + u * XSTEP) * S::QP + p] = r[u];
@@ -162,16 +161,15 @@ struct MmOperand {
         }
     }
     // lane (x, q): the KS values of row xr (within the tile) at chunk offsets q*KS .. q*KS+KS-1
-    static __device__ __forceinline__ void read(const T* lds, int xr, int q, T (&v)[S::KS]) {
+    static __device__ __forceinline__ void read(const float* lds, int xr, int q, float (&v)[S::KS]) {
         if (PM) {
-            typedef typename Mma<T>::v16b V;
-            constexpr int W = 16 / sizeof(T);
-            const T* row = lds + xr * S::QP + q * S::KS;
+            typedef Mma<float>::v4 V;
+            const float* row = lds + xr * S::QP + q * S::KS;
 #pragma unroll
-            for (int i = 0; i < S::KS / W; ++i) {
-                const V t = *reinterpret_cast<const V*>(row + i * W);
+            for (int i = 0; i < S::KS / 4; ++i) {
+                const V t = *reinterpret_cast<const V*>(row + i * 4);
 #pragma unroll
-                for (int j = 0; j < W; ++j) v[i * W + j] = t[j];
+                for (int j = 0; j < 4; ++j) v[i * 4 + j] = t[j];
             }
         } else {
 #pragma unroll
@@ -180,15 +178,15 @@ struct MmOperand {
     }
 };
 
-template <typename T, bool PM, int BR, int BC>
-__global__ void __launch_bounds__(256) k_mma(MmArgs<T> a) {
-    typedef MmShape<T> S;
-    typedef MmOperand<T, PM, BR> OA;
-    typedef MmOperand<T, PM, BC> OB;
-    typedef typename Mma<T>::v4 v4;
+template <bool PM, int BR, int BC>
+__global__ void __launch_bounds__(256) k_mma(MmArgs<float> a) {
+    typedef MmShape S;
+    typedef MmOperand<PM, BR> OA;
+    typedef MmOperand<PM, BC> OB;
+    typedef Mma<float>::v4 v4;
     constexpr int NR = BR / 32, NC = BC / 32;  // 16 x 16 tiles per wave along r and c
     extern __shared__ __align__(16) unsigned char mm_lds[];
-    T* lds = reinterpret_cast<T*>(mm_lds);  // 2 x (OA::ELEMS + OB::ELEMS)
+    float* lds = reinterpret_cast<float*>(mm_lds);  // 2 x (OA::ELEMS + OB::ELEMS)
     __shared__ double red4[16];
 
     const int tid = threadIdx.x;
@@ -198,15 +196,15 @@ __global__ void __launch_bounds__(256) k_mma(MmArgs<T> a) {
     const int rt = rest % a.ntr;
     const int b = rest / a.ntr;
     const int r0 = rt * BR, c0 = ct * BC;
-    const T* A = a.A + (size_t)b * a.sA;
-    const T* B = a.B + (size_t)b * a.sB;
-    T* C = a.C + (size_t)b * a.sC;
+    const float* A = a.A + (size_t)b * a.sA;
+    const float* B = a.B + (size_t)b * a.sB;
+    float* C = a.C + (size_t)b * a.sC;
 
     // the zero mode: shift and delta (the same for every workgroup of that batch)
     const bool zm = (b == a.zb);
-    T shift = T(0), delta = T(0);
+    float shift = 0.0f, delta = 0.0f;
     if (zm) {
-        shift = T(a.shiftL * mean_shift(a.shift, red4));
+        shift = float(a.shiftL * mean_shift(a.shift, red4));
         if (a.linesum) {
             double s = 0.0;
             for (int m = tid; m < a.dn; m += 256) s += (double)a.wsum[m] * (double)a.linesum[m];
@@ -215,10 +213,10 @@ __global__ void __launch_bounds__(256) k_mma(MmArgs<T> a) {
             if ((tid & 63) == 0) red4[tid >> 6] = s;
             __syncthreads();
             const double tot = red4[0] + red4[1] + red4[2] + red4[3];
-            delta = T(-tot / ((double)a.wsum[a.dnull] * a.dnorm));
+            delta = float(-tot / ((double)a.wsum[a.dnull] * a.dnorm));
         }
     }
-    const T deltaA = (a.dop == 0) ? delta : T(0), deltaB = (a.dop == 1) ? delta : T(0);
+    const float deltaA = (a.dop == 0) ? delta : 0.0f, deltaB = (a.dop == 1) ? delta : 0.0f;
 
     const int lane = tid & 63;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform: scalar branches
@@ -233,7 +231,7 @@ __global__ void __launch_bounds__(256) k_mma(MmArgs<T> a) {
 #pragma unroll
     for (int i = 0; i < NR; ++i)
 #pragma unroll
-        for (int j = 0; j < NC; ++j) acc[i][j] = v4{T(0), T(0), T(0), T(0)};
+        for (int j = 0; j < NC; ++j) acc[i][j] = v4{0.0f, 0.0f, 0.0f, 0.0f};
 
     OA oa;
     OB ob;
@@ -242,13 +240,13 @@ __global__ void __launch_bounds__(256) k_mma(MmArgs<T> a) {
     // chunk kc + 1 is loaded into registers while chunk kc's MFMAs run from LDS, then goes to
     // the other LDS buffer; one barrier per chunk
     const int nk = (a.P + S::KC - 1) / S::KC;
-    T ra[OA::LOADS], rb[OB::LOADS];
+    float ra[OA::LOADS], rb[OB::LOADS];
     auto put = [&](int kc) {
         if (zm) {
             oa.adjust(kc, shift, deltaA, a.dnull, ra);
-            ob.adjust(kc, T(0), deltaB, a.dnull, rb);
+            ob.adjust(kc, 0.0f, deltaB, a.dnull, rb);
         }
-        T* nA = lds + (kc & 1) * (OA::ELEMS + OB::ELEMS);
+        float* nA = lds + (kc & 1) * (OA::ELEMS + OB::ELEMS);
         oa.store(nA, ra);
         ob.store(nA + OA::ELEMS, rb);
     };
@@ -262,9 +260,9 @@ __global__ void __launch_bounds__(256) k_mma(MmArgs<T> a) {
             oa.load(A, kc + 1, a.P, ra);
             ob.load(B, kc + 1, a.P, rb);
         }
-        const T* As = lds + (kc & 1) * (OA::ELEMS + OB::ELEMS);
-        const T* Bs = As + OA::ELEMS;
-        T av[NR][S::KS], bv[NC][S::KS];
+        const float* As = lds + (kc & 1) * (OA::ELEMS + OB::ELEMS);
+        const float* Bs = As + OA::ELEMS;
+        float av[NR][S::KS], bv[NC][S::KS];
 #pragma unroll
         for (int i = 0; i < NR; ++i) OA::read(As, wr + 16 * i + x, q, av[i]);
 #pragma unroll
@@ -275,7 +273,7 @@ __global__ void __launch_bounds__(256) k_mma(MmArgs<T> a) {
 #pragma unroll
                 for (int i = 0; i < NR; ++i)
 #pragma unroll
-                    for (int j = 0; j < NC; ++j) acc[i][j] = Mma<T>::run(bv[j][s], av[i][s], acc[i][j]);
+                    for (int j = 0; j < NC; ++j) acc[i][j] = Mma<float>::run(bv[j][s], av[i][s], acc[i][j]);
         } else {
 #pragma unroll
             for (int s = 0; s < S::KS; ++s)
@@ -283,7 +281,7 @@ __global__ void __launch_bounds__(256) k_mma(MmArgs<T> a) {
                 for (int i = 0; i < NR; ++i)
 #pragma unroll
                     for (int j = 0; j < NC; ++j)
-                        if (i < nri && j < nci) acc[i][j] = Mma<T>::run(bv[j][s], av[i][s], acc[i][j]);
+                        if (i < nri && j < nci) acc[i][j] = Mma<float>::run(bv[j][s], av[i][s], acc[i][j]);
         }
         if (more) put(kc + 1);
         __syncthreads();
@@ -296,7 +294,7 @@ __global__ void __launch_bounds__(256) k_mma(MmArgs<T> a) {
         for (int j = 0; j < NC; ++j)
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
-                const int gc = c0 + wc + 16 * j + Mma<T>::row(q, v);
+                const int gc = c0 + wc + 16 * j + Mma<float>::row(q, v);
                 if (gc < a.Cn) C[(size_t)gr + (size_t)gc * a.ldc] = acc[i][j][v];
             }
     }
@@ -304,7 +302,7 @@ __global__ void __launch_bounds__(256) k_mma(MmArgs<T> a) {
 
 // ---- FP64 products with the operand tiles staged by LDS DMA ----------------------------------
 //
-// The same product and lane layout as k_mma (BR x BC tiles of 64 or 128, 4 waves of
+// The same product as k_mma (BR x BC tiles of 64 or 128, 4 waves of
 // (BR/2) x (BC/2), KC = 16), with the chunks copied from global memory straight into LDS by
 // global_load_lds_dwordx4 (lane l's 16 bytes land at the instruction's LDS base + 16 l): no
 // registers hold a chunk in flight, and two LDS stages let chunk kc+1 load while chunk kc's
@@ -781,14 +779,14 @@ static void launch_mma64(hipStream_t st, const MmArgs<double>& a) {
     }
 }
 
-template <typename T, bool PM, int BR, int BC>
-static void launch_mma_tiles(hipStream_t st, MmArgs<T> a) {
+template <bool PM, int BR, int BC>
+static void launch_mma_tiles(hipStream_t st, MmArgs<float> a) {
     a.ntr = ceil_div(a.R, BR);
     a.ntc = ceil_div(a.Cn, BC);
     const long nwg = (long)a.ntr * a.ntc * a.nb;
-    const size_t sh = 2 * (MmOperand<T, PM, BR>::ELEMS + MmOperand<T, PM, BC>::ELEMS) * sizeof(T);
-    (void)hipFuncSetAttribute((const void*)k_mma<T, PM, BR, BC>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sh);
-    hipLaunchKernelGGL((k_mma<T, PM, BR, BC>), dim3((unsigned)nwg), dim3(256), sh, st, a);
+    const size_t sh = 2 * (MmOperand<PM, BR>::ELEMS + MmOperand<PM, BC>::ELEMS) * sizeof(float);
+    (void)hipFuncSetAttribute((const void*)k_mma<PM, BR, BC>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sh);
+    hipLaunchKernelGGL((k_mma<PM, BR, BC>), dim3((unsigned)nwg), dim3(256), sh, st, a);
 }
 
 template <typename T>
@@ -797,8 +795,8 @@ static void launch_mma(hipStream_t st, bool pmajor, const MmArgs<T>& a) {
         if (pmajor) launch_mma64<true>(st, a);
         else launch_mma64<false>(st, a);
     } else {
-        if (pmajor) launch_mma_tiles<T, true, 64, 64>(st, a);
-        else launch_mma_tiles<T, false, 64, 64>(st, a);
+        if (pmajor) launch_mma_tiles<true, 64, 64>(st, a);
+        else launch_mma_tiles<false, 64, 64>(st, a);
     }
 }
 
