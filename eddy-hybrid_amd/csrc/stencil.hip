@@ -217,7 +217,10 @@ static CorrArgs corr_args(const Dims& d, const Metrics& mt, const double* us, co
 // takes the spans b, b + nbx, ... of `planes` consecutive planes and keeps w of the plane below
 // in registers on its way up, so that w is read once but for the lowest plane's neighbour. It leaves its
 // minimum at part[slot], its maximum at part[nb + slot]. 24 B/cell, HBM bound: 0.430 -> 0.360 ms at
-// 768 x 384 x 256 over a kernel of row blocks, and one fold instead of two and a log kernel after it.
+// 768 x 384 x 256 over a kernel of row blocks, and one fold instead of two and a log kernel after it. The x1
+// metrics are read once per span: inside the plane loop they were waited for behind the cells' branches, plane by
+// plane (whole calls at 768 x 384 x 256 0.367 -> 0.336 ms, 512 x 256 x 256 0.191 -> 0.166, 256 x 192 x 96 on the same
+// fields again 0.050 -> 0.045, where the row blocks had taken 0.046).
 __global__ void __launch_bounds__(256) k_div_minmax(Dims d, Metrics mt, const double* __restrict__ us,
                                                     const double* __restrict__ vs, const double* __restrict__ ws,
                                                     double* part, unsigned rnx, int nbx, int planes, int runs) {
@@ -230,7 +233,7 @@ __global__ void __launch_bounds__(256) k_div_minmax(Dims d, Metrics mt, const do
         // the span's elements of the group's first plane; the others' are whole planes above
         Pair pr[kSpanParts];
         unsigned o[kSpanParts];
-        d2 wm[kSpanParts];
+        d2 wm[kSpanParts], api[kSpanParts];
         double bpj[kSpanParts];
 #pragma unroll
         for (int q = 0; q < kSpanParts; ++q) {
@@ -238,6 +241,9 @@ __global__ void __launch_bounds__(256) k_div_minmax(Dims d, Metrics mt, const do
             pr[q] = span_pair(d, r, rnx);
             o[q] = 8u * ((pr[q].on ? r : nx) + pl * (unsigned)(k0 + 1));
             bpj[q] = mt.bp[pr[q].on ? pr[q].j : 1];
+            const int i = pr[q].on ? pr[q].i : 0;
+            api[q].x = mt.ap[i];
+            api[q].y = mt.ap[i + 1];
             wm[q] = ld_pair(ws, o[q] - 8u * pl);
         }
         for (int k = k0; k < k1; ++k) {
@@ -255,21 +261,21 @@ __global__ void __launch_bounds__(256) k_div_minmax(Dims d, Metrics mt, const do
 #pragma unroll
             for (int q = 0; q < kSpanParts; ++q) {
                 // div_at's arithmetic
-                auto one = [&](int I, double um1, double u1, double vm1, double v1, double wm1, double w1) {
+                auto one = [&](int I, double ap, double um1, double u1, double vm1, double v1, double wm1, double w1) {
                     if (!pr[q].on || I < 1 || I > d.M) return;
                     const double c = cpk * (w1 - wm1);
                     double x;
                     if (mt.cart) {
-                        x = mt.ap[I] * (u1 - um1) + bpj[q] * (v1 - vm1) + c;
+                        x = ap * (u1 - um1) + bpj[q] * (v1 - vm1) + c;
                     } else {
                         const double rpi = mt.rp[I];
-                        x = mt.ap[I] * (mt.ru[I] * u1 - mt.ru[I - 1] * um1) / rpi + bpj[q] * (v1 - vm1) / rpi + c;
+                        x = ap * (mt.ru[I] * u1 - mt.ru[I - 1] * um1) / rpi + bpj[q] * (v1 - vm1) / rpi + c;
                     }
                     mn = fmin(mn, x);
                     mx = fmax(mx, x);
                 };
-                one(pr[q].i, um[q], u[q].x, vm[q].x, v[q].x, wm[q].x, w[q].x);
-                one(pr[q].i + 1, u[q].x, u[q].y, vm[q].y, v[q].y, wm[q].y, w[q].y);
+                one(pr[q].i, api[q].x, um[q], u[q].x, vm[q].x, v[q].x, wm[q].x, w[q].x);
+                one(pr[q].i + 1, api[q].y, u[q].x, u[q].y, vm[q].y, v[q].y, wm[q].y, w[q].y);
                 wm[q] = w[q];
                 o[q] += 8u * pl;
             }
@@ -658,10 +664,12 @@ void launch_divergence(hipStream_t st, const Dims& d, const Metrics& mt, const d
 void launch_div_minmax(hipStream_t st, const Dims& d, const Metrics& mt, const double* us, const double* vs,
                        const double* ws, const Reduce& rd, double* log, int* step, int cap) {
     // at most M blocks a plane: the partials hold M * N of each
-    // (planes per block: as many as leave 1024 blocks, at most 8; whole calls at 768 x 384 x 256 with 1,
-    // 2, 4, 8 planes: 0.492, 0.411, 0.379, 0.370 ms, 0.436 with one row per thread; at 64 x 64 x 32: 28, 29, 30, 33 us)
+    // (planes per block: as many as leave 2048 blocks, at most 8; whole calls with 1 plane and with the planes that
+    // leave 8192, 4096, 2048 and 1024 blocks: 768 x 384 x 256 0.389, 0.336 (8 planes in all four) ms, 512 x 256 x 192
+    // 0.147, 0.130, 0.131, 0.134, 0.134, 300 x 256 x 250 0.118, 0.109, 0.107, 0.108, 0.109, 300 x 128 x 256 0.072, 0.073,
+    // 0.071, 0.071, 0.073, 256 x 192 x 128 0.059, 0.058, 0.059, 0.057, 0.058)
     const int nbx = std::min(span_blocks(d), d.M);
-    const int planes = std::max(1, std::min(8, (int)((long)span_blocks(d) * d.N / 1024)));
+    const int planes = std::max(1, std::min(8, (int)((long)span_blocks(d) * d.N / 2048)));
     const int nb = nbx * ceil_div(d.N, planes);
     const int runs = 3 * sizeof(double) * (size_t)d.nx * d.ny * d.nz > ((size_t)256 << 20);
     hipLaunchKernelGGL(k_div_minmax, dim3(nb), dim3(256), 0, st, d, mt, us, vs, ws, rd.part, row_magic(d), nbx, planes,
