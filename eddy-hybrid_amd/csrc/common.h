@@ -44,7 +44,7 @@ struct Tables {
     // y real DFT as dense matrices for the matrix-core variant (FP32 tables only, else null):
     // ydft_f[j*L + p] = F(p, j) forward, ydft_b[p*L + j] = G(j, p) inverse with 1/L
     const T* ydft_f; const T* ydft_b;
-    // y real DFT of the lengths the radix FFT does not take (ydft_tab in yfft.hip), else null
+    // y real DFT of the lengths the radix FFT does not take (ydft_tab in api.hip), else null
     const T* ydm;
 };
 

@@ -45,9 +45,10 @@ enum YfftFwdMode { YF_DIRECT = 0, YF_RESIDUAL = 1, YF_DIVERGENCE = 2 };
 // What the forward y-FFT reads: YF_DIRECT the RHS in src (minus the solvability shift
 // red[RED_VOLB]/red[RED_VOL] when shift != 0); YF_RESIDUAL r = (src - that shift when
 // shift != 0) - L(phi) in FP64 (src is the RHS); YF_DIVERGENCE
-// b = DIV(us, vs, ws) * scale formed on the fly (sum vol*b -> red[RED_VOLB], sum vol ->
-// red[RED_VOL]; the solvability shift is then applied to the zero y-mode by the x2 transform;
-// the FP32 transform also stores b in FP64 at rhs_out, the RHS of the defect correction).
+// b = DIV(us, vs, ws) * scale formed on the fly (each workgroup leaves its sum of vol*b in the
+// partials; with fold, sum vol*b -> red[RED_VOLB] and sum vol -> red[RED_VOL]; the x2 transform
+// applies the solvability shift to the zero y-mode from the one or the other; the FP32 transform
+// also stores b in FP64 at rhs_out, the RHS of the defect correction).
 struct FwdInput {
     int mode;
     const double* src;

@@ -11,7 +11,8 @@
 // at one interior cell, found by mapping the z index, then the y index, then the x index (with its
 // sign and the axis reflection). The thread of an interior cell writes the ghosts that copy it beside
 // its own value, so that no pass over the shell waits for the interior to be done. Bound by memory at
-// large sizes (512 x 256 x 256 0.163 -> 0.155 ms, 5.2 TB/s on its 24 B/cell) and by its two dependent
+// large sizes (512 x 256 x 256 0.163 -> 0.155 ms, 5.2 TB/s on its 24 B/cell; with the implicit y correction 0.201
+// as before, 4.0 TB/s) and by its two dependent
 // launches at small ones (203 x 101 x 90 0.0176 -> 0.0142 ms, 32 x 32 x 32 0.0120 -> 0.0078).
 #include <algorithm>
 

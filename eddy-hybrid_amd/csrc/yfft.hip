@@ -6,7 +6,7 @@
 //
 // Periodic lengths the radix FFT cannot take (L odd, or L/2 with a prime factor >= 7) go through
 // the same tiles with the transform done as a dense real DFT on the matrix cores (the DENSE
-// kernels, dft_fwd_tile / dft_inv_tile), the packing and scaling as above.
+// kernels, dft_block), the packing and scaling as above.
 //
 // A workgroup owns TI (a power of two) consecutive x1 pencils at one x2 index k. The pencils
 // are read row by row (TI contiguous doubles per y index: coalesced), with several loads in
@@ -197,7 +197,7 @@ __device__ __forceinline__ void residual_rows(const Dims& d, const Op64& op, con
 // with P_j = x_j + x_{L-j} (P_0 = x_0, P_{L/2} = x_{L/2}) and Q_j = x_j - x_{L-j} (Q_0 = 0),
 //   Re X_q = sum_{j <= L/2} P_j cos(2 pi q j/L),   Im X_q = -sum_{j <= L/2} Q_j sin(2 pi q j/L),
 // and the inverse takes the same two symmetric matrices over q to x_j and x_{L-j}. The plan lays
-// them out in operand order (ydft_tab: block rb of 16 outputs, step ks of 4 samples, cosine then
+// them out in operand order (ydft_tab in api.hip: block rb of 16 outputs, step ks of 4 samples, cosine then
 // sine, lane), so an operand load is one contiguous 512-byte (FP32 256-byte) read served by L2.
 // A wave owns 16 outputs of 16 pencils: per step two LDS reads feed one cosine and one sine
 // product, 64 matrix-core cycles each in FP64, which hide both the reads and the additions of
@@ -258,9 +258,9 @@ __device__ __forceinline__ void dft_zero_pads(T* rows, int pitch, int L, int TI,
 }
 
 // One tile (TI pencils at one x2 index) of the forward transform; `tile` is the logical tile,
-// ntx the tiles per x2 row, `slot`/`nslots` the reduction partial index and count.
+// ntx the tiles per x2 row, `slot` the reduction partial's index.
 template <typename T, int MODE, bool DENSE = false, bool NT = false>
-__device__ __forceinline__ void yfft_fwd_tile(const YArgs<T>& a, int tile, int ntx, int slot, int nslots) {
+__device__ __forceinline__ void yfft_fwd_tile(const YArgs<T>& a, int tile, int ntx, int slot) {
     extern __shared__ unsigned char smem_raw[];
     T* smem = reinterpret_cast<T*>(smem_raw);
     const Dims d = a.d;
@@ -430,12 +430,17 @@ __device__ __forceinline__ void yfft_fwd_tile(const YArgs<T>& a, int tile, int n
 // NT: the spectrum's rows are whole lines (M a multiple of 16) and it fills the 256 MiB memory-side
 // cache, which non-temporal stores leave to the velocities (512 x 256 x 256: this kernel 0.2746 -> 0.2727 ms,
 // the line solve 0.1148 -> 0.1097). Rows that begin inside a line lose by it (500 x 256 x 256 0.278 -> 0.327),
-// and smaller spectra are read back from the cache (256 x 192 x 128: x2 transform 0.0284 -> 0.0320).
+// and smaller spectra are read back from the cache (256 x 192 x 128: x2 transform 0.0284 -> 0.0320). Whole
+// projections without and with it, by the size of the spectrum: 72 MiB 0.3170 -> 0.3210 ms and 0.3274 -> 0.3310; 112 and
+// 117 equal; 160 0.6912 -> 0.6910; 192 0.8005 -> 0.7976, 0.8083 -> 0.8052 and 0.7728 -> 0.7784; 240 0.9968 -> 0.9965;
+// 256 1.0620 -> 1.0509 and 1.0678 -> 1.0591; 288 1.2742 -> 1.2685; 320 1.4172 -> 1.4092; 384 to 960 within 0.4 % of each
+// other, both ways. Solves of a stored RHS: 256 0.5616 -> 0.5604, 288 0.7231 -> 0.7216, 320 0.7908 -> 0.7960, 384
+// 0.9014 -> 0.9094, 480 1.1504 -> 1.1566, 960 2.4089 -> 2.4001.
 template <typename T, int MODE, bool DENSE, bool NT = false>
 __global__ void __launch_bounds__(kFftThreads) k_yfft_fwd(YArgs<T> a) {
     const int nb = gridDim.x * gridDim.y;
     const int t = iblock_tile(xcd_tile(blockIdx.x + gridDim.x * blockIdx.y, nb), gridDim.x, gridDim.y, a.iblk);
-    yfft_fwd_tile<T, MODE, DENSE, NT>(a, t, gridDim.x, linear_bid(), nb);
+    yfft_fwd_tile<T, MODE, DENSE, NT>(a, t, gridDim.x, linear_bid());
 }
 
 // The forward transform of a stored RHS at no more than 80 VGPRs: with its 42 KB LDS tile
@@ -444,7 +449,7 @@ template <typename T, bool DENSE, bool NT = false>
 __global__ void __launch_bounds__(kFftThreads) __attribute__((amdgpu_waves_per_eu(6))) k_yfft_fwd_rhs(YArgs<T> a) {
     const int nb = gridDim.x * gridDim.y;
     const int t = iblock_tile(xcd_tile(blockIdx.x + gridDim.x * blockIdx.y, nb), gridDim.x, gridDim.y, a.iblk);
-    yfft_fwd_tile<T, YF_DIRECT, DENSE, NT>(a, t, gridDim.x, linear_bid(), nb);
+    yfft_fwd_tile<T, YF_DIRECT, DENSE, NT>(a, t, gridDim.x, linear_bid());
 }
 
 template <typename T, int MODE, bool DENSE = false, bool NT = false>
@@ -659,7 +664,9 @@ __device__ __forceinline__ void yfft_inv_tile(const YArgs<T>& a, int tile, int n
 // NT: the spectrum's rows are whole lines and it fills the memory-side cache with the pressure; its
 // last read, past the caches, leaves them the pressure for CORRECT (512 x 256 x 256: this kernel 0.137 -> 0.131 ms
 // and CORRECT 0.343 -> 0.330; 512 x 256 x 192 0.100 -> 0.089 and 0.256 -> 0.244; 768 x 384 x 256 0.278 -> 0.259 but
-// CORRECT 0.777 -> 0.795). A smaller spectrum comes from the caches, and lines that two tiles share would be
+// CORRECT 0.777 -> 0.795). Whole projections without and with it: spectra of 117 MiB 0.5578 -> 0.5567 ms, 128 0.5243 ->
+// 0.5162, 160 0.7037 -> 0.6912, 192 0.8237 -> 0.8005, 256 1.0771 -> 1.0620, 320 1.4175 -> 1.4172; past that within 0.7 % of
+// each other, both ways (768 x 384 x 256 2.4607 -> 2.4603). A smaller spectrum (72 MiB 0.3281 -> 0.3338) comes from the caches, and lines that two tiles share would be
 // read twice (300 x 256 x 250: 0.084 -> 0.097 and 0.195 -> 0.187; 300 x 128 x 128 0.0252 -> 0.0280).
 template <typename T, int MODE, bool DENSE, bool NT = false>
 // at most 80 VGPRs (the last defect-correction update needs 82 unbounded): with its 42 KB LDS
@@ -807,7 +814,7 @@ template <typename T, int MODE>
 __global__ void __launch_bounds__(kFftThreads) __attribute__((amdgpu_waves_per_eu(MODE == YF_RESIDUAL ? 4 : 1)))
 k_batch_yfft_fwd(const Job<YArgs<T>>* jobs, int njobs, int total) {
     run_item(jobs, njobs, total,
-             [](const Job<YArgs<T>>& J, int t) { yfft_fwd_tile<T, MODE>(J.a, t, J.ntx, t, J.ntiles); });
+             [](const Job<YArgs<T>>& J, int t) { yfft_fwd_tile<T, MODE>(J.a, t, J.ntx, t); });
 }
 
 // the stored-RHS form at no more than 80 VGPRs, as k_yfft_fwd_rhs
@@ -815,7 +822,7 @@ template <typename T>
 __global__ void __launch_bounds__(kFftThreads) __attribute__((amdgpu_waves_per_eu(6)))
 k_batch_yfft_fwd_rhs(const Job<YArgs<T>>* jobs, int njobs, int total) {
     run_item(jobs, njobs, total,
-             [](const Job<YArgs<T>>& J, int t) { yfft_fwd_tile<T, YF_DIRECT>(J.a, t, J.ntx, t, J.ntiles); });
+             [](const Job<YArgs<T>>& J, int t) { yfft_fwd_tile<T, YF_DIRECT>(J.a, t, J.ntx, t); });
 }
 
 template <typename T, int MODE>
