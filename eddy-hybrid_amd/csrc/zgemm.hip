@@ -733,15 +733,15 @@ static void launch_mma64_tiles(hipStream_t st, MmArgs<double> a) {
     const long tiles = (long)wr * a.ntc * a.nb, rounds = (tiles + 1023) / 1024;
     const long nwg = (long)ceil_div(wr * a.ntc, 4) * a.nb;
     // Row tiles that four waves do not divide left workgroups of one or two waves, which spread unevenly
-    // over the SIMDs: with the last of several rounds of waves more than half full, a third one landed on
-    // SIMDs that should run two (a product: 220 x 260 x 48 0.0392 -> 0.0345 ms, 395 x 161 x 24 0.0238 -> 0.0204, 104 x 266 x
-    // 84 0.0212 -> 0.0185, 188 x 239 x 58 0.0339 -> 0.0297, 437 x 309 x 14 0.0435 -> 0.0337; over 140 products at random
-    // shapes 0.76 to 1.04 of the time, 0.96 in the mean). With it less full four to a workgroup lose: over 227 products
-    // 0.90 to 1.25, 1.02 in the mean (203 x 101 x 90, 2.46 rounds, 0.0182 -> 0.0188; 122 x 130 x 116, 2.27, 0.0216 -> 0.0242;
-    // 200 x 200 x 64, 3.06, 0.0343 -> 0.0353), and so they do where filling up to four adds a round (150 x 150 x 150
-    // 0.0311 -> 0.0360; over 56 products 0.95 to 1.30, 1.09 in the mean). In the first round it goes either way (0.72 to
-    // 1.40 over 60).
-    if (wr % 4 && rounds > 1 && 20 * tiles >= 1024 * (20 * rounds - 9) && 4 * nwg <= 1024 * rounds) {
+    // over the SIMDs: with the last of several rounds of waves well filled, a third one landed on SIMDs that
+    // should run two (a product: 220 x 260 x 48 0.0392 -> 0.0345 ms, 395 x 161 x 24 0.0238 -> 0.0204, 104 x 266 x 84 0.0212 ->
+    // 0.0185, 188 x 239 x 58 0.0339 -> 0.0297, 437 x 309 x 14 0.0435 -> 0.0337). Workgroups of two gain by four from a last
+    // round a fifth full (334 products at random shapes 0.76 to 1.18 of the time, 0.98 in the mean; below it 48 0.91 to
+    // 1.25, 1.03), workgroups of one from half (312 products 0.83 to 1.14, 0.99; from a fifth to a half 394 0.93 to 1.22,
+    // 1.02: 203 x 101 x 90, 2.46 rounds, 0.0182 -> 0.0188, 122 x 130 x 116, 2.27, 0.0216 -> 0.0242). Not where filling up to four
+    // adds a round (150 x 150 x 150 0.0311 -> 0.0360; 56 products 0.95 to 1.30, 1.09), nor in the first round, which goes
+    // either way (60 products 0.72 to 1.40).
+    if (wr % 4 && rounds > 1 && 10 * tiles >= 1024 * (10 * rounds - (wr % 2 ? 5 : 8)) && 4 * nwg <= 1024 * rounds) {
         a.flat = 1;
         a.ntr = wr;
         hipLaunchKernelGGL((k_mma64<PM, NR, NC>), dim3((unsigned)nwg), dim3(256), 0, st, a);
